@@ -48,6 +48,7 @@ inline DevParams make_dev_params(const fhdx_params& p)
         d.bo[i] = 0;
         d.bn[i] = p.n_cells[i];
         d.dx[i] = p.dx[i];
+        d.rdx[i] = 1. / p.dx[i];
         d.grav[i] = p.grav[i];
     }
     d.algorithm_type = p.algorithm_type;
@@ -57,6 +58,7 @@ inline DevParams make_dev_params(const fhdx_params& p)
     d.transport_type = p.transport_type;
     for (int n = 0; n < MS; ++n) {
         d.molmass[n] = p.molmass[n];
+        d.rmolmass[n] = 1. / p.molmass[n];
         d.diameter[n] = p.diameter[n];
         d.hcv[n] = p.hcv[n];
         d.hcp[n] = p.hcp[n];

@@ -17,6 +17,56 @@ namespace fhdx {
 
 constexpr int MS = FHDX_MAX_SPECIES;
 
+// ---- division and square root ---------------------------------------------------------------
+//
+// The compiler's FP64 division is 11 VALU instructions (two div_scale, rcp, four fma, a mul and a
+// fma of the quotient, div_fmas, div_fixup) with four wait states before div_fmas, and the step
+// divides several hundred times per cell, most often by a constant of the run (dx, a molar mass) or
+// several times by one value (rho, a mean pressure).  Rcp holds a divisor and its reciprocal to
+// the last bit, so each further quotient is 4 instructions: q = a r, the exact remainder
+// a - b q, q corrected by it, div_fixup (zero, infinite and NaN operands).  These are the
+// compiler's own steps with the two scalings left out, and with r correctly rounded the corrected
+// quotient is the IEEE one (Markstein, IBM J. Res. Dev. 34, 1990; Brisebarre, Muller and Raina,
+// IEEE Trans. Comput. 53, 2004), so the bits are those of a / b.  What the scalings are for:
+// divisors or quotients outside about 2^+-1000 and dividends below 2^-968, where the last bit may
+// differ.
+// 256^3 argon: the face kernel 4.49 ms a launch with the compiler's divisions and roots, 3.92 ms with
+// these (its vector instructions 6545 and 5620).
+struct Rcp {
+    double b, r;
+};
+
+__device__ __forceinline__ double operator/(double a, const Rcp& d)
+{
+    const double q = a * d.r;
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d.b, q, a), d.r, q), d.b, a);
+}
+
+// The reciprocal by two Newton steps from v_rcp_f64, as the compiler's division refines it.
+__device__ __forceinline__ Rcp rcp_of(double b)
+{
+    double r = __builtin_amdgcn_rcp(b);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+    return Rcp{b, r};
+}
+
+__device__ __forceinline__ double quot(double a, double b) { return a / rcp_of(b); }
+
+// sqrt of x = +-0 or x >= 2^-767 (infinity and NaN included): the compiler's refinement of
+// v_rsq_f64 without the scaling of smaller x, 13 instructions for 19.
+__device__ __forceinline__ double root(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double s = x * y, h = y * 0.5;
+    const double e = __builtin_fma(-h, s, 0.5);
+    s = __builtin_fma(s, e, s);
+    h = __builtin_fma(h, e, h);
+    s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+    s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+    return __builtin_amdgcn_class(x, 0x260) ? x : s;  // +-0, +infinity
+}
+
 // Kernel-argument copy of the run parameters plus per-call constants.
 constexpr int MR = 8;  // reactions (FHDX_MAX_REACTION)
 
@@ -37,6 +87,7 @@ struct DevParams {
     int algorithm_type, advection_type, visc_type, stoch_on;
     int transport_type;  // 1 Giovangigli, 3 Hirschfelder-Curtiss-Bird binary
     double dx[3];
+    double rdx[3], rmolmass[MS];  // reciprocals of dx and molmass
     double molmass[MS], diameter[MS], hcv[MS], hcp[MS], e0[MS];
     double k_B, Runiv, zeta_ratio;
     double grav[3];
@@ -49,6 +100,9 @@ struct DevParams {
     int wall[6], bcv[6], bct[6], bcm[6];
     double tw[6], pw[6], rhow[6];  // wall / reservoir temperature; reservoir pressure, density
     double Yw[6][MS], Xw[6][MS];
+
+    __device__ Rcp h(int d) const { return Rcp{dx[d], rdx[d]}; }
+    __device__ Rcp M(int n) const { return Rcp{molmass[n], rmolmass[n]}; }
 };
 
 // Strided view of one FAB (AMReX Array4 layout: x fastest, then y, z, component).
@@ -84,7 +138,7 @@ __device__ inline double eos_temperature(const DevParams& P, double energy, cons
         cvmix += Yk[n] * P.hcv[n];
         e0mix += Yk[n] * P.e0[n];
     }
-    return (energy - e0mix) / cvmix;
+    return quot(energy - e0mix, cvmix);
 }
 
 template <int NS>
@@ -92,9 +146,9 @@ __device__ inline double eos_pressure(const DevParams& P, const double* Yk, doub
 {
     double molmix = 0.;
 #pragma unroll
-    for (int n = 0; n < NS; ++n) molmix += Yk[n] / P.molmass[n];
-    molmix = 1. / molmix;
-    return rho * (P.Runiv / molmix) * T;
+    for (int n = 0; n < NS; ++n) molmix += Yk[n] / P.M(n);
+    molmix = quot(1., molmix);
+    return rho * quot(P.Runiv, molmix) * T;
 }
 
 template <int NS>
@@ -115,31 +169,33 @@ template <int NS>
 __device__ inline void cons_to_prim_cell(const DevParams& P, const double* c, double* pr)
 {
     double Yk[NS], Yf[NS];
+    const Rcp rho = rcp_of(c[0]);
     pr[0] = c[0];
-    pr[1] = c[1] / c[0];
-    pr[2] = c[2] / c[0];
-    pr[3] = c[3] / c[0];
+    pr[1] = c[1] / rho;
+    pr[2] = c[2] / rho;
+    pr[3] = c[3] / rho;
     double vsqr = pr[1] * pr[1] + pr[2] * pr[2] + pr[3] * pr[3];
-    double intenergy = c[4] / c[0] - 0.5 * vsqr;
+    double intenergy = c[4] / rho - 0.5 * vsqr;
     double sumYk = 0.;
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
-        Yk[n] = c[5 + n] / c[0];
+        Yk[n] = c[5 + n] / rho;
         Yf[n] = clamp01(Yk[n]);
         sumYk += Yf[n];
     }
+    const Rcp sum = rcp_of(sumYk);
 #pragma unroll
-    for (int n = 0; n < NS; ++n) Yf[n] /= sumYk;
+    for (int n = 0; n < NS; ++n) Yf[n] = Yf[n] / sum;
     pr[4] = eos_temperature<NS>(P, intenergy, Yf);
     // GetMolfrac of the raw mass fractions
     double molmix = 0.;
 #pragma unroll
-    for (int n = 0; n < NS; ++n) molmix += Yk[n] / P.molmass[n];
-    molmix = 1. / molmix;
+    for (int n = 0; n < NS; ++n) molmix += Yk[n] / P.M(n);
+    molmix = quot(1., molmix);
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
         pr[6 + n] = Yk[n];
-        pr[6 + NS + n] = Yk[n] * molmix / P.molmass[n];
+        pr[6 + NS + n] = Yk[n] * molmix / P.M(n);
     }
     pr[5] = eos_pressure<NS>(P, Yk, pr[0], pr[4]);
 }
@@ -783,6 +839,7 @@ __device__ inline void cholesky(double* a, double* sqda)
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
         bool ising = false;
+        Rcp pivot{0., 0.};
 #pragma unroll
         for (int j = i; j < NS; ++j) {
             double sum1 = a[i * NS + j];
@@ -793,10 +850,12 @@ __device__ inline void cholesky(double* a, double* sqda)
                     p[i] = 0.;
                     ising = true;
                 } else {
-                    p[i] = sqrt(sum1);
+                    p[i] = root(sum1);
                 }
+                pivot = rcp_of(p[i]);
+            } else {
+                a[j * NS + i] = ising ? 0. : sum1 / pivot;
             }
-            a[j * NS + i] = ising ? 0. : sum1 / p[i];
         }
     }
 #pragma unroll
@@ -811,16 +870,22 @@ struct U4 {
     uint32_t x, y, z, w;
 };
 
-__host__ __device__ inline U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1)
+// gfx950's three-operand bitwise instruction: one per output word and round instead of two.
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c)
+{
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+
+__device__ inline U4 philox4x32_10(U4 c, uint32_t k0, uint32_t k1)
 {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
         uint64_t p0 = (uint64_t)0xD2511F53u * c.x;
         uint64_t p1 = (uint64_t)0xCD9E8D57u * c.z;
         U4 o;
-        o.x = (uint32_t)(p1 >> 32) ^ c.y ^ k0;
+        o.x = xor3((uint32_t)(p1 >> 32), c.y, k0);
         o.y = (uint32_t)p1;
-        o.z = (uint32_t)(p0 >> 32) ^ c.w ^ k1;
+        o.z = xor3((uint32_t)(p0 >> 32), c.w, k1);
         o.w = (uint32_t)p0;
         c = o;
         k0 += 0x9E3779B9u;
@@ -844,7 +909,7 @@ __device__ inline double bm_log(double x)
         m = m * 0.5;
         e = e + 1;
     }
-    const double sr = (m - 1.0) / (m + 1.0);
+    const double sr = quot(m - 1.0, m + 1.0);
     const double z = sr * sr;
     double p = 1.0 / 23.0;
     p = fma(p, z, 1.0 / 21.0);
@@ -899,15 +964,19 @@ __device__ inline void bm_sincospi(double t, double& sn, double& cs)
     cs = ((q + 1) & 2) ? -b : b;
 }
 
+// The top 53 bits of hi:lo as a double (exact): its upper 21 and lower 32 bits joined by one fma.
+__device__ __forceinline__ double top53(uint32_t hi, uint32_t lo)
+{
+    return __builtin_fma((double)(hi >> 11), 4294967296.0, (double)__builtin_amdgcn_alignbit(hi, lo, 11));
+}
+
 // Two N(0,1) values from one Philox block: 53-bit u1 in (0,1], u2 in [0,1).
 __device__ inline void normal_pair(U4 r, double& z0, double& z1)
 {
     const double two_m53 = 1.1102230246251565e-16;
-    uint64_t a = ((((uint64_t)r.x) << 32) | r.y) >> 11;
-    uint64_t b = ((((uint64_t)r.z) << 32) | r.w) >> 11;
-    double u1 = ((double)a + 0.5) * two_m53;
-    double u2 = (double)b * two_m53;
-    double rad = sqrt(-2.0 * bm_log(u1));
+    double u1 = (top53(r.x, r.y) + 0.5) * two_m53;
+    double u2 = top53(r.z, r.w) * two_m53;
+    double rad = root(-2.0 * bm_log(u1));
     double s, c;
     bm_sincospi(2.0 * u2, s, c);
     z0 = rad * c;

@@ -152,8 +152,9 @@ __device__ inline void cell_record(const DevParams& P, const double* c, const Fl
     for (int s = 0; s < NS; ++s) yn[s] = clamp01(pr[6 + s]);
 #pragma unroll
     for (int s = 0; s < NS; ++s) sumy += yn[s];
+    const Rcp ry = rcp_of(sumy);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) yn[s] /= sumy;
+    for (int s = 0; s < NS; ++s) yn[s] = yn[s] / ry;
     double rec[8 + 4 * NS + NS * NS];
     rec[RecLayout::U] = pr[1];
     rec[RecLayout::V] = pr[2];
@@ -258,7 +259,8 @@ __device__ inline void node_body(const DevParams& P, const Fld& R, const Fld& N,
         zetaxp = 0.125 * (z[nc8(1, 0, 0)] + z[nc8(0, 0, 0)] + z[nc8(1, 1, 0)] + z[nc8(0, 1, 0)] +
                           z[nc8(1, 0, 1)] + z[nc8(0, 0, 1)] + z[nc8(1, 1, 1)] + z[nc8(0, 1, 1)]);
     }
-    const double DX0 = P.dx[0], DX1 = P.dx[1], DX2 = P.dx[2];
+    const Rcp DX0 = P.h(0), DX1 = P.h(1), DX2 = P.h(2);
+    constexpr Rcp three{3., 1. / 3.}, twelve{12., 1. / 12.};
     double out[NODE_NCOMP];
 #pragma unroll
     for (int bcomp = 0; bcomp < 3; ++bcomp) {
@@ -278,7 +280,7 @@ __device__ inline void node_body(const DevParams& P, const Fld& R, const Fld& N,
     }
     // flux.cpp:1705-1711
     out[NODE_VC] =
-        (muxp / 12. + zetaxp / 4.) *
+        (muxp / twelve + zetaxp / 4.) *
         ((u[nc8(1, 0, 0)] - u[nc8(0, 0, 0)]) / DX0 + (u[nc8(1, 1, 0)] - u[nc8(0, 1, 0)]) / DX0 +
          (u[nc8(1, 0, 1)] - u[nc8(0, 0, 1)]) / DX0 + (u[nc8(1, 1, 1)] - u[nc8(0, 1, 1)]) / DX0 +
          (v[nc8(0, 1, 0)] - v[nc8(0, 0, 0)]) / DX1 + (v[nc8(1, 1, 0)] - v[nc8(1, 0, 0)]) / DX1 +
@@ -299,7 +301,7 @@ __device__ inline void node_body(const DevParams& P, const Fld& R, const Fld& N,
                 const double term = eta * T[cell];
                 sm = (q == 0) ? term : sm + term;
             }
-            double mu = 0.25 * sm / 3.;
+            double mu = 0.25 * sm / three;
             if (visc3) {
                 double zs = 0.;
 #pragma unroll
@@ -313,7 +315,7 @@ __device__ inline void node_body(const DevParams& P, const Fld& R, const Fld& N,
                 }
                 mu += 0.25 * zs;
             }
-            out[NODE_S + v2] = sqrt(mu) * W;
+            out[NODE_S + v2] = root(mu) * W;
         }
     }
     const int nout = P.stoch_on ? NODE_NCOMP : NODE_S;
@@ -352,10 +354,14 @@ __device__ inline double node_sum(const Fld& N, int c, unsigned cb, bool zorder,
 // INL: the face's A/B noise is evaluated in place from Philox key K (the values fhdx_fill_noise
 // writes for that key); otherwise it is read from the step's arrays A, B.
 template <int NS, int D, bool INL>
-__device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R, const Fld& N, const Fld& A,
-                                 const Fld& B, const NoiseKey& K, double w, double volinv, double dtinv, double dt,
-                                 int i, int j, int k, unsigned cb, double* fo)
+__device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A, Fld B, const NoiseKey& K, double w,
+                                 double volinv, double dtinv, double dt, int i, int j, int k, unsigned cb, double* fo)
 {
+    // a component stride of this direction's own, so that the component bases are not shared (and
+    // kept) across the three directions
+    long sn = R.sn;
+    asm("" : "+s"(sn));
+    Us.sn = R.sn = N.sn = A.sn = B.sn = sn;
     // the face lies between cell (i,j,k) ("U", offset cb) and its lower neighbour ("L", -e)
     constexpr int ex = (D == 0), ey = (D == 1), ez = (D == 2);
     constexpr int nv = NS + 5;
@@ -415,14 +421,14 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
             }
         }
         double wi[nv];
-        double fw1 = sqrt(P.k_B * mup * volinv * dtinv);
-        double fw4 = sqrt(P.k_B * kp * volinv * dtinv);
+        double fw1 = root(P.k_B * mup * volinv * dtinv);
+        double fw4 = root(P.k_B * kp * volinv * dtinv);
         wi[0] = 0.;
         wi[1] = fw1 * wn[1];
         wi[2] = fw1 * wn[2];
         wi[3] = fw1 * wn[3];
         wi[4] = fw4 * wn[4];
-        double nweight = sqrt(P.k_B * volinv * dtinv);
+        double nweight = root(P.k_B * volinv * dtinv);
         // edge terms sqrt(mu)*rancorn of the pp, mp, pm, mm edges (flux.cpp:277-280, 644-647, 1011-1014)
         double sum;
         if (D == 0) {
@@ -464,7 +470,7 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
             double MWmix = 0.;
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                MWmix = MWmix + 0.5 * (yy[s] + yyp[s]) / P.molmass[s];
+                MWmix = MWmix + 0.5 * (yy[s] + yyp[s]) / P.M(s);
 #pragma unroll
                 for (int l = 0; l < NS; ++l)
                     DijY[s * NS + l] = 0.5 * (DL[l * NS + s] * yy[l] + DU[l * NS + s] * yyp[l] +
@@ -478,9 +484,9 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
                         DijY[s * NS + n] = 0.;
                         DijY[n * NS + s] = 0.;
                     }
-            MWmix = 1. / MWmix;
+            MWmix = quot(1., MWmix);
             cholesky<NS>(DijY, sqD);
-            double wsp = sqrt(P.k_B * MWmix * volinv / (P.Runiv * dt));
+            double wsp = root(quot(P.k_B * MWmix * volinv, P.Runiv * dt));
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
 #pragma unroll
@@ -491,7 +497,7 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 double hk = P.e0[s] + P.hcp[s] * meanT;
-                double ss = (hk + P.Runiv * meanT / P.molmass[s] * 0.5 * (chiL[s] + chiU[s])) * wi[5 + s];
+                double ss = (hk + P.Runiv * meanT / P.M(s) * 0.5 * (chiL[s] + chiU[s])) * wi[5 + s];
                 soret = soret + ss;
             }
             f[nv + 3] = f[nv + 3] + soret;
@@ -500,7 +506,8 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
 
     // ---- diffusive (flux.cpp:1193-1623) ----
     {
-        const double half = 0.5, h = P.dx[D];
+        const double half = 0.5;
+        const Rcp h = P.h(D);
         double mup = half * (etaU + etaL);
         double kp = half * (kapU + kapL);
         double tau1 = mup * (velU(1) - velL(1)) / h;
@@ -523,6 +530,7 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
         double meanT = 0.5 * (TL + TU);
         double meanP = 0.5 * (PL + PU);
         if (species) {
+            const Rcp rT = rcp_of(meanT), rP = rcp_of(meanP);
             double dk[NS], soret[NS], Fk[NS];
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
@@ -530,14 +538,14 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
                 double term1 = (XU - XL) / h;
                 double mX = 0.5 * (XL + XU);
                 double mY = 0.5 * (R(cb, RecLayout::Y + s, -ex, -ey, -ez) + R(cb, RecLayout::Y + s));
-                double term2 = (mX - mY) * (PU - PL) / h / meanP;
+                double term2 = (mX - mY) * (PU - PL) / h / rP;
                 dk[s] = term1 + term2;
                 double ChiX;
                 if (D == 2)  // flux.cpp:1561 reads chi at k and k+1
                     ChiX = 0.5 * (chiU[s] * XL + R(cb, L.CHI() + s, 0, 0, 1) * XU);
                 else
                     ChiX = 0.5 * (chiL[s] * XL + chiU[s] * XU);
-                soret[s] = ChiX * (TU - TL) / h / meanT;
+                soret[s] = ChiX * (TU - TL) / h / rT;
             }
 #pragma unroll
             for (int kk = 0; kk < NS; ++kk) {
@@ -555,7 +563,7 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
                 double hk = P.e0[s] + P.hcp[s] * meanT;
                 double csum = (D == 2) ? chiU[s] + chiU[s]  // flux.cpp:1604
                                        : chiL[s] + chiU[s];
-                double Q5s = (hk + 0.5 * P.Runiv * meanT * csum / P.molmass[s]) * Fk[s];
+                double Q5s = (hk + 0.5 * P.Runiv * meanT * csum / P.M(s)) * Fk[s];
                 Q5 = Q5 + Q5s;
             }
             f[nv + 3] = f[nv + 3] + Q5;
@@ -619,12 +627,13 @@ __device__ inline void face_flux(const DevParams& P, const Fld& Us, const Fld& R
             for (int l = 0; l < NS + 5; ++l)
                 cv[l] = wgt1 * (Us(cb, l) + Us(cb, l, -ex, -ey, -ez)) -
                         wgt2 * (Us(cb, l, -2 * ex, -2 * ey, -2 * ez) + Us(cb, l, ex, ey, ez));
+            const Rcp rho = rcp_of(cv[0]);
 #pragma unroll
-            for (int l = 1; l < 4; ++l) pv[l] = cv[l] / cv[0];
+            for (int l = 1; l < 4; ++l) pv[l] = cv[l] / rho;
 #pragma unroll
-            for (int n = 0; n < NS; ++n) Yk[n] = cv[5 + n] / cv[0];
+            for (int n = 0; n < NS; ++n) Yk[n] = cv[5 + n] / rho;
             double vsqr = pv[1] * pv[1] + pv[2] * pv[2] + pv[3] * pv[3];
-            double ie = cv[4] / cv[0] - 0.5 * vsqr;
+            double ie = cv[4] / rho - 0.5 * vsqr;
             pv[4] = eos_temperature<NS>(P, ie, Yk);
             pv[5] = eos_pressure<NS>(P, Yk, cv[0], pv[4]);
         }
@@ -758,8 +767,8 @@ __device__ inline void update_body(const DevParams& P, const Fld& out, const Fld
 #pragma unroll
     for (int n = 0; n < NS + 5; ++n)
         // face n holds face 0 of the periodic box (store_face)
-        div[n] = (fx(cb, n, 1, 0, 0) - fx(cb, n)) / P.dx[0] + (fy(cb, n, 0, 1, 0) - fy(cb, n)) / P.dx[1] +
-                 (fz(cb, n, 0, 0, 1) - fz(cb, n)) / P.dx[2];
+        div[n] = (fx(cb, n, 1, 0, 0) - fx(cb, n)) / P.h(0) + (fy(cb, n, 0, 1, 0) - fy(cb, n)) / P.h(1) +
+                 (fz(cb, n, 0, 0, 1) - fz(cb, n)) / P.h(2);
     update_from_div<NS>(P, out, u0, us, div, dt, mode, prim, write_prim, i, j, k, cb, rec_next, err, chem);
 }
 
