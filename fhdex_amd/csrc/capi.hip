@@ -566,15 +566,21 @@ int fhdx_ctx_create(const fhdx_params* p, fhdx_ctx** out)
     hipError_t e = hipGetDevice(&c->device);
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_err, sizeof(int));
     if (e == hipSuccess) e = hipMemset(c->d_err, 0, sizeof(int));
+    const MixTab mix = make_mix_tab(*p);
+    if (e == hipSuccess) e = hipMalloc((void**)&c->d_mix, sizeof(MixTab));
+    if (e == hipSuccess) e = hipMemcpy(c->d_mix, &mix, sizeof(MixTab), hipMemcpyHostToDevice);
+    c->dp.mix = c->d_mix;
     if (e != hipSuccess) {
         set_error(std::string("context setup failed: ") + hipGetErrorString(e));
         if (c->d_err) (void)hipFree(c->d_err);
+        if (c->d_mix) (void)hipFree(c->d_mix);
         delete c;
         return FHDX_ERR_HIP;
     }
     // this device's copy of the no-allocation scratch, looked up once per device
     if ((r = noalloc_scratch_init(c->device))) {
         (void)hipFree(c->d_err);
+        (void)hipFree(c->d_mix);
         delete c;
         return r;
     }
@@ -593,6 +599,7 @@ int fhdx_ctx_destroy(fhdx_ctx* c)
     if (c->st_part) (void)hipFree(c->st_part);
     if (c->st_misc) (void)hipFree(c->st_misc);
     if (c->d_err) (void)hipFree(c->d_err);
+    if (c->d_mix) (void)hipFree(c->d_mix);
     delete c;
     return FHDX_OK;
 }

@@ -92,6 +92,30 @@ inline DevParams make_dev_params(const fhdx_params& p)
     return d;
 }
 
+// The mixture table of a parameter set (MixTab): the operations of the transport formulas, on the host.
+inline MixTab make_mix_tab(const fhdx_params& p)
+{
+    MixTab m{};
+    for (int i = 0; i < p.nspecies; ++i) {
+        m.mm[i] = p.molmass[i] * (p.k_B / p.Runiv);
+        m.rmm[i] = 1. / m.mm[i];
+        m.mk[i] = m.mm[i] * p.k_B;
+    }
+    for (int i = 0; i < p.nspecies; ++i)
+        for (int j = 0; j < p.nspecies; ++j) {
+            const double mi = m.mm[i], mj = m.mm[j];
+            m.dia[i][j] = 0.5 * (p.diameter[i] + p.diameter[j]);
+            m.sum[i][j] = mi + mj;
+            m.rsum[i][j] = 1. / m.sum[i][j];
+            m.mu[i][j] = mi * mj / (mi + mj);
+            m.rmu[i][j] = 1. / m.mu[i][j];
+            m.visc[i][j] = 1.0 + 0.6 * mj / mi;
+            m.cond[i][j] = 7.5 * mi / mj + 6.25 * mj / mi - 3.0 * mj / mi + 4.0;
+        }
+    for (int i = 0; i < p.nspecies; ++i) m.c5[i] = 5.0 / (16.0 * m.dia[i][i] * m.dia[i][i]);
+    return m;
+}
+
 inline NoiseKey make_noise_key(uint64_t seed, uint64_t step, uint32_t instance)
 {
     NoiseKey k;

@@ -26,6 +26,7 @@ struct RefWorkspace {
 struct fhdx_ctx {
     fhdx_params p;
     fhdx::DevParams dp;
+    fhdx::MixTab* d_mix = nullptr;  // dp.mix
     int device = 0;
     int* d_err = nullptr;  // device-side error flags (bit 0: mass fraction outside (0,1))
     RefWorkspace ref;

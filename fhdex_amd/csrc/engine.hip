@@ -204,6 +204,7 @@ int engine_create(int max_inst, uint64_t budget, Engine** out)
     if (r == hipSuccess) r = hipMemset(e->d_inst, 0, sizeof(Inst) * max_inst);
     if (r == hipSuccess) r = hipMalloc((void**)&e->d_err, sizeof(int) * max_inst);
     if (r == hipSuccess) r = hipMemset(e->d_err, 0, sizeof(int) * max_inst);
+    if (r == hipSuccess) r = hipMalloc((void**)&e->d_mix, sizeof(MixTab) * max_inst);
     if (r == hipSuccess) r = hipMalloc((void**)&e->d_active, sizeof(int) * max_inst);
     if (r == hipSuccess) r = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
     if (r != hipSuccess) {
@@ -241,6 +242,7 @@ int engine_destroy(Engine* e)
     for (EngineSlot& s : e->slots) free_slot(s);
     if (e->d_inst) (void)hipFree(e->d_inst);
     if (e->d_err) (void)hipFree(e->d_err);
+    if (e->d_mix) (void)hipFree(e->d_mix);
     if (e->d_active) (void)hipFree(e->d_active);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
@@ -297,6 +299,8 @@ int engine_add(Engine* e, const fhdx_params& p, double dt, uint64_t seed, uint64
     s.p = p;
     Inst& d = s.desc;
     d.P = make_dev_params(p);
+    d.P.mix = e->d_mix + sid;
+    const MixTab mix = make_mix_tab(p);
     d.G = grid_of(d.P);
     const int NS = p.nspecies, nv = 5 + NS;
     const RecLayout L{NS};
@@ -333,6 +337,7 @@ int engine_add(Engine* e, const fhdx_params& p, double dt, uint64_t seed, uint64
                                                                                p.n_cells[1], p.n_cells[2], d.nghost);
     FHDX_HIP_TRY(hipGetLastError());
     FHDX_HIP_TRY(hipMemcpyAsync(e->d_inst + sid, &d, sizeof(Inst), hipMemcpyHostToDevice, e->stream));
+    FHDX_HIP_TRY(hipMemcpyAsync(e->d_mix + sid, &mix, sizeof(MixTab), hipMemcpyHostToDevice, e->stream));
     FHDX_HIP_TRY(hipMemsetAsync(e->d_err + sid, 0, sizeof(int), e->stream));
     FHDX_HIP_TRY(hipStreamSynchronize(e->stream));
     e->dirty = true;

@@ -51,6 +51,7 @@ struct Engine {
     std::vector<EngineSlot> slots;
     Inst* d_inst = nullptr;
     int* d_err = nullptr;
+    MixTab* d_mix = nullptr;  // one mixture table per slot
     hipStream_t stream = nullptr;
     // work tables per species count (index ns-2): cell chunks
     WorkItem* d_cells[kEngineGroups] = {};

@@ -78,6 +78,21 @@ struct DevChem {
     double T0, Navo;                  // T0_chem; avogadro = Runiv / k_B (common_functions.cpp:775)
 };
 
+// What the Giovangigli transport solves take from the species alone (transport_cell): masses, mean
+// diameters, reduced masses and the factors of the viscosity and conductivity matrices.  The host
+// computes each entry once, with the operations (and so the bits) the cell's formula has; kernels
+// read them through the scalar cache.  In the cell they were most of its divisions: four species, 128^3: the cell
+// kernel 416 us a launch without the table, 277 with it.
+struct MixTab {
+    double mm[MS], rmm[MS];             // molecular mass and its reciprocal
+    double mk[MS];                      // mass times k_B
+    double c5[MS];                      // 5 / (16 d^2)
+    double dia[MS][MS];                 // mean diameter
+    double mu[MS][MS], rmu[MS][MS];     // reduced mass and its reciprocal
+    double sum[MS][MS], rsum[MS][MS];   // sum of the masses and its reciprocal
+    double visc[MS][MS], cond[MS][MS];  // diagonal factors of the two matrices
+};
+
 struct DevParams {
     int ns, nvars, nprim, ngc;
     int n[3];       // domain cells per direction
@@ -100,6 +115,8 @@ struct DevParams {
     int wall[6], bcv[6], bct[6], bcm[6];
     double tw[6], pw[6], rhow[6];  // wall / reservoir temperature; reservoir pressure, density
     double Yw[6][MS], Xw[6][MS];
+
+    const MixTab* mix;  // device memory
 
     __device__ Rcp h(int d) const { return Rcp{dx[d], rdx[d]}; }
     __device__ Rcp M(int n) const { return Rcp{molmass[n], rmolmass[n]}; }
@@ -204,24 +221,27 @@ __device__ inline void cons_to_prim_cell(const DevParams& P, const double* c, do
 
 // Gaussian elimination without pivoting and back substitution (H:1254-1271).
 template <int NS>
-__device__ inline void gio_solve(double (&a)[NS][NS], double* Bi)
+__device__ __forceinline__ void gio_solve(double (&a)[NS][NS], double* Bi)
 {
+    Rcp pivot[NS];
 #pragma unroll
-    for (int j = 0; j < NS - 1; ++j)
+    for (int j = 0; j < NS; ++j) {
+        pivot[j] = rcp_of(a[j][j]);
 #pragma unroll
         for (int i = j + 1; i < NS; ++i) {
-            double fact1 = a[i][j] / a[j][j];
+            double fact1 = a[i][j] / pivot[j];
 #pragma unroll
             for (int k = 0; k < NS; ++k) a[i][k] -= fact1 * a[j][k];
             Bi[i] -= fact1 * Bi[j];
         }
-    Bi[NS - 1] /= a[NS - 1][NS - 1];
+    }
+    Bi[NS - 1] = Bi[NS - 1] / pivot[NS - 1];
 #pragma unroll
     for (int i = NS - 2; i > -1; --i) {
         double sum1 = 0.0;
 #pragma unroll
         for (int j = NS - 1; j > i; --j) sum1 += a[i][j] * Bi[j];
-        Bi[i] = (Bi[i] - sum1) / a[i][i];
+        Bi[i] = (Bi[i] - sum1) / pivot[i];
     }
 }
 
@@ -301,35 +321,30 @@ __device__ inline void hcb_binary(const DevParams& P, double density, double tem
 // D_GIO1 (compressible_functions.H:647-778; D_GIO at :513-646 is the same arithmetic): the
 // three-term series of the multicomponent diffusion matrix, D[j*NS+i] = Diff_ij Ykp_i.
 template <int NS>
-__device__ __forceinline__ void d_gio_series(const double (&Dbin)[NS][NS], const double* Ykp, const double* Xkp,
+__device__ __forceinline__ void d_gio_series(const Rcp (&Dbin)[NS][NS], const double* Ykp, const double* Xkp,
                                              double* D)
 {
-    double Di[NS], Minv[NS], Mmat[NS];
-    double Pm[NS][NS], Zm[NS][NS], PJ[NS][NS], m1[NS][NS], m2[NS][NS], Diff[NS][NS];
+    double Di[NS], Minv[NS], Mmat[NS], PJ[NS][NS];
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
         double term2 = 0.;
 #pragma unroll
         for (int j = 0; j < NS; ++j)
             if (j != i) term2 = term2 + Xkp[j] / Dbin[i][j];
-        Di[i] = (1. - Ykp[i]) / term2;
+        Di[i] = quot(1. - Ykp[i], term2);
     }
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
-        Mmat[i] = Xkp[i] / Di[i];
-        Minv[i] = Di[i] / Xkp[i];
+        Mmat[i] = quot(Xkp[i], Di[i]);
+        Minv[i] = quot(Di[i], Xkp[i]);
     }
+    auto Pm = [&](int i, int j) { return i == j ? -Ykp[j] + 1. : -Ykp[j]; };
+    // Jmat = Minv_i * Zmat_ij, PJ = P * J, a column at a time: Zmat's column is all it needs
 #pragma unroll
-    for (int i = 0; i < NS; ++i)
+    for (int j = 0; j < NS; ++j) {
+        double J[NS];
 #pragma unroll
-        for (int j = 0; j < NS; ++j) {
-            Pm[i][j] = -Ykp[j];
-            if (i == j) Pm[i][j] = Pm[i][j] + 1.;
-        }
-#pragma unroll
-    for (int i = 0; i < NS; ++i)
-#pragma unroll
-        for (int j = 0; j < NS; ++j) {
+        for (int i = 0; i < NS; ++i) {
             double Delta;
             if (i == j) {
                 double term1 = 0.;
@@ -340,50 +355,51 @@ __device__ __forceinline__ void d_gio_series(const double (&Dbin)[NS][NS], const
             } else {
                 Delta = -Xkp[i] * Xkp[j] / Dbin[i][j];
             }
-            Zm[i][j] = -Delta;
+            double Z = -Delta;
+            if (i == j) Z = Z + Mmat[i];
+            J[i] = Minv[i] * Z;
         }
 #pragma unroll
-    for (int i = 0; i < NS; ++i) Zm[i][i] = Zm[i][i] + Mmat[i];
-    // Jmat = Minv_i * Zmat_ij, PJ = P * J
-#pragma unroll
-    for (int i = 0; i < NS; ++i)
-#pragma unroll
-        for (int j = 0; j < NS; ++j) {
+        for (int i = 0; i < NS; ++i) {
             double s = 0.;
 #pragma unroll
-            for (int k = 0; k < NS; ++k) s = s + Pm[i][k] * (Minv[k] * Zm[k][j]);
+            for (int k = 0; k < NS; ++k) s = s + Pm(i, k) * J[k];
             PJ[i][j] = s;
         }
+        if (NS > 4) __builtin_amdgcn_sched_barrier(0);
+    }
+    // Diff <- PJ Diff + P Minv P^T, three times: the columns are independent, so one column's
+    // start, iterate and result are all that is live beside PJ (the whole matrices are 5 NS^2
+    // doubles, past the register file at eight species: 456 bytes of scratch a lane and 253 us for
+    // the cell kernel at 64^3, none and 224 us so; 338 us with neither this nor the table)
 #pragma unroll
-    for (int i = 0; i < NS; ++i)
+    for (int j = 0; j < NS; ++j) {
+        double base[NS], col[NS];
 #pragma unroll
-        for (int j = 0; j < NS; ++j) {
+        for (int i = 0; i < NS; ++i) {
             double scr = 0.;
 #pragma unroll
-            for (int k = 0; k < NS; ++k) scr = scr + Pm[i][k] * Minv[k] * Pm[j][k];
-            m2[i][j] = scr;
-            Diff[i][j] = scr;
+            for (int k = 0; k < NS; ++k) scr = scr + Pm(i, k) * Minv[k] * Pm(j, k);
+            base[i] = scr;
+            col[i] = scr;
         }
 #pragma unroll
-    for (int ll = 0; ll < 3; ++ll) {
+        for (int ll = 0; ll < 3; ++ll) {
+            double next[NS];
 #pragma unroll
-        for (int i = 0; i < NS; ++i)
-#pragma unroll
-            for (int j = 0; j < NS; ++j) {
+            for (int i = 0; i < NS; ++i) {
                 double scr = 0.;
 #pragma unroll
-                for (int k = 0; k < NS; ++k) scr = scr + PJ[i][k] * Diff[k][j];
-                m1[i][j] = scr + m2[i][j];
+                for (int k = 0; k < NS; ++k) scr = scr + PJ[i][k] * col[k];
+                next[i] = scr + base[i];
             }
 #pragma unroll
-        for (int i = 0; i < NS; ++i)
+            for (int i = 0; i < NS; ++i) col[i] = next[i];
+        }
 #pragma unroll
-            for (int j = 0; j < NS; ++j) Diff[i][j] = m1[i][j];
+        for (int i = 0; i < NS; ++i) D[j * NS + i] = col[i] * Ykp[i];
+        if (NS > 4) __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int i = 0; i < NS; ++i)
-#pragma unroll
-        for (int j = 0; j < NS; ++j) D[j * NS + i] = Diff[i][j] * Ykp[i];
 }
 
 // ---- transport_type 2: IdealMixtureTransportVW (compressible_functions.H:1047-1150) ----------
@@ -606,7 +622,8 @@ __device__ inline int vw_transport(const DevParams& P, double density, double T,
 {
     const double kB = P.k_B, pi = 3.1415926535897932;
     double mk[NS], xx[NS], yy[NS];
-    double Dflat[NS * NS], om[NS * NS], a1[NS * NS], a2[NS * NS], ab[NS * NS], Dbin[NS][NS];
+    double Dflat[NS * NS], om[NS * NS], a1[NS * NS], a2[NS * NS], ab[NS * NS];
+    Rcp Dbin[NS][NS];
     for (int n = 0; n < NS; ++n) mk[n] = P.molmass[n] * (kB / P.Runiv);
     for (int ii = 0; ii < NS; ++ii) {
         double sumXk = 0.;
@@ -630,7 +647,7 @@ __device__ inline int vw_transport(const DevParams& P, double density, double T,
             ab[i * NS + j] = 8.0 / (3.0 * kB) * mu * mu * (-.5 * s11bar);
             Dflat[i * NS + j] = 3.0 / 16.0 * sqrt(2.0 * pi * vw_cube(kB) * (mi + mj) / mi / mj) /
                                 (pi * vw_sq(diamat)) * T * sqrtT / pressure;
-            Dbin[i][j] = Dflat[i * NS + j];
+            Dbin[i][j] = rcp_of(Dflat[i * NS + j]);
             om[i * NS + j] = sqrt(pi * kB / (2.0 * mu)) * vw_sq(diamat) * sqrtT;
             a1[i * NS + j] = (5.0 / (kB) * mi * mj / (mi + mj) * Fij * s11bar) / sqrtT;
             a2[i * NS + j] = (5.0 / (kB) * mi * mj * mi * mj / (vw_cube(mi + mj)) * Fijstar * s11bar) / sqrtT;
@@ -673,7 +690,7 @@ __device__ inline int transport_cell_vw(const DevParams& P, double rho, double T
 // Transport coefficients of one cell (transCoeffs.cpp:37-88).  chi[NS], D[NS*NS] out.
 // Returns true if a mass fraction lies outside (0,1) (the reference aborts there).
 template <int NS>
-__device__ inline bool transport_cell(const DevParams& P, double rho, double T, double p,
+__device__ __forceinline__ bool transport_cell(const DevParams& P, double rho, double T, double p,
                                       const double* Yraw, Transport& tr, double* chi, double* D)
 {
     double Yk[NS];
@@ -686,8 +703,9 @@ __device__ inline bool transport_cell(const DevParams& P, double rho, double T, 
         Yk[n] = clamp01(y);
         sumYk += Yk[n];
     }
+    const Rcp sum = rcp_of(sumYk);
 #pragma unroll
-    for (int n = 0; n < NS; ++n) Yk[n] /= sumYk;
+    for (int n = 0; n < NS; ++n) Yk[n] = Yk[n] / sum;
 
     if constexpr (NS == 2) {
         if (P.transport_type == 3) {  // Hirschfelder-Curtiss-Bird, binary (transCoeffs.cpp:71-75)
@@ -705,65 +723,60 @@ __device__ inline bool transport_cell(const DevParams& P, double rho, double T, 
         }
     }
 
+    // the constant address space: uniform entries come by scalar loads
+    const MixTab& m = *(const MixTab*)(const MixTab __attribute__((address_space(4)))*)P.mix;
     const double pi = 3.1415926535897932;
-    double mm[NS], Xk[NS], Xkp[NS], Ykp[NS], eta1[NS], rhs[NS], Bi[NS];
-    double mu[NS][NS], diam[NS][NS], Dbin[NS][NS], amat[NS][NS];
-#pragma unroll
-    for (int n = 0; n < NS; ++n) mm[n] = P.molmass[n] * (P.k_B / P.Runiv);
+    constexpr Rcp rpi{3.1415926535897932, 1. / 3.1415926535897932};
+    double Xk[NS], Xkp[NS], Ykp[NS], eta1[NS], rhs[NS], Bi[NS];
+    double amat[NS][NS];
+    Rcp Dbin[NS][NS];
     double mbar = 0.0;
 #pragma unroll
-    for (int n = 0; n < NS; ++n) mbar += Yk[n] / mm[n];
-    mbar = 1.0 / mbar;
+    for (int n = 0; n < NS; ++n) mbar += Yk[n] / Rcp{m.mm[n], m.rmm[n]};
+    const Rcp rbar = rcp_of(quot(1.0, mbar));
+    mbar = rbar.b;
     double Xksum = 0.0;
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
-        Xk[n] = Yk[n] * mbar / mm[n];
+        Xk[n] = Yk[n] * mbar / Rcp{m.mm[n], m.rmm[n]};
         Xksum += Xk[n];
     }
 #pragma unroll
     for (int n = 0; n < NS; ++n) Xkp[n] = Xk[n] + 1.0e-16 * (Xksum / double(NS) - Xk[n]);
 #pragma unroll
-    for (int n = 0; n < NS; ++n) Ykp[n] = Xkp[n] * mm[n] / mbar;
-#pragma unroll
-    for (int i = 0; i < NS; ++i)
-#pragma unroll
-        for (int j = 0; j < NS; ++j) {
-            diam[i][j] = 0.5 * (P.diameter[i] + P.diameter[j]);
-            mu[i][j] = mm[i] * mm[j] / (mm[i] + mm[j]);
-        }
+    for (int n = 0; n < NS; ++n) Ykp[n] = Xkp[n] * m.mm[n] / rbar;
     const double kT = P.k_B * T;
+    // the binary diffusion coefficients (symmetric) as the divisors they are below
+    const double kT3 = 2.0 * pi * kT * kT * kT;
 #pragma unroll
     for (int i = 0; i < NS; ++i)
 #pragma unroll
-        for (int j = 0; j < NS; ++j)
-            Dbin[i][j] = (3.0 / 16.0) * sqrt(2.0 * pi * kT * kT * kT / mu[i][j]) /
-                         (p * pi * diam[i][j] * diam[i][j]);
-    const double AKL = 1.0, BKL = 1.0, CKL = 1.0;
+        for (int j = i; j < NS; ++j) {
+            const double root_mu = root(kT3 / Rcp{m.mu[i][j], m.rmu[i][j]});
+            Dbin[i][j] = rcp_of(quot((3.0 / 16.0) * root_mu, p * pi * m.dia[i][j] * m.dia[i][j]));
+            Dbin[j][i] = Dbin[i][j];
+        }
 
     // viscosity
 #pragma unroll
-    for (int i = 0; i < NS; ++i)
-        eta1[i] = 5.0 / (16.0 * diam[i][i] * diam[i][i]) * sqrt(mm[i] * P.k_B * T / pi);
+    for (int i = 0; i < NS; ++i) eta1[i] = m.c5[i] * root(m.mk[i] * T / rpi);
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
         rhs[i] = Xkp[i];
         Bi[i] = rhs[i];
-#pragma unroll
-        for (int j = 0; j < NS; ++j) {
-            if (i == j) {
-                amat[i][i] = Xkp[i] * Xkp[i] / eta1[i];
-#pragma unroll
-                for (int k = 0; k < NS; ++k)
-                    if (k != i)
-                        amat[i][i] += 2.0 * kT * Xkp[i] * Xkp[k] /
-                                      (p * Dbin[i][k] * (mm[i] + mm[k])) *
-                                      (1.0 + 0.6 * mm[k] / mm[i] * AKL);
-            } else {
-                amat[i][j] = 2.0 * kT * Xkp[i] * Xkp[j] / (p * Dbin[i][j] * (mm[i] + mm[j])) *
-                             (0.6 * AKL - 1.0);
-            }
-        }
+        amat[i][i] = quot(Xkp[i] * Xkp[i], eta1[i]);
     }
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+            if (k != i) {
+                const int lo = i < k ? i : k, hi = i < k ? k : i;
+                const Rcp den = rcp_of(p * Dbin[lo][hi].b * m.sum[lo][hi]);
+                const double q = 2.0 * kT * Xkp[i] * Xkp[k] / den;
+                amat[i][i] += q * m.visc[i][k];
+                amat[i][k] = q * (0.6 - 1.0);
+            }
     gio_solve<NS>(amat, Bi);
     double e = 0.0;
 #pragma unroll
@@ -776,45 +789,39 @@ __device__ inline bool transport_cell(const DevParams& P, double rho, double T, 
     for (int i = 0; i < NS; ++i) {
         rhs[i] = 2.5 * Xkp[i];
         Bi[i] = rhs[i];
-#pragma unroll
-        for (int j = 0; j < NS; ++j) {
-            if (i == j) {
-                amat[i][i] = Xkp[i] * Xkp[i] / Dbin[i][j] * 2.0 * AKL;
-#pragma unroll
-                for (int k = 0; k < NS; ++k)
-                    if (k != i)
-                        amat[i][i] += Xkp[i] * Xkp[k] / Dbin[i][k] * mu[i][k] / (mm[i] + mm[k]) *
-                                      (7.5 * mm[i] / mm[k] + 6.25 * mm[k] / mm[i] -
-                                       3.0 * mm[k] / mm[i] * BKL + 4.0 * AKL);
-            } else {
-                amat[i][j] = -1.0 * Xkp[i] * Xkp[j] / Dbin[i][j] * mu[i][j] / (mm[i] + mm[j]) *
-                             (55.0 / 4.0 - 3.0 * BKL - 4.0 * AKL);
-            }
-        }
+        amat[i][i] = Xkp[i] * Xkp[i] / Dbin[i][i] * 2.0;
     }
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+            if (k != i) {
+                const int lo = i < k ? i : k, hi = i < k ? k : i;
+                const double q = Xkp[lo] * Xkp[hi] / Dbin[lo][hi] * m.mu[lo][hi] / Rcp{m.sum[lo][hi], m.rsum[lo][hi]};
+                amat[i][i] += q * m.cond[i][k];
+                amat[i][k] = -q * (55.0 / 4.0 - 3.0 - 4.0);
+            }
     gio_solve<NS>(amat, Bi);
     double kap = 0.0;
 #pragma unroll
     for (int i = 0; i < NS; ++i) kap += rhs[i] * Bi[i];
-    kap *= p / T;
+    kap *= quot(p, T);
     tr.kappa = kap;
 
     // thermal diffusion ratios
 #pragma unroll
+    for (int i = 0; i < NS; ++i) amat[i][i] = 0.0;
+#pragma unroll
     for (int i = 0; i < NS; ++i)
 #pragma unroll
-        for (int j = 0; j < NS; ++j) {
-            if (i == j) {
-                amat[i][i] = 0.0;
-#pragma unroll
-                for (int k = 0; k < NS; ++k)
-                    if (k != i)
-                        amat[i][i] -= 0.5 * Xkp[k] / Dbin[i][k] * mm[k] / (mm[i] + mm[k]) *
-                                      (6.0 * CKL - 5.0);
-            } else {
-                amat[i][j] = 0.5 * Xkp[j] / Dbin[i][j] * mm[i] / (mm[i] + mm[j]) * (6.0 * CKL - 5.0);
+        for (int k = 0; k < NS; ++k)
+            if (k != i) {
+                const int lo = i < k ? i : k, hi = i < k ? k : i;
+                const Rcp sm{m.sum[lo][hi], m.rsum[lo][hi]};
+                const double x = 0.5 * Xkp[k] / Dbin[lo][hi];
+                amat[i][i] -= x * m.mm[k] / sm;
+                amat[i][k] = x * m.mm[i] / sm;
             }
-        }
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
         double c = 0.0;

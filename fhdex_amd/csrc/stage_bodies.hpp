@@ -131,7 +131,7 @@ __device__ inline void ghost_body(const Arr& a, int nc, int g, int n0, int n1, i
 // The record of cell (i,j,k) from its conserved values c[] (held in registers by the caller).
 // VW: transport_type 2 (Valk-Waldmann); otherwise the type the parameters name (1 or 3).
 template <int NS, bool VW = false>
-__device__ inline void cell_record(const DevParams& P, const double* c, const Fld& R, int* err, int i, int j, int k,
+__device__ __forceinline__ void cell_record(const DevParams& P, const double* c, const Fld& R, int* err, int i, int j, int k,
                                    unsigned cb)
 {
     const RecLayout L{NS};
@@ -177,7 +177,7 @@ __device__ inline void cell_record(const DevParams& P, const double* c, const Fl
 }
 
 template <int NS, bool VW = false>
-__device__ inline void cell_body(const DevParams& P, const Fld& U, const Fld& R, int* err, int i, int j, int k,
+__device__ __forceinline__ void cell_body(const DevParams& P, const Fld& U, const Fld& R, int* err, int i, int j, int k,
                                  unsigned cb)
 {
     double c[NS + 5];
@@ -707,7 +707,7 @@ struct ChemStage {
 
 // div[] = (fx(i+1)-fx(i))/dx + (fy(j+1)-fy(j))/dy + (fz(k+1)-fz(k))/dz, evaluated left to right.
 template <int NS>
-__device__ inline void update_from_div(const DevParams& P, const Fld& out, const Fld& u0, const Fld& us,
+__device__ __forceinline__ void update_from_div(const DevParams& P, const Fld& out, const Fld& u0, const Fld& us,
                                        const double* div, double dt, int mode, const Fld& prim, int write_prim, int i,
                                        int j, int k, unsigned cb, const Fld* rec_next = nullptr, int* err = nullptr,
                                        const ChemStage* chem = nullptr)
@@ -758,7 +758,7 @@ __device__ inline void update_from_div(const DevParams& P, const Fld& out, const
 }
 
 template <int NS>
-__device__ inline void update_body(const DevParams& P, const Fld& out, const Fld& u0, const Fld& us, const Fld& fx,
+__device__ __forceinline__ void update_body(const DevParams& P, const Fld& out, const Fld& u0, const Fld& us, const Fld& fx,
                                    const Fld& fy, const Fld& fz, double dt, int mode, const Fld& prim, int write_prim,
                                    int i, int j, int k, unsigned cb, const Fld* rec_next = nullptr,
                                    int* err = nullptr, const ChemStage* chem = nullptr)
