@@ -405,24 +405,10 @@ int ensure_ref_workspace(fhdx_ctx* c)
     auto cell = [&](fhdx_fab& f, int nc) {
         if (!r) r = alloc_fab(w.blocks, f, -g, -g, -g, n0 - 1 + g, n1 - 1 + g, n2 - 1 + g, nc);
     };
-    auto face = [&](fhdx_fab& f, int d, int nc) {
-        if (!r) r = alloc_fab(w.blocks, f, 0, 0, 0, n0 - 1 + (d == 0), n1 - 1 + (d == 1), n2 - 1 + (d == 2), nc);
-    };
-    auto node = [&](fhdx_fab& f) {
-        if (!r) r = alloc_fab(w.blocks, f, 0, 0, 0, n0, n1, n2, 1);
-    };
-    for (int d = 0; d < 3; ++d) {
-        face(w.sA[d], d, nv);
-        face(w.sB[d], d, nv);
-    }
-    node(w.rA);
-    node(w.rB);
-    if (c->p.nreaction > 0) {
-        cell(w.source, nv);  // components 0..4 stay zero (main_driver.cpp:241-242)
-        cell(w.ranA, c->p.nreaction);
-        cell(w.ranB, c->p.nreaction);
-        cell(w.ran, c->p.nreaction);
-    }
+    cell(w.source, nv);  // components 0..4 stay zero (main_driver.cpp:241-242)
+    cell(w.ranA, c->p.nreaction);
+    cell(w.ranB, c->p.nreaction);
+    cell(w.ran, c->p.nreaction);
     if (r) return r;
     FHDX_HIP_TRY(hipDeviceSynchronize());
     w.ready = true;
@@ -456,8 +442,9 @@ struct StageArrays {
 // transport on the grown box, the stage-weighted noise, calculateFlux, the chemistry source,
 // the stage combination and prim on the valid cells.  The ghost cells of the output state and
 // of prim are left to the caller (FillBoundary, then setBC: timeStep.cpp:204-209, 309-314,
-// 417-425).
-int rk3_stage(const fhdx_ctx* c, const DevParams& P, const StageArrays& A, int st, double dt, hipStream_t s)
+// 417-425).  K: the noise is drawn in place from this key; null: it is in A's sets.  keep: see FluxArgs.
+int rk3_stage(const fhdx_ctx* c, const DevParams& P, const StageArrays& A, const NoiseKey* K, bool keep, int st,
+              double dt, hipStream_t s)
 {
     const bool chem = c->p.nreaction > 0;
     const int nv = P.nvars;
@@ -486,24 +473,20 @@ int rk3_stage(const fhdx_ctx* c, const DevParams& P, const StageArrays& A, int s
     a.cons = make_arr(in[st]);
     int r;
     if ((r = ref_transport(P, a.prim, a.eta, a.zeta, a.kappa, a.chi, a.D, c->d_err, s))) return r;
-    if (P.stoch_on) {
-        // the stochastic and node passes form stochFlux = A + w B and rancorn themselves
-        a.weigh = true;
-        for (int d = 0; d < 3; ++d) {
-            a.nA[d] = make_arr(A.sA[d]);
-            a.nB[d] = make_arr(A.sB[d]);
-        }
-        a.rA = make_arr(A.rA);
-        a.rB = make_arr(A.rB);
-        a.w = ws[st];
+    a.noise.w = ws[st];
+    if (K) {
+        a.noise.mode = kNoisePhilox;
+        a.noise.K = *K;
     } else {
-        double* const dst[4] = {A.stochFlux[0].p, A.stochFlux[1].p, A.stochFlux[2].p, A.rancorn.p};
-        const double* const la[4] = {A.sA[0].p, A.sA[1].p, A.sA[2].p, A.rA.p};
-        const double* const lb[4] = {A.sB[0].p, A.sB[1].p, A.sB[2].p, A.rB.p};
-        const long np[4] = {npts(A.stochFlux[0]), npts(A.stochFlux[1]), npts(A.stochFlux[2]), npts(A.rancorn)};
-        const int lnc[4] = {nv, nv, nv, 1}, lc0[4] = {1, 1, 1, 0};
-        if ((r = ref_lincomb4(dst, la, lb, np, lnc, lc0, ws[st], s))) return r;
+        a.noise.mode = kNoiseSets;
+        for (int d = 0; d < 3; ++d) {
+            a.noise.A[d] = make_arr(A.sA[d]);
+            a.noise.B[d] = make_arr(A.sB[d]);
+        }
+        a.noise.rA = make_arr(A.rA);
+        a.noise.rB = make_arr(A.rB);
     }
+    a.keep = keep;
     const int fnc[3] = {A.flux[0].ncomp, A.flux[1].ncomp, A.flux[2].ncomp};
     if ((r = ref_calculate_flux(P, a, const_cast<int*>(fnc), s))) return r;
     Arr src{};
@@ -514,19 +497,18 @@ int rk3_stage(const fhdx_ctx* c, const DevParams& P, const StageArrays& A, int s
             return r;
         if ((r = ref_chem_source(P, a.prim, src, make_arr(A.ranchem), dt, s))) return r;
     }
-    if ((r = ref_stage(P, make_arr(out[st]), make_arr(A.cu), make_arr(in[st]), fl, src, dt, st, s))) return r;
-    return ref_c2p(P, a.prim, make_arr(out[st]), s);
+    return ref_stage(P, make_arr(out[st]), make_arr(A.cu), make_arr(in[st]), fl, src, a.prim, dt, st, s);
 }
 
 // The reference RK3step with the reference's arrays (timeStep.cpp:11-427) on a single-box
 // domain: each stage, then the periodic images and setBC of the new state and prim.
-int rk3_ref(fhdx_ctx* c, const StageArrays& A, double dt, hipStream_t s)
+int rk3_ref(fhdx_ctx* c, const StageArrays& A, const NoiseKey* K, double dt, hipStream_t s)
 {
     const DevParams& P = c->dp;
     const fhdx_fab out[3] = {A.cup, A.cup2, A.cu};
     for (int st = 0; st < 3; ++st) {
         int r;
-        if ((r = rk3_stage(c, P, A, st, dt, s))) return r;
+        if ((r = rk3_stage(c, P, A, K, st == 2, st, dt, s))) return r;
         if ((r = ref_fill_boundary2(P, make_arr(out[st]), P.nvars, make_arr(A.prim), P.nprim, s))) return r;
         if ((r = ref_set_bc(P, make_arr(A.prim), make_arr(out[st]), s))) return r;  // timeStep.cpp:209, 314, 425
     }
@@ -790,26 +772,20 @@ int fhdx_rk3_step_ref(fhdx_ctx* c, fhdx_fab cu, fhdx_fab cup, fhdx_fab cup2, fhd
         }
         A.rA = *rancornA;
         A.rB = *rancornB;
-        return rk3_ref(c, A, dt, s);
+        return rk3_ref(c, A, nullptr, dt, s);
     }
-    int r = ensure_ref_workspace(c);
-    if (r) return r;
-    RefWorkspace& w = c->ref;
-    if ((r = fhdx_fill_noise(c, seed, step, 0, w.sA, w.sB, w.rA, w.rB, stream))) return r;
-    if (c->p.nreaction > 0 &&
-        (r = ref_fill_chem_noise(c->dp, make_noise_key(seed, step, 0), make_arr(w.ranA), make_arr(w.ranB), s)))
-        return r;
-    for (int d = 0; d < 3; ++d) {
-        A.sA[d] = w.sA[d];
-        A.sB[d] = w.sB[d];
+    const NoiseKey K = make_noise_key(seed, step, 0);
+    if (c->p.nreaction > 0) {
+        int r = ensure_ref_workspace(c);
+        RefWorkspace& w = c->ref;
+        if (!r) r = ref_fill_chem_noise(c->dp, K, make_arr(w.ranA), make_arr(w.ranB), s);
+        if (r) return r;
+        A.source = w.source;
+        A.ranchem = w.ran;
+        A.ranchemA = w.ranA;
+        A.ranchemB = w.ranB;
     }
-    A.rA = w.rA;
-    A.rB = w.rB;
-    A.source = w.source;
-    A.ranchem = w.ran;
-    A.ranchemA = w.ranA;
-    A.ranchemB = w.ranB;
-    return rk3_ref(c, A, dt, s);
+    return rk3_ref(c, A, &K, dt, s);
 }
 
 int fhdx_rk3_stage_ref(fhdx_ctx* c, int stage, fhdx_fab cu, fhdx_fab cup, fhdx_fab cup2, fhdx_fab prim,
@@ -877,7 +853,7 @@ int fhdx_rk3_stage_ref(fhdx_ctx* c, int stage, fhdx_fab cu, fhdx_fab cup, fhdx_f
         A.ranchemA = ranchemA;
         A.ranchemB = ranchemB;
     }
-    return rk3_stage(c, box_params(c, b), A, stage, dt, S(stream));
+    return rk3_stage(c, box_params(c, b), A, nullptr, true, stage, dt, S(stream));
 }
 
 int fhdx_rk3_step(fhdx_ctx* c, fhdx_fab cu, fhdx_fab prim, double dt, uint64_t seed, uint64_t step, void* stream)

@@ -13,14 +13,12 @@ namespace fhdx {
 void stag_workspace_free(StagWorkspace* w);
 }
 
-// Device buffers a context owns for the reference-shaped RK3 step: the step's two noise sets
-// when the caller supplies none, and the chemistry arrays.  Every other array of that step is
-// the caller's (the reference's RK3step argument list).
+// Device buffers a context owns for the reference-shaped RK3 step with chemistry.  Every other array
+// of that step is the caller's (the reference's RK3step argument list).
 struct RefWorkspace {
     bool ready = false;
     std::vector<double*> blocks;
-    fhdx_fab sA[3], sB[3], rA, rB;
-    fhdx_fab source, ranA, ranB, ran;  // chemistry (nreaction > 0): source, reaction noise A, B, A + w B
+    fhdx_fab source, ranA, ranB, ran;  // source, reaction noise A, B, A + w B
 };
 
 struct fhdx_ctx {

@@ -5,20 +5,28 @@
 
 namespace fhdx {
 
+// The noise of a calculateFlux call: ran[] and rancorn hold it weighted already (calculateFlux's
+// own arguments), or it is A + w B of a stage, from the caller's sets or drawn in place from key K.  In
+// the last two cases the kernels store the weighted noise into rancorn (the faces read it there)
+// and, with keep, ran[], as the reference's MultiFab::LinComb leaves them (timeStep.cpp:99-107).
+constexpr int kNoiseWeighted = 0, kNoiseSets = 1, kNoisePhilox = 2;
+
+struct FaceNoise {
+    int mode = kNoiseWeighted;
+    Arr A[3], B[3], rA, rB;
+    NoiseKey K{};
+    double w = 0.;
+};
+
 // Views of every array calculateFlux touches (flux.cpp:4-16).
-// With weigh set, ran[] and rancorn are outputs: the stochastic pass reads the step's noise sets
-// A, B and stores ran = 1*A + w*B (component 0 zero) for each face it computes, and the node pass
-// rancorn likewise (the reference's MultiFab::LinComb, timeStep.cpp:99-107), so no separate
-// weighting launch runs; otherwise ran[] and rancorn hold the weighted noise already.
 struct FluxArgs {
     Arr cons, prim, eta, zeta, kappa, chi, D;
     Arr flux[3], ran[3];
     Arr corn[3][3];  // [derivative direction][velocity component]: cornx/corny/cornz
     Arr visccorn, rancorn;
     double dt;
-    bool weigh = false;
-    Arr nA[3], nB[3], rA, rB;
-    double w = 0.;
+    FaceNoise noise;
+    bool keep = true;  // also store ran[] and the flux components past nvars, which no later pass reads
 };
 
 int ref_c2p(const DevParams& P, Arr prim, Arr cons, hipStream_t s);
@@ -32,17 +40,15 @@ int ref_set_bc(const DevParams& P, Arr prim, Arr cons, hipStream_t s);
 int fill_value(double* p, long n, double v, hipStream_t s);
 // flux_ncomp: the components of each flux FAB (>= nvars + 4)
 int ref_calculate_flux(const DevParams& P, const FluxArgs& a, int flux_ncomp[3], hipStream_t s);
-// source: the source MultiFab (p == nullptr: zero)
-int ref_stage(const DevParams& P, Arr out, Arr u0, Arr us, const Arr flux[3], Arr source, double dt, int mode,
-              hipStream_t s);
+// The stage combination and conservedToPrimitive of its result on the valid cells; source: the source
+// MultiFab (p == nullptr: zero).
+int ref_stage(const DevParams& P, Arr out, Arr u0, Arr us, const Arr flux[3], Arr source, Arr prim, double dt,
+              int mode, hipStream_t s);
 // compute_compressible_chemistry_source_CLE over the valid cells; reaction noise sets A, B.
 int ref_chem_source(const DevParams& P, Arr prim, Arr source, Arr ranchem, double dt, hipStream_t s);
 int ref_fill_chem_noise(const DevParams& P, const NoiseKey& K, Arr A, Arr B, hipStream_t s);
 int ref_lincomb(double* dst, const double* a, const double* b, long npts, int nc, int c0, double w,
                 hipStream_t s);
-// The same for four arrays at once (a stage's three face noise arrays and the node array).
-int ref_lincomb4(double* const dst[4], const double* const a[4], const double* const b[4], const long npts[4],
-                 const int nc[4], const int c0[4], double w, hipStream_t s);
 int ref_fill_noise(const DevParams& P, const NoiseKey& K, const Arr A[3], const Arr B[3], Arr rA, Arr rB,
                    hipStream_t s);
 

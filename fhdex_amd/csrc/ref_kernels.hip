@@ -6,6 +6,7 @@
 // arrays (fhdx_calculate_flux, fhdx_rk3_step_ref).  Arithmetic follows the reference
 // operation by operation (see physics.hpp for why that is required).
 #include "kernels.hpp"
+#include "stage_bodies.hpp"
 
 namespace fhdx {
 
@@ -14,7 +15,7 @@ constexpr int BLK = 256;
 // Edge-viscosity summation order per face direction and edge (pp, mp, pm, mm): offsets of the
 // eta cell then of the T cell relative to the face index, flux.cpp:117-135 (x), 481-499 (y),
 // 847-865 (z, including the eta(k-2)*T(k) terms of 857-858).
-__constant__ signed char c_mu_order[3][4][8][6] = {
+__device__ constexpr signed char c_mu_order[3][4][8][6] = {
     {{{0,0,0,0,0,0},{-1,0,0,-1,0,0},{0,1,0,0,1,0},{-1,1,0,-1,1,0},{0,0,1,0,0,1},{-1,0,1,-1,0,1},{0,1,1,0,1,1},{-1,1,1,-1,1,1}},
      {{0,-1,0,0,-1,0},{-1,-1,0,-1,-1,0},{0,0,0,0,0,0},{-1,0,0,-1,0,0},{0,-1,1,0,-1,1},{-1,-1,1,-1,-1,1},{0,0,1,0,0,1},{-1,0,1,-1,0,1}},
      {{0,0,-1,0,0,-1},{-1,0,-1,-1,0,-1},{0,1,-1,0,1,-1},{-1,1,-1,-1,1,-1},{0,0,0,0,0,0},{-1,0,0,-1,0,0},{0,1,0,0,1,0},{-1,1,0,-1,1,0}},
@@ -29,14 +30,14 @@ __constant__ signed char c_mu_order[3][4][8][6] = {
      {{-1,-1,0,-1,-1,0},{0,-1,0,0,-1,0},{-1,0,0,-1,0,0},{0,0,0,0,0,0},{-1,-1,-1,-1,-1,-1},{0,-1,-1,0,-1,-1},{-1,0,-1,-1,0,-1},{0,0,-1,0,0,-1}}}};
 
 // Node (rancorn) offsets of the pp, mp, pm, mm edges (flux.cpp:277-280, 644-647, 1011-1014).
-__constant__ signed char c_rc_node[3][4][3] = {{{0, 1, 1}, {0, 0, 1}, {0, 1, 0}, {0, 0, 0}},
+__device__ constexpr signed char c_rc_node[3][4][3] = {{{0, 1, 1}, {0, 0, 1}, {0, 1, 0}, {0, 0, 0}},
                                                {{1, 0, 1}, {0, 0, 1}, {1, 0, 0}, {0, 0, 0}},
                                                {{1, 1, 0}, {0, 1, 0}, {1, 0, 0}, {0, 0, 0}}};
 
 // Wall faces: the four edge-viscosity cells in the ghost layer (normal offset -1 at a lo face,
 // 0 at a hi face), transverse offsets per face direction and edge in the reference's order
 // (flux.cpp:137-156 x, 501-520 y, 867-886 z).
-__constant__ signed char c_mu_wall[3][4][4][3] = {
+__device__ constexpr signed char c_mu_wall[3][4][4][3] = {
     {{{0, 0, 0}, {0, 1, 0}, {0, 0, 1}, {0, 1, 1}}, {{0, -1, 0}, {0, 0, 0}, {0, -1, 1}, {0, 0, 1}},
      {{0, 0, -1}, {0, 1, -1}, {0, 0, 0}, {0, 1, 0}}, {{0, -1, -1}, {0, 0, -1}, {0, -1, 0}, {0, 0, 0}}},
     {{{1, 0, 0}, {0, 0, 0}, {1, 0, 1}, {0, 0, 1}}, {{-1, 0, 0}, {0, 0, 0}, {-1, 0, 1}, {0, 0, 1}},
@@ -88,12 +89,32 @@ __device__ inline bool box_index(const DevParams& P, long t, int ex, int ey, int
     return true;
 }
 
+// The entry points check that every cell array of a call has one shape, and likewise its face arrays
+// of a direction and its node arrays, so a thread forms one byte offset per kind and every access is a
+// scalar base and that offset (Fld), not an index product of each array's own strides.
+__device__ __forceinline__ Fld fld_of(const Arr& a, const Arr& like) { return Fld{a.p, like.sn, like.sy, like.sz}; }
+__device__ __forceinline__ unsigned off_of(const Arr& a, int i, int j, int k)
+{
+    return (unsigned)((i - a.lo0) + (j - a.lo1) * a.sy + (k - a.lo2) * a.sz) << 3;
+}
+
+// Thread number with the blocks of an XCD contiguous: workgroup b runs on XCD b % 8, and XCD x takes
+// the block numbers [x nb/8, (x+1) nb/8), so the rows and planes that neighbouring blocks share are
+// fetched into one L2 instead of several.
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb)
+{
+    const unsigned xcd = b & 7, r = b >> 3, per = nb >> 3, rem = nb & 7;
+    return xcd * per + (xcd < rem ? xcd : rem) + r;
+}
+
+__device__ __forceinline__ long xcd_thread() { return (long)xcd_block(blockIdx.x, gridDim.x) * BLK + threadIdx.x; }
+
 // ---- cell kernels -------------------------------------------------------------------------
 
 template <int NS>
 __global__ void __launch_bounds__(BLK) k_c2p(DevParams P, Arr prim, Arr cons)
 {
-    long t = (long)blockIdx.x * BLK + threadIdx.x;
+    const long t = xcd_thread();
     int i, j, k;
     if (!box_index(P, t, 0, 0, 0, i, j, k)) return;
     double c[NS + 5], pr[2 * NS + 6];
@@ -105,37 +126,40 @@ __global__ void __launch_bounds__(BLK) k_c2p(DevParams P, Arr prim, Arr cons)
 }
 
 template <int NS, bool VW>
-__global__ void __launch_bounds__(BLK) k_transport(DevParams P, Arr prim, Arr eta, Arr zeta,
-                                                   Arr kappa, Arr chi, Arr Dm, int* err)
+__global__ void __launch_bounds__(BLK) k_transport(DevParams P, Arr prima, Arr etaa, Arr zetaa,
+                                                   Arr kappaa, Arr chia, Arr Da, int* err)
 {
     const int g = P.ngc;
     const int gx = P.bn[0] + 2 * g, gy = P.bn[1] + 2 * g, gz = P.bn[2] + 2 * g;
-    long t = (long)blockIdx.x * BLK + threadIdx.x;
+    const long t = xcd_thread();
     if (t >= (long)gx * gy * gz) return;
     int i, j, k;
     face_index(t, gx, gy, i, j, k);
     i += P.bo[0] - g;
     j += P.bo[1] - g;
     k += P.bo[2] - g;
+    const Fld prim = fld_of(prima, prima), eta = fld_of(etaa, prima), zeta = fld_of(zetaa, prima),
+              kappa = fld_of(kappaa, prima), chi = fld_of(chia, prima), Dm = fld_of(Da, prima);
+    const unsigned cb = off_of(prima, i, j, k);
     double Y[NS], chiv[NS], Dv[NS * NS];
 #pragma unroll
-    for (int n = 0; n < NS; ++n) Y[n] = prim(i, j, k, 6 + n);
+    for (int n = 0; n < NS; ++n) Y[n] = prim(cb, 6 + n);
     Transport tr;
     if constexpr (VW) {  // transport_type 2
-        const int fl = transport_cell_vw<NS>(P, prim(i, j, k, 0), prim(i, j, k, 4), prim(i, j, k, 5), Y, tr, chiv, Dv);
+        const int fl = transport_cell_vw<NS>(P, prim(cb, 0), prim(cb, 4), prim(cb, 5), Y, tr, chiv, Dv);
         if (fl) atomicOr(err, fl);
     } else {
-        bool bad = transport_cell<NS>(P, prim(i, j, k, 0), prim(i, j, k, 4), prim(i, j, k, 5), Y, tr,
+        bool bad = transport_cell<NS>(P, prim(cb, 0), prim(cb, 4), prim(cb, 5), Y, tr,
                                       chiv, Dv);
         if (bad) atomicOr(err, 1);
     }
-    eta(i, j, k) = tr.eta;
-    zeta(i, j, k) = tr.zeta;
-    kappa(i, j, k) = tr.kappa;
+    eta(cb, 0) = tr.eta;
+    zeta(cb, 0) = tr.zeta;
+    kappa(cb, 0) = tr.kappa;
 #pragma unroll
-    for (int n = 0; n < NS; ++n) chi(i, j, k, n) = chiv[n];
+    for (int n = 0; n < NS; ++n) chi(cb, n) = chiv[n];
 #pragma unroll
-    for (int n = 0; n < NS * NS; ++n) Dm(i, j, k, n) = Dv[n];
+    for (int n = 0; n < NS * NS; ++n) Dm(cb, n) = Dv[n];
 }
 
 // Periodic ghost fill of a cell FAB: ghost (i,j,k) <- valid (i mod n, ...) along periodic
@@ -291,50 +315,41 @@ __global__ void __launch_bounds__(BLK) k_fill(double* p, long n, double v)
 // are scaled by sqrt(2) (slip) or 0 (no slip) (:250-280).  StochFlux (boundary.cpp:1392-1970)
 // then scales the face's stochastic fluxes, applied here to the values this thread wrote.
 
-// The step's noise of one stage: with WN the weighted values 1*A + w*B are formed here (and
-// stored into ran for the face, as MultiFab::LinComb leaves them); otherwise ran holds them.
-struct NoiseW {
-    Arr A, B, rA, rB;
-    double w;
+// A face's views and byte offsets: cell (i,j,k) and the one below it, the lower and upper cells of
+// the face averages (both the wall-side cell at a wall), and node (i,j,k).
+struct FaceView {
+    Fld cons, prim, eta, zeta, kappa, chi, Dm, visccorn, rancorn;
+    Fld corn[3][3];
+    unsigned c0, cm, lo, up, nd;
 };
 
-template <int NS, int D, bool WN>
-__device__ __forceinline__ void stoch_body(const DevParams& P, Arr prim, Arr eta, Arr zeta, Arr kappa, Arr chi,
-                                           Arr Dm, Arr fl, Arr ran, Arr rc, const NoiseW& nw, double volinv,
-                                           double dtinv, double dt, long t)
+template <int NS, int D, bool WALL>
+__device__ __forceinline__ void stoch_part(const DevParams& P, const FaceView& V, const WallFace& W, const double* ran,
+                                           double* o, double volinv, double dtinv, double dt, int i, int j, int k)
 {
-    int i, j, k;
-    if (!box_index(P, t, D == 0, D == 1, D == 2, i, j, k)) return;
-    if constexpr (WN) {
-#pragma unroll
-        for (int c = 0; c < NS + 5; ++c)
-            ran(i, j, k, c) = (c < 1) ? 0.0 : 1.0 * nw.A(i, j, k, c) + nw.w * nw.B(i, j, k, c);
-    }
-    const WallFace W = wall_face<D>(P, i, j, k);
-    // lower and upper cells of the face averages; both the wall-side cell at a wall
-    const int il = W.any() ? W.wi : i - (D == 0), jl = W.any() ? W.wj : j - (D == 1),
-              kl = W.any() ? W.wk : k - (D == 2);
-    const int iu = W.any() ? W.wi : i, ju = W.any() ? W.wj : j, ku = W.any() ? W.wk : k;
+    const Fld &prim = V.prim, &eta = V.eta, &zeta = V.zeta, &kappa = V.kappa, &chi = V.chi, &Dm = V.Dm;
+    const unsigned lo = V.lo, up = V.up;
+    const bool wall = WALL && W.any();
+    constexpr Rcp three{3., 1. / 3.};
     const int nv = NS + 5;
 
-    double Tu = prim(iu, ju, ku, 4), Tl = prim(il, jl, kl, 4);
-    double mup = eta(iu, ju, ku) * Tu + eta(il, jl, kl) * Tl;
-    double kp = kappa(iu, ju, ku) * Tu * Tu + kappa(il, jl, kl) * Tl * Tl;
+    double Tu = prim(up, 4), Tl = prim(lo, 4);
+    double mup = eta(up, 0) * Tu + eta(lo, 0) * Tl;
+    double kp = kappa(up, 0) * Tu * Tu + kappa(lo, 0) * Tl * Tl;
     double meanT = 0.5 * (Tu + Tl);
     double w[NS + 5];
-    double fw1 = sqrt(P.k_B * mup * volinv * dtinv);
-    double fw4 = sqrt(P.k_B * kp * volinv * dtinv);
-    w[0] = 0 * ran(i, j, k, 0);
-    w[1] = fw1 * ran(i, j, k, 1);
-    w[2] = fw1 * ran(i, j, k, 2);
-    w[3] = fw1 * ran(i, j, k, 3);
-    w[4] = fw4 * ran(i, j, k, 4);
-    double nweight = sqrt(P.k_B * volinv * dtinv);
+    double fw1 = root(P.k_B * mup * volinv * dtinv);
+    double fw4 = root(P.k_B * kp * volinv * dtinv);
+    w[1] = fw1 * ran[1];
+    w[2] = fw1 * ran[2];
+    w[3] = fw1 * ran[3];
+    w[4] = fw4 * ran[4];
+    double nweight = root(P.k_B * volinv * dtinv);
 
     // tangential-wall factors of the four edges (pp, mp, pm, mm) over transverse axes (A, B)
     constexpr int TA = (D == 0) ? 1 : 0, TB = (D == 2) ? 1 : 2;
     double fac[4] = {1., 1., 1., 1.};
-    if (P.any_wall) {
+    if (WALL) {
         const int idx[3] = {i, j, k};
         double flo[2] = {1., 1.}, fhi[2] = {1., 1.};
         const int ax[2] = {TA, TB};
@@ -355,65 +370,57 @@ __device__ __forceinline__ void stoch_body(const DevParams& P, Arr prim, Arr eta
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         double mu;
-        if (W.any()) {
-            const int oi = W.wi - i, oj = W.wj - j, ok = W.wk - k;  // ghost-layer shift
+        if (wall) {
             double s4 = 0., z4 = 0.;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const signed char* o = c_mu_wall[D][c][q];
-                const int ci = i + oi + o[0], cj = j + oj + o[1], ck = k + ok + o[2];
-                const double T = prim(ci, cj, ck, 4);
-                const double e = eta(ci, cj, ck) * T;
+                const double T = prim(up, 4, o[0], o[1], o[2]);
+                const double e = eta(up, 0, o[0], o[1], o[2]) * T;
                 s4 = (q == 0) ? e : s4 + e;
                 if (P.visc_type == 3 || P.visc_type == -3) {
-                    const double zz = zeta(ci, cj, ck) * T;
+                    const double zz = zeta(up, 0, o[0], o[1], o[2]) * T;
                     z4 = (q == 0) ? zz : z4 + zz;
                 }
             }
-            mu = 0.5 * s4 / 3.;
-            if (P.visc_type == 3 || P.visc_type == -3) mu += (D == 0) ? 0.5 * z4 : 0.5 * z4 / 3.;
+            mu = 0.5 * s4 / three;
+            if (P.visc_type == 3 || P.visc_type == -3) mu += (D == 0) ? 0.5 * z4 : 0.5 * z4 / three;
         } else {
             double s8 = 0.;
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
                 const signed char* o = c_mu_order[D][c][q];
-                double term = eta(i + o[0], j + o[1], k + o[2]) * prim(i + o[3], j + o[4], k + o[5], 4);
+                double term = eta(V.c0, 0, o[0], o[1], o[2]) * prim(V.c0, 4, o[3], o[4], o[5]);
                 s8 = (q == 0) ? term : s8 + term;
             }
-            mu = 0.25 * s8 / 3.;
+            mu = 0.25 * s8 / three;
             if (P.visc_type == 3 || P.visc_type == -3) {
                 double z = 0.;
 #pragma unroll
                 for (int q = 0; q < 8; ++q) {
                     const signed char* o = c_mu_order[D][c][q];
-                    double term = zeta(i + o[0], j + o[1], k + o[2]) * prim(i + o[3], j + o[4], k + o[5], 4);
+                    double term = zeta(V.c0, 0, o[0], o[1], o[2]) * prim(V.c0, 4, o[3], o[4], o[5]);
                     z = (q == 0) ? term : z + term;
                 }
                 mu += 0.25 * z;
             }
         }
         const signed char* nd = c_rc_node[D][c];
-        double rcv;
-        if constexpr (WN) rcv = 1.0 * nw.rA(i + nd[0], j + nd[1], k + nd[2]) + nw.w * nw.rB(i + nd[0], j + nd[1], k + nd[2]);
-        else rcv = rc(i + nd[0], j + nd[1], k + nd[2]);
-        double term = fac[c] * sqrt(mu) * rcv;
+        double term = fac[c] * root(mu) * V.rancorn(V.nd, 0, nd[0], nd[1], nd[2]);
         sum = (c == 0) ? term : sum + term;
     }
     w[1 + D] = w[1 + D] + 0.25 * nweight * sum;
 
-    // this face's flux after the stochastic pass, every one of the nvars + 4 components: the
-    // reference adds to a zeroed array (flux.cpp:24-26), so each term is 0.0 + term
-    double o[NS + 9];
-#pragma unroll
-    for (int n = 0; n < NS + 9; ++n) o[n] = 0.0;
+    // this face's flux after the stochastic pass: the reference adds to a zeroed array
+    // (flux.cpp:24-26), so each term is 0.0 + term
 #pragma unroll
     for (int n = 1; n < 4; ++n) o[n] = 0.0 + w[n];
     o[nv] = 0.0 + w[4];
 
     constexpr int t1 = (D == 0) ? 2 : 1, t2 = (D == 2) ? 2 : 3;
-    double phidiag = w[1 + D] * (prim(il, jl, kl, 1 + D) + prim(iu, ju, ku, 1 + D));
-    double phishear = w[t1] * (prim(il, jl, kl, t1) + prim(iu, ju, ku, t1)) +
-                      w[t2] * (prim(il, jl, kl, t2) + prim(iu, ju, ku, t2));
+    double phidiag = w[1 + D] * (prim(lo, 1 + D) + prim(up, 1 + D));
+    double phishear = w[t1] * (prim(lo, t1) + prim(up, t1)) +
+                      w[t2] * (prim(lo, t2) + prim(up, t2));
     phidiag = -0.5 * phidiag;
     phishear = -0.5 * phishear;
     o[nv + 1] = 0.0 - phidiag;
@@ -424,8 +431,8 @@ __device__ __forceinline__ void stoch_body(const DevParams& P, Arr prim, Arr eta
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             w[5 + s] = 0.;
-            yy[s] = clamp01(prim(il, jl, kl, 6 + s));
-            yyp[s] = clamp01(prim(iu, ju, ku, 6 + s));
+            yy[s] = clamp01(prim(lo, 6 + s));
+            yyp[s] = clamp01(prim(up, 6 + s));
         }
         double sumy = 0., sumyp = 0.;
 #pragma unroll
@@ -433,19 +440,20 @@ __device__ __forceinline__ void stoch_body(const DevParams& P, Arr prim, Arr eta
             sumy += yy[n];
             sumyp += yyp[n];
         }
+        const Rcp ry = rcp_of(sumy), ryp = rcp_of(sumyp);
 #pragma unroll
         for (int n = 0; n < NS; ++n) {
-            yy[n] /= sumy;
-            yyp[n] /= sumyp;
+            yy[n] = yy[n] / ry;
+            yyp[n] = yyp[n] / ryp;
         }
         double MWmix = 0.;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            MWmix = MWmix + 0.5 * (yy[s] + yyp[s]) / P.molmass[s];
+            MWmix = MWmix + 0.5 * (yy[s] + yyp[s]) / P.M(s);
 #pragma unroll
             for (int l = 0; l < NS; ++l)
-                DijY[s * NS + l] = 0.5 * (Dm(il, jl, kl, l * NS + s) * yy[l] + Dm(iu, ju, ku, l * NS + s) * yyp[l] +
-                                          (Dm(il, jl, kl, s * NS + l) * yy[s] + Dm(iu, ju, ku, s * NS + l) * yyp[s]));
+                DijY[s * NS + l] = 0.5 * (Dm(lo, l * NS + s) * yy[l] + Dm(up, l * NS + s) * yyp[l] +
+                                          (Dm(lo, s * NS + l) * yy[s] + Dm(up, s * NS + l) * yyp[s]));
         }
 #pragma unroll
         for (int s = 0; s < NS; ++s)
@@ -455,27 +463,27 @@ __device__ __forceinline__ void stoch_body(const DevParams& P, Arr prim, Arr eta
                     DijY[s * NS + n] = 0.;
                     DijY[n * NS + s] = 0.;
                 }
-        MWmix = 1. / MWmix;
+        MWmix = quot(1., MWmix);
         cholesky<NS>(DijY, sqD);
-        double wsp = sqrt(P.k_B * MWmix * volinv / (P.Runiv * dt));
+        double wsp = root(quot(P.k_B * MWmix * volinv, P.Runiv * dt));
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
 #pragma unroll
-            for (int l = 0; l <= s; ++l) w[5 + s] = w[5 + s] + (wsp * sqD[s * NS + l]) * ran(i, j, k, 5 + l);
+            for (int l = 0; l <= s; ++l) w[5 + s] = w[5 + s] + (wsp * sqD[s * NS + l]) * ran[5 + l];
             o[5 + s] = w[5 + s];
         }
         double soret = 0.;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             double hk = P.e0[s] + P.hcp[s] * meanT;
-            double ss = (hk + P.Runiv * meanT / P.molmass[s] * 0.5 * (chi(il, jl, kl, s) + chi(iu, ju, ku, s))) *
+            double ss = (hk + P.Runiv * meanT / P.M(s) * 0.5 * (chi(lo, s) + chi(up, s))) *
                         w[5 + s];
             soret = soret + ss;
         }
         o[nv + 3] = o[nv + 3] + soret;
     }
 
-    if (P.any_wall) {  // StochFlux on the wall planes of direction D
+    if (WALL) {  // StochFlux on the wall planes of direction D
         const int c = (D == 0) ? i : (D == 1) ? j : k;
         const int f = (c == 0) ? 2 * D : (c == P.n[D]) ? 2 * D + 1 : -1;
         if (f >= 0) {
@@ -508,8 +516,6 @@ __device__ __forceinline__ void stoch_body(const DevParams& P, Arr prim, Arr eta
             }
         }
     }
-#pragma unroll
-    for (int n = 0; n < NS + 9; ++n) fl(i, j, k, n) = o[n];
 }
 
 // ---- diffusive face flux (flux.cpp:1193-1623) ----------------------------------------------
@@ -519,67 +525,64 @@ __device__ __forceinline__ void stoch_body(const DevParams& P, Arr prim, Arr eta
 // zeroes species, density and Dufour fluxes on bc_mass 1 faces; the corner pass in between
 // touches none of those components, so it is applied here.
 
-template <int NS, int D>
-__device__ __forceinline__ void diff_body(const DevParams& P, Arr prim, Arr eta, Arr kappa, Arr chi, Arr Dm,
-                                          Arr fl, long t)
+template <int NS, int D, bool WALL>
+__device__ __forceinline__ void diff_part(const DevParams& P, const FaceView& V, const WallFace& W, double* o)
 {
-    int i, j, k;
-    if (!box_index(P, t, D == 0, D == 1, D == 2, i, j, k)) return;
-    const int il = i - (D == 0), jl = j - (D == 1), kl = k - (D == 2);
-    const WallFace W = wall_face<D>(P, i, j, k);
-    const bool wall = W.any();
-    // coefficient / mean cells: the two neighbours, or the wall-side cell twice
-    const int ai = wall ? W.wi : il, aj = wall ? W.wj : jl, ak = wall ? W.wk : kl;
-    const int bi = wall ? W.wi : i, bj = wall ? W.wj : j, bk = wall ? W.wk : k;
+    const Fld &prim = V.prim, &eta = V.eta, &kappa = V.kappa, &chi = V.chi, &Dm = V.Dm;
+    // gradients between c0 and cm; coefficients and means of lo and up (the wall-side cell twice)
+    const unsigned c0 = V.c0, cm = V.cm, lo = V.lo, up = V.up;
+    const bool wall = WALL && W.any();
     const int nv = NS + 5;
-    const double half = 0.5, h = wall ? 0.5 * P.dx[D] : P.dx[D];
+    const double half = 0.5;
+    const Rcp h{wall ? 0.5 * P.dx[D] : P.dx[D], wall ? 2.0 * P.rdx[D] : P.rdx[D]};
 
-    double mup = half * (eta(bi, bj, bk) + eta(ai, aj, ak));
-    double kp = half * (kappa(bi, bj, bk) + kappa(ai, aj, ak));
-    double tau1 = mup * (prim(i, j, k, 1) - prim(il, jl, kl, 1)) / h;
-    double tau2 = mup * (prim(i, j, k, 2) - prim(il, jl, kl, 2)) / h;
-    double tau3 = mup * (prim(i, j, k, 3) - prim(il, jl, kl, 3)) / h;
+    double mup = half * (eta(up, 0) + eta(lo, 0));
+    double kp = half * (kappa(up, 0) + kappa(lo, 0));
+    double tau1 = mup * (prim(c0, 1) - prim(cm, 1)) / h;
+    double tau2 = mup * (prim(c0, 2) - prim(cm, 2)) / h;
+    double tau3 = mup * (prim(c0, 3) - prim(cm, 3)) / h;
     double divp = 0.;
-    double s1 = prim(ai, aj, ak, 1) + prim(bi, bj, bk, 1);
-    double s2 = prim(ai, aj, ak, 2) + prim(bi, bj, bk, 2);
-    double s3 = prim(ai, aj, ak, 3) + prim(bi, bj, bk, 3);
+    double s1 = prim(lo, 1) + prim(up, 1);
+    double s2 = prim(lo, 2) + prim(up, 2);
+    double s3 = prim(lo, 3) + prim(up, 3);
     double phiflx;
     if (D == 0) phiflx = tau1 * s1 + divp * s1 + tau2 * s2 + tau3 * s3;
     else if (D == 1) phiflx = tau1 * s1 + tau2 * s2 + divp * s2 + tau3 * s3;
     else phiflx = tau1 * s1 + tau2 * s2 + tau3 * s3 + divp * s3;
-    double Qflux = kp * (prim(i, j, k, 4) - prim(il, jl, kl, 4)) / h;
-    fl(i, j, k, 1) = fl(i, j, k, 1) - (D == 0 ? tau1 + divp : tau1);
-    fl(i, j, k, 2) = fl(i, j, k, 2) - (D == 1 ? tau2 + divp : tau2);
-    fl(i, j, k, 3) = fl(i, j, k, 3) - (D == 2 ? tau3 + divp : tau3);
-    fl(i, j, k, nv) = fl(i, j, k, nv) - Qflux;
-    fl(i, j, k, nv + 1) = fl(i, j, k, nv + 1) - (half * phiflx);
+    double Qflux = kp * (prim(c0, 4) - prim(cm, 4)) / h;
+    o[1] = o[1] - (D == 0 ? tau1 + divp : tau1);
+    o[2] = o[2] - (D == 1 ? tau2 + divp : tau2);
+    o[3] = o[3] - (D == 2 ? tau3 + divp : tau3);
+    o[nv] = o[nv] - Qflux;
+    o[nv + 1] = o[nv + 1] - (half * phiflx);
 
-    double meanT = 0.5 * (prim(ai, aj, ak, 4) + prim(bi, bj, bk, 4));
-    double meanP = 0.5 * (prim(ai, aj, ak, 5) + prim(bi, bj, bk, 5));
+    double meanT = 0.5 * (prim(lo, 4) + prim(up, 4));
+    double meanP = 0.5 * (prim(lo, 5) + prim(up, 5));
     if (P.algorithm_type == 2) {
+        const Rcp rT = rcp_of(meanT), rP = rcp_of(meanP);
         double dk[NS], soret[NS], Fk[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            double XU = prim(i, j, k, 6 + NS + s), XL = prim(il, jl, kl, 6 + NS + s);
+            double XU = prim(c0, 6 + NS + s), XL = prim(cm, 6 + NS + s);
             double term1 = (XU - XL) / h;
-            double mX = 0.5 * (prim(ai, aj, ak, 6 + NS + s) + prim(bi, bj, bk, 6 + NS + s));
-            double mY = 0.5 * (prim(ai, aj, ak, 6 + s) + prim(bi, bj, bk, 6 + s));
-            double term2 = (mX - mY) * (prim(i, j, k, 5) - prim(il, jl, kl, 5)) / h / meanP;
+            double mX = 0.5 * (prim(lo, 6 + NS + s) + prim(up, 6 + NS + s));
+            double mY = 0.5 * (prim(lo, 6 + s) + prim(up, 6 + s));
+            double term2 = (mX - mY) * (prim(c0, 5) - prim(cm, 5)) / h / rP;
             dk[s] = term1 + term2;
             double ChiX;
             if (D == 2 && !wall)  // flux.cpp:1561 reads chi at k and k+1
-                ChiX = 0.5 * (chi(i, j, k, s) * XL + chi(i, j, k + 1, s) * XU);
+                ChiX = 0.5 * (chi(c0, s) * XL + chi(c0, s, 0, 0, 1) * XU);
             else
-                ChiX = 0.5 * (chi(ai, aj, ak, s) * prim(ai, aj, ak, 6 + NS + s) +
-                              chi(bi, bj, bk, s) * prim(bi, bj, bk, 6 + NS + s));
-            soret[s] = ChiX * (prim(i, j, k, 4) - prim(il, jl, kl, 4)) / h / meanT;
+                ChiX = 0.5 * (chi(lo, s) * prim(lo, 6 + NS + s) +
+                              chi(up, s) * prim(up, 6 + NS + s));
+            soret[s] = ChiX * (prim(c0, 4) - prim(cm, 4)) / h / rT;
         }
 #pragma unroll
         for (int kk = 0; kk < NS; ++kk) {
             double f = 0.;
 #pragma unroll
             for (int ll = 0; ll < NS; ++ll) {
-                double Fks = half * (Dm(ai, aj, ak, ll * NS + kk) + Dm(bi, bj, bk, ll * NS + kk)) * (dk[ll] + soret[ll]);
+                double Fks = half * (Dm(lo, ll * NS + kk) + Dm(up, ll * NS + kk)) * (dk[ll] + soret[ll]);
                 f = f - Fks;
             }
             Fk[kk] = f;
@@ -588,43 +591,81 @@ __device__ __forceinline__ void diff_body(const DevParams& P, Arr prim, Arr eta,
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             double hk = P.e0[s] + P.hcp[s] * meanT;
-            double csum = (D == 2 && !wall) ? chi(i, j, k, s) + chi(i, j, k, s)  // flux.cpp:1604
-                                            : chi(ai, aj, ak, s) + chi(bi, bj, bk, s);
-            double Q5s = (hk + 0.5 * P.Runiv * meanT * csum / P.molmass[s]) * Fk[s];
+            double csum = (D == 2 && !wall) ? chi(c0, s) + chi(c0, s)  // flux.cpp:1604
+                                            : chi(lo, s) + chi(up, s);
+            double Q5s = (hk + 0.5 * P.Runiv * meanT * csum / P.M(s)) * Fk[s];
             Q5 = Q5 + Q5s;
         }
-        fl(i, j, k, nv + 3) = fl(i, j, k, nv + 3) + Q5;
+        o[nv + 3] = o[nv + 3] + Q5;
 #pragma unroll
-        for (int s = 0; s < NS; ++s) fl(i, j, k, 5 + s) = fl(i, j, k, 5 + s) + Fk[s];
+        for (int s = 0; s < NS; ++s) o[5 + s] = o[5 + s] + Fk[s];
     }
     if (wall && P.bcm[2 * D + (W.hi ? 1 : 0)] == 1) {  // BCWallSpeciesFlux
 #pragma unroll
-        for (int s = 0; s < NS; ++s) fl(i, j, k, 5 + s) = 0.;
-        fl(i, j, k, 0) = 0.;
-        fl(i, j, k, nv + 3) = 0.;
+        for (int s = 0; s < NS; ++s) o[5 + s] = 0.;
+        o[0] = 0.;
+        o[nv + 3] = 0.;
     }
+}
+
+// The A/B noise of component comp of face (i,j,k) of direction D, and of node (i,j,k): N(0,1) times
+// the component's scale, keyed by the wrapped index.
+template <int D>
+__device__ __forceinline__ void face_noise(const DevParams& P, const NoiseKey& K, int comp, int i, int j, int k,
+                                           double& A, double& B)
+{
+    const int iw = (D == 0 && i == P.n[0]) ? 0 : i;
+    const int jw = (D == 1 && j == P.n[1]) ? 0 : j;
+    const int kw = (D == 2 && k == P.n[2]) ? 0 : k;
+    uint32_t lin = (uint32_t)(((long)kw * P.n[1] + jw) * P.n[0] + iw);
+    // in a wall direction face n is a face of its own, drawn from its own field
+    const int c = (D == 0) ? i : (D == 1) ? j : k;
+    const uint32_t wall_hi = (c == P.n[D] && !P.periodic[D]) ? 128u : 0u;
+    const double scale = (comp <= 3) ? P.var_mom : (comp == 4) ? P.var_ener : P.var_mass;
+    double za, zb;
+    noise_ab(K, (uint32_t)(16 * D + comp) + wall_hi, lin, za, zb);
+    A = za * scale;
+    B = zb * scale;
+}
+
+__device__ __forceinline__ void node_noise(const DevParams& P, const NoiseKey& K, double scale, int i, int j, int k,
+                                           double& A, double& B)
+{
+    const int iw = (i == P.n[0]) ? 0 : i, jw = (j == P.n[1]) ? 0 : j, kw = (k == P.n[2]) ? 0 : k;
+    uint32_t lin = (uint32_t)(((long)kw * P.n[1] + jw) * P.n[0] + iw);
+    // nodes on the hi plane of a wall direction are distinct: field NODE_FIELD + mask
+    const uint32_t mask = ((i == P.n[0] && !P.periodic[0]) ? 1u : 0u) |
+                          ((j == P.n[1] && !P.periodic[1]) ? 2u : 0u) |
+                          ((k == P.n[2] && !P.periodic[2]) ? 4u : 0u);
+    double za, zb;
+    noise_ab(K, NODE_FIELD + mask, lin, za, zb);
+    A = za * scale;
+    B = zb * scale;
 }
 
 // ---- corner viscous terms at nodes (flux.cpp:1627-1713) ------------------------------------
 
-__global__ void __launch_bounds__(BLK) k_corner_node(DevParams P, Arr prim, Arr eta, Arr zeta,
+__global__ void __launch_bounds__(BLK) k_corner_node(DevParams P, Arr prima, Arr etaa, Arr zetaa,
                                                      Arr cux, Arr cvx, Arr cwx, Arr cuy, Arr cvy,
                                                      Arr cwy, Arr cuz, Arr cvz, Arr cwz, Arr vcorn, Arr rancorn,
-                                                     Arr rA, Arr rB, double w, int weigh)
+                                                     FaceNoise nz)
 {
-    long t = (long)blockIdx.x * BLK + threadIdx.x;
+    const long t = xcd_thread();
     int i, j, k;
     if (!box_index(P, t, 1, 1, 1, i, j, k)) return;
-    if (weigh) rancorn(i, j, k) = 1.0 * rA(i, j, k) + w * rB(i, j, k);  // the node's weighted noise
-    double muxp = 0.125 * (eta(i, j - 1, k - 1) + eta(i - 1, j - 1, k - 1) + eta(i, j, k - 1) +
-                           eta(i - 1, j, k - 1) + eta(i, j - 1, k) + eta(i - 1, j - 1, k) + eta(i, j, k) +
-                           eta(i - 1, j, k));
+    const Fld prim = fld_of(prima, prima), eta = fld_of(etaa, prima), zeta = fld_of(zetaa, prima);
+    const unsigned cb = off_of(prima, i, j, k), nd0 = off_of(rancorn, i, j, k);
+    const long nd8 = (long)(nd0 >> 3);
+    double muxp = 0.125 * (eta(cb, 0, 0, -1, -1) + eta(cb, 0, -1, -1, -1) + eta(cb, 0, 0, 0, -1) +
+                           eta(cb, 0, -1, 0, -1) + eta(cb, 0, 0, -1, 0) + eta(cb, 0, -1, -1, 0) + eta(cb, 0, 0, 0, 0) +
+                           eta(cb, 0, -1, 0, 0));
     double zetaxp = 0.;
     if (P.visc_type == 3 || P.visc_type == -3)
-        zetaxp = 0.125 * (zeta(i, j - 1, k - 1) + zeta(i - 1, j - 1, k - 1) + zeta(i, j, k - 1) +
-                          zeta(i - 1, j, k - 1) + zeta(i, j - 1, k) + zeta(i - 1, j - 1, k) + zeta(i, j, k) +
-                          zeta(i - 1, j, k));
-    double DXa[3] = {P.dx[0], P.dx[1], P.dx[2]};
+        zetaxp = 0.125 * (zeta(cb, 0, 0, -1, -1) + zeta(cb, 0, -1, -1, -1) + zeta(cb, 0, 0, 0, -1) +
+                          zeta(cb, 0, -1, 0, -1) + zeta(cb, 0, 0, -1, 0) + zeta(cb, 0, -1, -1, 0) + zeta(cb, 0, 0, 0, 0) +
+                          zeta(cb, 0, -1, 0, 0));
+    Rcp DXa[3] = {P.h(0), P.h(1), P.h(2)};
+    constexpr Rcp twelve{12., 1. / 12.};
     if (P.any_wall) {
         // wall nodes (flux.cpp:1647-1682): half spacing across each wall met, viscosities from
         // the four ghost-layer cells of the last wall met (the checks run lo x .. hi z)
@@ -633,7 +674,7 @@ __global__ void __launch_bounds__(BLK) k_corner_node(DevParams P, Arr prim, Arr 
         for (int f = 0; f < 6; ++f) {
             const int d = f >> 1, side = f & 1;
             if (!P.wall[f] || nd[d] != (side ? P.n[d] : 0)) continue;
-            DXa[d] = 0.5 * P.dx[d];
+            DXa[d] = Rcp{0.5 * P.dx[d], 2.0 * P.rdx[d]};
             const int a = (d == 0) ? 1 : 0, b = (d == 2) ? 1 : 2;
             double e4 = 0., z4 = 0.;
 #pragma unroll
@@ -642,44 +683,62 @@ __global__ void __launch_bounds__(BLK) k_corner_node(DevParams P, Arr prim, Arr 
                 c[d] = side ? nd[d] : nd[d] - 1;
                 c[a] = nd[a] - 1 + (q >> 1);
                 c[b] = nd[b] - 1 + (q & 1);
-                e4 = (q == 0) ? eta(c[0], c[1], c[2]) : e4 + eta(c[0], c[1], c[2]);
-                z4 = (q == 0) ? zeta(c[0], c[1], c[2]) : z4 + zeta(c[0], c[1], c[2]);
+                const unsigned cw = off_of(prima, c[0], c[1], c[2]);
+                e4 = (q == 0) ? eta(cw, 0) : e4 + eta(cw, 0);
+                z4 = (q == 0) ? zeta(cw, 0) : z4 + zeta(cw, 0);
             }
             muxp = 0.25 * e4;
             zetaxp = (P.visc_type == 3 || P.visc_type == -3) ? 0.25 * z4 : 0.;
         }
     }
-    const double DX0 = DXa[0], DX1 = DXa[1], DX2 = DXa[2];
-    Arr gx[3] = {cux, cvx, cwx}, gy[3] = {cuy, cvy, cwy}, gz[3] = {cuz, cvz, cwz};
+    const Rcp DX0 = DXa[0], DX1 = DXa[1], DX2 = DXa[2];
+    // all values first, then the stores: a store in between would make the cells load again
+    double gx[3], gy[3], gz[3], vc;
 #pragma unroll
     for (int n = 1; n < 4; ++n) {
-        gx[n - 1](i, j, k) = 0.25 * muxp *
-                             (prim(i, j - 1, k - 1, n) - prim(i - 1, j - 1, k - 1, n) + prim(i, j, k - 1, n) -
-                              prim(i - 1, j, k - 1, n) + prim(i, j - 1, k, n) - prim(i - 1, j - 1, k, n) +
-                              prim(i, j, k, n) - prim(i - 1, j, k, n)) /
+        gx[n - 1] = 0.25 * muxp *
+                             (prim(cb, n, 0, -1, -1) - prim(cb, n, -1, -1, -1) + prim(cb, n, 0, 0, -1) -
+                              prim(cb, n, -1, 0, -1) + prim(cb, n, 0, -1, 0) - prim(cb, n, -1, -1, 0) +
+                              prim(cb, n, 0, 0, 0) - prim(cb, n, -1, 0, 0)) /
                              DX0;
-        gy[n - 1](i, j, k) = 0.25 * muxp *
-                             (prim(i - 1, j, k - 1, n) - prim(i - 1, j - 1, k - 1, n) + prim(i, j, k - 1, n) -
-                              prim(i, j - 1, k - 1, n) + prim(i - 1, j, k, n) - prim(i - 1, j - 1, k, n) +
-                              prim(i, j, k, n) - prim(i, j - 1, k, n)) /
+        gy[n - 1] = 0.25 * muxp *
+                             (prim(cb, n, -1, 0, -1) - prim(cb, n, -1, -1, -1) + prim(cb, n, 0, 0, -1) -
+                              prim(cb, n, 0, -1, -1) + prim(cb, n, -1, 0, 0) - prim(cb, n, -1, -1, 0) +
+                              prim(cb, n, 0, 0, 0) - prim(cb, n, 0, -1, 0)) /
                              DX1;
-        gz[n - 1](i, j, k) = 0.25 * muxp *
-                             (prim(i - 1, j - 1, k, n) - prim(i - 1, j - 1, k - 1, n) + prim(i, j - 1, k, n) -
-                              prim(i, j - 1, k - 1, n) + prim(i - 1, j, k, n) - prim(i - 1, j, k - 1, n) +
-                              prim(i, j, k, n) - prim(i, j, k - 1, n)) /
+        gz[n - 1] = 0.25 * muxp *
+                             (prim(cb, n, -1, -1, 0) - prim(cb, n, -1, -1, -1) + prim(cb, n, 0, -1, 0) -
+                              prim(cb, n, 0, -1, -1) + prim(cb, n, -1, 0, 0) - prim(cb, n, -1, 0, -1) +
+                              prim(cb, n, 0, 0, 0) - prim(cb, n, 0, 0, -1)) /
                              DX2;
     }
-    vcorn(i, j, k) =
-        (muxp / 12. + zetaxp / 4.) *
-        ((prim(i, j - 1, k - 1, 1) - prim(i - 1, j - 1, k - 1, 1)) / DX0 +
-         (prim(i, j, k - 1, 1) - prim(i - 1, j, k - 1, 1)) / DX0 +
-         (prim(i, j - 1, k, 1) - prim(i - 1, j - 1, k, 1)) / DX0 + (prim(i, j, k, 1) - prim(i - 1, j, k, 1)) / DX0 +
-         (prim(i - 1, j, k - 1, 2) - prim(i - 1, j - 1, k - 1, 2)) / DX1 +
-         (prim(i, j, k - 1, 2) - prim(i, j - 1, k - 1, 2)) / DX1 +
-         (prim(i - 1, j, k, 2) - prim(i - 1, j - 1, k, 2)) / DX1 + (prim(i, j, k, 2) - prim(i, j - 1, k, 2)) / DX1 +
-         (prim(i - 1, j - 1, k, 3) - prim(i - 1, j - 1, k - 1, 3)) / DX2 +
-         (prim(i, j - 1, k, 3) - prim(i, j - 1, k - 1, 3)) / DX2 +
-         (prim(i - 1, j, k, 3) - prim(i - 1, j, k - 1, 3)) / DX2 + (prim(i, j, k, 3) - prim(i, j, k - 1, 3)) / DX2);
+    vc =
+        (muxp / twelve + zetaxp / 4.) *
+        ((prim(cb, 1, 0, -1, -1) - prim(cb, 1, -1, -1, -1)) / DX0 +
+         (prim(cb, 1, 0, 0, -1) - prim(cb, 1, -1, 0, -1)) / DX0 +
+         (prim(cb, 1, 0, -1, 0) - prim(cb, 1, -1, -1, 0)) / DX0 + (prim(cb, 1, 0, 0, 0) - prim(cb, 1, -1, 0, 0)) / DX0 +
+         (prim(cb, 2, -1, 0, -1) - prim(cb, 2, -1, -1, -1)) / DX1 +
+         (prim(cb, 2, 0, 0, -1) - prim(cb, 2, 0, -1, -1)) / DX1 +
+         (prim(cb, 2, -1, 0, 0) - prim(cb, 2, -1, -1, 0)) / DX1 + (prim(cb, 2, 0, 0, 0) - prim(cb, 2, 0, -1, 0)) / DX1 +
+         (prim(cb, 3, -1, -1, 0) - prim(cb, 3, -1, -1, -1)) / DX2 +
+         (prim(cb, 3, 0, -1, 0) - prim(cb, 3, 0, -1, -1)) / DX2 +
+         (prim(cb, 3, -1, 0, 0) - prim(cb, 3, -1, 0, -1)) / DX2 + (prim(cb, 3, 0, 0, 0) - prim(cb, 3, 0, 0, -1)) / DX2);
+    const Arr ax[3] = {cux, cvx, cwx}, ay[3] = {cuy, cvy, cwy}, az[3] = {cuz, cvz, cwz};
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        ax[n].p[nd8] = gx[n];
+        ay[n].p[nd8] = gy[n];
+        az[n].p[nd8] = gz[n];
+    }
+    vcorn.p[nd8] = vc;
+    // the node's weighted noise
+    if (nz.mode == kNoiseSets) {
+        rancorn(i, j, k) = 1.0 * nz.rA(i, j, k) + nz.w * nz.rB(i, j, k);
+    } else if (nz.mode == kNoisePhilox) {
+        double A, B;
+        node_noise(P, nz.K, P.var_mom, i, j, k, A, B);
+        rancorn(i, j, k) = 1.0 * A + nz.w * B;
+    }
 }
 
 // ---- corner-to-face terms (flux.cpp:1770-1980) -------------------------------------------
@@ -697,7 +756,7 @@ struct Transverse {
 // Left-to-right sum of `a` over the 4 nodes of face (i,j,k), starting from `s0` unless
 // `first`; zorder selects (hi,hi),(hi,lo),(lo,hi),(lo,lo) instead of (hi,hi),(lo,hi),(hi,lo),(lo,lo).
 template <int D>
-__device__ inline double node4(const Arr& a, int i, int j, int k, bool zorder, double s0 = 0., bool first = true)
+__device__ inline double node4(const Fld& a, unsigned nd, bool zorder, double s0 = 0., bool first = true)
 {
     using T = Transverse<D>;
     const int oa[4] = {1, zorder ? 1 : 0, zorder ? 0 : 1, 0};
@@ -705,50 +764,50 @@ __device__ inline double node4(const Arr& a, int i, int j, int k, bool zorder, d
     double s = s0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        double v = a(i + oa[q] * T::AI, j + oa[q] * T::AJ + ob[q] * T::BJ, k + ob[q] * T::BK);
+        double v = a(nd, 0, oa[q] * T::AI, oa[q] * T::AJ + ob[q] * T::BJ, ob[q] * T::BK);
         s = (first && q == 0) ? v : s + v;
     }
     return s;
 }
 
 template <int NS, int D>
-__device__ __forceinline__ void corner_face_body(const DevParams& P, Arr prim, Arr fl, Arr vcorn, Arr c1,
-                                                 Arr c2, Arr ta1, Arr ta2, long t)
+__device__ __forceinline__ void corner_part(const FaceView& V, double* o)
 {
-    int i, j, k;
-    if (!box_index(P, t, D == 0, D == 1, D == 2, i, j, k)) return;
-    const WallFace W = wall_face<D>(P, i, j, k);
+    const Fld& prim = V.prim;
+    // corn[a][b]: derivative direction a, velocity component b (cornx/corny/cornz of flux.cpp)
+    // x face: div pair (vy, wz), tangential (uy, uz); y: (ux, wz), (vx, vz); z: (vy, ux), (wx, wy)
+    const Fld &c1 = D == 1 ? V.corn[0][0] : V.corn[1][1], &c2 = D == 2 ? V.corn[0][0] : V.corn[2][2];
+    const Fld &ta1 = D == 0 ? V.corn[1][0] : V.corn[0][D], &ta2 = D == 2 ? V.corn[1][2] : V.corn[2][D];
     // velocity cells of the heating term: the two neighbours, or the wall-side cell twice
     // (flux.cpp:1791-1822: 0.5*x*u_wall equals 0.25*x*(u_wall + u_wall) exactly)
-    const int il = W.any() ? W.wi : i - (D == 0), jl = W.any() ? W.wj : j - (D == 1),
-              kl = W.any() ? W.wk : k - (D == 2);
-    const int iu = W.any() ? W.wi : i, ju = W.any() ? W.wj : j, ku = W.any() ? W.wk : k;
+    const unsigned lo = V.lo, up = V.up;
     const int nv = NS + 5;
     const bool zo = (D == 2);
-    double vc4 = node4<D>(vcorn, i, j, k, false);
-    double div8 = node4<D>(c1, i, j, k, zo);
-    div8 = node4<D>(c2, i, j, k, zo, div8, false);
-    double s1 = node4<D>(ta1, i, j, k, zo);
-    double s2 = node4<D>(ta2, i, j, k, zo);
+    double vc4 = node4<D>(V.visccorn, V.nd, false);
+    double div8 = node4<D>(c1, V.nd, zo);
+    div8 = node4<D>(c2, V.nd, zo, div8, false);
+    double s1 = node4<D>(ta1, V.nd, zo);
+    double s2 = node4<D>(ta2, V.nd, zo);
     constexpr int cn = 1 + D;
     constexpr int tc1 = (D == 0) ? 2 : 1, tc2 = (D == 2) ? 2 : 3;
-    fl(i, j, k, cn) = fl(i, j, k, cn) - 0.25 * vc4;
-    fl(i, j, k, cn) = fl(i, j, k, cn) + .25 * div8;
-    fl(i, j, k, tc1) = fl(i, j, k, tc1) - .25 * s1;
-    fl(i, j, k, tc2) = fl(i, j, k, tc2) - .25 * s2;
-    double phiflx = 0.25 * (vc4 - div8) * (prim(il, jl, kl, cn) + prim(iu, ju, ku, cn));
-    phiflx = phiflx + .25 * s1 * (prim(il, jl, kl, tc1) + prim(iu, ju, ku, tc1));
-    phiflx = phiflx + .25 * s2 * (prim(il, jl, kl, tc2) + prim(iu, ju, ku, tc2));
-    fl(i, j, k, nv + 1) = fl(i, j, k, nv + 1) - 0.5 * phiflx;
+    o[cn] = o[cn] - 0.25 * vc4;
+    o[cn] = o[cn] + .25 * div8;
+    o[tc1] = o[tc1] - .25 * s1;
+    o[tc2] = o[tc2] - .25 * s2;
+    double phiflx = 0.25 * (vc4 - div8) * (prim(lo, cn) + prim(up, cn));
+    phiflx = phiflx + .25 * s1 * (prim(lo, tc1) + prim(up, tc1));
+    phiflx = phiflx + .25 * s2 * (prim(lo, tc2) + prim(up, tc2));
+    o[nv + 1] = o[nv + 1] - 0.5 * phiflx;
 }
 
 // ---- hyperbolic face flux (flux.cpp:2016-2372) ---------------------------------------------
 
-template <int NS, int D>
-__device__ __forceinline__ void hyp_body(const DevParams& P, Arr cons, Arr prim, Arr fl, long t)
+template <int NS, int D, bool WALL>
+__device__ __forceinline__ void hyp_part(const DevParams& P, const FaceView& V, const WallFace& W, double* o, int i,
+                                         int j, int k)
 {
-    int i, j, k;
-    if (!box_index(P, t, D == 0, D == 1, D == 2, i, j, k)) return;
+    const Fld &cons = V.cons, &prim = V.prim;
+    const unsigned c0 = V.c0;
     constexpr int ex = (D == 0), ey = (D == 1), ez = (D == 2);
     const int nv = NS + 5;
     const double wgt2 = 1. / 12.;
@@ -756,16 +815,16 @@ __device__ __forceinline__ void hyp_body(const DevParams& P, Arr cons, Arr prim,
     double cv[NS + 5], pv[NS + 6], Yk[NS];
     // walls: the wall face takes the wall-side cell (flux.cpp:2028-2037); with conserved
     // interpolation the next face in uses the one-sided weights of :1994-1997 (:2190-2206)
-    const WallFace W = wall_face<D>(P, i, j, k);
+    const bool wall = WALL && W.any();
     const int c = (D == 0) ? i : (D == 1) ? j : k;
-    const bool near_lo = P.any_wall && c == 1 && P.wall[2 * D];
-    const bool near_hi = P.any_wall && c == P.n[D] - 1 && P.wall[2 * D + 1];
+    const bool near_lo = WALL && c == 1 && P.wall[2 * D];
+    const bool near_hi = WALL && c == P.n[D] - 1 && P.wall[2 * D + 1];
     if (P.advection_type == 1) {
 #pragma unroll
         for (int l = 0; l < NS + 6; ++l)
-            pv[l] = W.any() ? prim(W.wi, W.wj, W.wk, l)
-                            : wgt1 * (prim(i, j, k, l) + prim(i - ex, j - ey, k - ez, l)) -
-                                  wgt2 * (prim(i - 2 * ex, j - 2 * ey, k - 2 * ez, l) + prim(i + ex, j + ey, k + ez, l));
+            pv[l] = wall ? prim(V.up, l)
+                            : wgt1 * (prim(c0, l) + prim(c0, l, -ex, -ey, -ez)) -
+                                  wgt2 * (prim(c0, l, -2 * ex, -2 * ey, -2 * ez) + prim(c0, l, ex, ey, ez));
         double rho = pv[0];
         cv[0] = rho;
 #pragma unroll
@@ -779,74 +838,80 @@ __device__ __forceinline__ void hyp_body(const DevParams& P, Arr cons, Arr prim,
         const double wgta = -0.2, wgtb = 0.75, wgtc = 0.5, wgtd = -0.05;
 #pragma unroll
         for (int l = 0; l < NS + 5; ++l) {
-            const double cm2 = cons(i - 2 * ex, j - 2 * ey, k - 2 * ez, l), cm1 = cons(i - ex, j - ey, k - ez, l);
-            const double c0 = cons(i, j, k, l), cp1 = cons(i + ex, j + ey, k + ez, l);
-            if (W.lo) cv[l] = cm1;
-            else if (W.hi) cv[l] = c0;
-            else if (near_lo) cv[l] = wgta * cm2 + wgtb * cm1 + wgtc * c0 + wgtd * cp1;
-            else if (near_hi) cv[l] = wgta * cp1 + wgtb * c0 + wgtc * cm1 + wgtd * cm2;
-            else cv[l] = wgt1 * (c0 + cm1) - wgt2 * (cm2 + cp1);
+            const double cm2 = cons(c0, l, -2 * ex, -2 * ey, -2 * ez), cm1 = cons(c0, l, -ex, -ey, -ez);
+            const double cc = cons(c0, l), cp1 = cons(c0, l, ex, ey, ez);
+            if (WALL && W.lo) cv[l] = cm1;
+            else if (WALL && W.hi) cv[l] = cc;
+            else if (near_lo) cv[l] = wgta * cm2 + wgtb * cm1 + wgtc * cc + wgtd * cp1;
+            else if (near_hi) cv[l] = wgta * cp1 + wgtb * cc + wgtc * cm1 + wgtd * cm2;
+            else cv[l] = wgt1 * (cc + cm1) - wgt2 * (cm2 + cp1);
         }
+        const Rcp rho = rcp_of(cv[0]);
 #pragma unroll
-        for (int l = 1; l < 4; ++l) pv[l] = cv[l] / cv[0];
+        for (int l = 1; l < 4; ++l) pv[l] = cv[l] / rho;
 #pragma unroll
-        for (int n = 0; n < NS; ++n) Yk[n] = cv[5 + n] / cv[0];
+        for (int n = 0; n < NS; ++n) Yk[n] = cv[5 + n] / rho;
         double vsqr = pv[1] * pv[1] + pv[2] * pv[2] + pv[3] * pv[3];
-        double ie = cv[4] / cv[0] - 0.5 * vsqr;
+        double ie = cv[4] / rho - 0.5 * vsqr;
         pv[4] = eos_temperature<NS>(P, ie, Yk);
         pv[5] = eos_pressure<NS>(P, Yk, cv[0], pv[4]);
     }
     const double un = pv[1 + D];
-    fl(i, j, k, 0) += cv[0] * un;
+    o[0] += cv[0] * un;
     if (D == 0) {
-        fl(i, j, k, 1) += cv[0] * (pv[1] * pv[1]) + pv[5];
-        fl(i, j, k, 2) += cv[0] * pv[1] * pv[2];
-        fl(i, j, k, 3) += cv[0] * pv[1] * pv[3];
+        o[1] += cv[0] * (pv[1] * pv[1]) + pv[5];
+        o[2] += cv[0] * pv[1] * pv[2];
+        o[3] += cv[0] * pv[1] * pv[3];
     } else if (D == 1) {
-        fl(i, j, k, 1) += cv[0] * pv[1] * pv[2];
-        fl(i, j, k, 2) += cv[0] * pv[2] * pv[2] + pv[5];
-        fl(i, j, k, 3) += cv[0] * pv[3] * pv[2];
+        o[1] += cv[0] * pv[1] * pv[2];
+        o[2] += cv[0] * pv[2] * pv[2] + pv[5];
+        o[3] += cv[0] * pv[3] * pv[2];
     } else {
-        fl(i, j, k, 1) += cv[0] * pv[1] * pv[3];
-        fl(i, j, k, 2) += cv[0] * pv[2] * pv[3];
-        fl(i, j, k, 3) += cv[0] * pv[3] * pv[3] + pv[5];
+        o[1] += cv[0] * pv[1] * pv[3];
+        o[2] += cv[0] * pv[2] * pv[3];
+        o[3] += cv[0] * pv[3] * pv[3] + pv[5];
     }
-    fl(i, j, k, 4) += un * cv[4] + pv[5] * un;
-    fl(i, j, k, 4) += fl(i, j, k, nv) + fl(i, j, k, nv + 1) + fl(i, j, k, nv + 2) + fl(i, j, k, nv + 3);
+    o[4] += un * cv[4] + pv[5] * un;
+    o[4] += o[nv] + o[nv + 1] + o[nv + 2] + o[nv + 3];
     if (P.algorithm_type == 2) {
         if (P.advection_type == 1) {
 #pragma unroll
-            for (int n = 0; n < NS; ++n) fl(i, j, k, 5 + n) += cv[0] * pv[6 + n] * un;
+            for (int n = 0; n < NS; ++n) o[5 + n] += cv[0] * pv[6 + n] * un;
         } else {
 #pragma unroll
-            for (int n = 0; n < NS; ++n) fl(i, j, k, 5 + n) += cv[5 + n] * un;
+            for (int n = 0; n < NS; ++n) o[5 + n] += cv[5 + n] * un;
         }
     }
 }
 
 // ---- stage combination (timeStep.cpp:158-201, 266-306, 370-413) ----------------------------
 
-// src: the source MultiFab (null: zero, main_driver.cpp:241-242)
+// src: the source MultiFab (null: zero, main_driver.cpp:241-242).  The conservedToPrimitive that
+// follows reads this cell's new state only, so prim is formed here from registers.
 template <int NS>
-__global__ void __launch_bounds__(BLK) k_stage(DevParams P, Arr out, Arr u0, Arr us, Arr fx, Arr fy,
-                                               Arr fz, Arr srcf, double dt, int mode)
+__global__ void __launch_bounds__(BLK) k_stage(DevParams P, Arr outa, Arr u0a, Arr usa, Arr fxa, Arr fya,
+                                               Arr fza, Arr srca, Arr prima, double dt, int mode)
 {
-    long t = (long)blockIdx.x * BLK + threadIdx.x;
+    const long t = xcd_thread();
     int i, j, k;
     if (!box_index(P, t, 0, 0, 0, i, j, k)) return;
+    const Fld out = fld_of(outa, prima), u0 = fld_of(u0a, prima), us = fld_of(usa, prima), prim = fld_of(prima, prima),
+              srcf = fld_of(srca, prima), fx = fld_of(fxa, fxa), fy = fld_of(fya, fya), fz = fld_of(fza, fza);
+    const unsigned cb = off_of(prima, i, j, k), ox = off_of(fxa, i, j, k), oy = off_of(fya, i, j, k),
+                   oz = off_of(fza, i, j, k);
     double o[NS + 5];
 #pragma unroll
     for (int n = 0; n < NS + 5; ++n) {
-        const double src = srcf.p ? srcf(i, j, k, n) : 0.0;
-        double div = (fx(i + 1, j, k, n) - fx(i, j, k, n)) / P.dx[0] +
-                     (fy(i, j + 1, k, n) - fy(i, j, k, n)) / P.dx[1] +
-                     (fz(i, j, k + 1, n) - fz(i, j, k, n)) / P.dx[2];
-        if (mode == 0) o[n] = us(i, j, k, n) - dt * div + dt * src;
-        else if (mode == 1) o[n] = 0.25 * (3.0 * u0(i, j, k, n) + us(i, j, k, n) - dt * div + dt * src);
-        else o[n] = (2. / 3.) * (0.5 * u0(i, j, k, n) + us(i, j, k, n) - dt * div + dt * src);
+        const double src = srcf.p ? srcf(cb, n) : 0.0;
+        double div = (fx(ox, n, 1, 0, 0) - fx(ox, n)) / P.h(0) +
+                     (fy(oy, n, 0, 1, 0) - fy(oy, n)) / P.h(1) +
+                     (fz(oz, n, 0, 0, 1) - fz(oz, n)) / P.h(2);
+        if (mode == 0) o[n] = us(cb, n) - dt * div + dt * src;
+        else if (mode == 1) o[n] = 0.25 * (3.0 * u0(cb, n) + us(cb, n) - dt * div + dt * src);
+        else o[n] = (2. / 3.) * (0.5 * u0(cb, n) + us(cb, n) - dt * div + dt * src);
     }
     const double* g = P.grav;
-    double r0 = us(i, j, k, 0), r1 = us(i, j, k, 1), r2 = us(i, j, k, 2), r3 = us(i, j, k, 3);
+    double r0 = us(cb, 0), r1 = us(cb, 1), r2 = us(cb, 2), r3 = us(cb, 3);
     if (mode == 0) {
 #pragma unroll
         for (int n = 0; n < 3; ++n) o[n + 1] += dt * r0 * g[n];
@@ -861,7 +926,11 @@ __global__ void __launch_bounds__(BLK) k_stage(DevParams P, Arr out, Arr u0, Arr
         o[4] += 2. / 3. * dt * (g[0] * r1 + g[1] * r2 + g[2] * r3);
     }
 #pragma unroll
-    for (int n = 0; n < NS + 5; ++n) out(i, j, k, n) = o[n];
+    for (int n = 0; n < NS + 5; ++n) out(cb, n) = o[n];
+    double pr[2 * NS + 6];
+    cons_to_prim_cell<NS>(P, o, pr);
+#pragma unroll
+    for (int n = 0; n < 2 * NS + 6; ++n) prim(cb, n) = pr[n];
 }
 
 // ---- chemistry source (chemistry_functions.cpp:128-193) ------------------------------------
@@ -899,30 +968,7 @@ __global__ void __launch_bounds__(BLK) k_chem_noise(DevParams P, NoiseKey K, Arr
 
 // ---- noise --------------------------------------------------------------------------------
 
-// The four weighted-noise arrays of a stage in one launch: stochFlux[d] = 1*A + w*B on comps
-// 1..nvars-1 (comp 0 zeroed), rancorn likewise on its one component (MultiFab::LinComb).
-struct LinSet {
-    double* dst[4];
-    const double* a[4];
-    const double* b[4];
-    long npts[4];
-    int nc[4], c0[4];
-};
-
-__global__ void __launch_bounds__(BLK) k_lincomb4(LinSet L, double w)
-{
-    long t = (long)blockIdx.x * BLK + threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if (t >= L.npts[q]) continue;
-        for (int n = 0; n < L.nc[q]; ++n) {
-            const long x = t + (long)n * L.npts[q];
-            L.dst[q][x] = (n < L.c0[q]) ? 0.0 : 1.0 * L.a[q][x] + w * L.b[q][x];
-        }
-    }
-}
-
-// stochFlux = 1*A + w*B on comps 1..nvars-1 (comp 0 zeroed), MultiFab::LinComb.
+// dst = 1*A + w*B (MultiFab::LinComb), components below c0 zeroed.
 __global__ void __launch_bounds__(BLK) k_lincomb(double* dst, const double* a, const double* b, long npts,
                                                  int nc, int c0, double w)
 {
@@ -941,21 +987,13 @@ __device__ __forceinline__ void noise_face_body(const DevParams& P, const NoiseK
 {
     int i, j, k;
     if (!box_index(P, t, D == 0, D == 1, D == 2, i, j, k)) return;
-    const int iw = (D == 0 && i == P.n[0]) ? 0 : i;
-    const int jw = (D == 1 && j == P.n[1]) ? 0 : j;
-    const int kw = (D == 2 && k == P.n[2]) ? 0 : k;
-    uint32_t lin = (uint32_t)(((long)kw * P.n[1] + jw) * P.n[0] + iw);
-    // in a wall direction face n is a face of its own, drawn from its own field
-    const int c = (D == 0) ? i : (D == 1) ? j : k;
-    const uint32_t wall_hi = (c == P.n[D] && !P.periodic[D]) ? 128u : 0u;
     A(i, j, k, 0) = 0.0;
     B(i, j, k, 0) = 0.0;
     for (int comp = 1; comp < P.nvars; ++comp) {
-        const double scale = (comp <= 3) ? P.var_mom : (comp == 4) ? P.var_ener : P.var_mass;
-        double za, zb;
-        noise_ab(K, (uint32_t)(16 * D + comp) + wall_hi, lin, za, zb);
-        A(i, j, k, comp) = za * scale;
-        B(i, j, k, comp) = zb * scale;
+        double a, b;
+        face_noise<D>(P, K, comp, i, j, k, a, b);
+        A(i, j, k, comp) = a;
+        B(i, j, k, comp) = b;
     }
 }
 
@@ -964,16 +1002,10 @@ __device__ __forceinline__ void noise_node_body(const DevParams& P, const NoiseK
 {
     int i, j, k;
     if (!box_index(P, t, 1, 1, 1, i, j, k)) return;
-    const int iw = (i == P.n[0]) ? 0 : i, jw = (j == P.n[1]) ? 0 : j, kw = (k == P.n[2]) ? 0 : k;
-    uint32_t lin = (uint32_t)(((long)kw * P.n[1] + jw) * P.n[0] + iw);
-    // nodes on the hi plane of a wall direction are distinct: field NODE_FIELD + mask
-    const uint32_t mask = ((i == P.n[0] && !P.periodic[0]) ? 1u : 0u) |
-                          ((j == P.n[1] && !P.periodic[1]) ? 2u : 0u) |
-                          ((k == P.n[2] && !P.periodic[2]) ? 4u : 0u);
-    double za, zb;
-    noise_ab(K, NODE_FIELD + mask, lin, za, zb);
-    A(i, j, k) = za * scale;
-    B(i, j, k) = zb * scale;
+    double a, b;
+    node_noise(P, K, scale, i, j, k, a, b);
+    A(i, j, k) = a;
+    B(i, j, k) = b;
 }
 
 // One launch for a step's whole noise set (blockIdx.y: face direction 0..2, 3 = nodes); every
@@ -990,68 +1022,89 @@ __global__ void __launch_bounds__(BLK) k_noise_all(DevParams P, NoiseKey K, Arr 
     }
 }
 
-// ---- the face passes, one launch for all three directions ------------------------------------
-// blockIdx.y is the face direction; each thread runs the same per-face body as a launch of that
-// direction alone would, so the arithmetic and its order are unchanged.  A pass writes only
-// the flux of its own direction and reads shared inputs, so the directions are independent.
-// On small boxes (the wall decks), three directions' faces in one launch keep three times as
-// many waves in flight as one direction's.
+// ---- calculateFlux's face passes in one launch -----------------------------------------------
+//
+// The stochastic, diffusive, corner and hyperbolic terms of a face only add to that face's flux, so one
+// thread forms all of them in registers, in the reference's order, and the flux is written once
+// and never read back (four passes read and wrote its nvars + 4 components through memory, and read
+// the same cells four times).  The noise of a step that draws its own is evaluated in place, with
+// the bits fhdx_fill_noise gives, instead of being written once and read in each of the three stages.
+// Until the last stage of a whole step nobody sees the weighted noise and the four energy
+// components, and they are not stored (F.keep).  Consecutive work items are the three
+// directions of one chunk of faces, so they find each other's cells in L2.
+// Argon 128^3: the four passes took 1614 us a stage and the noise 269 us a step; this takes 677 us.
+// RT_3d deck (64x32x32, four species): 85 us a stage before, 54 us now.
 
-template <int NS, bool WN>
-__global__ void __launch_bounds__(BLK) k_stoch3(DevParams P, Arr prim, Arr eta, Arr zeta, Arr kappa, Arr chi,
-                                                Arr Dm, Arr f0, Arr f1, Arr f2, Arr r0, Arr r1, Arr r2, Arr rc,
-                                                NoiseW n0, NoiseW n1, NoiseW n2, double volinv, double dtinv,
-                                                double dt)
+template <int NS, int D, bool WALL>
+__device__ __forceinline__ void flux_body(const DevParams& P, const FluxArgs& F, double volinv, double dtinv, long t)
 {
-    const long t = (long)blockIdx.x * BLK + threadIdx.x;
-    if (blockIdx.y == 0)
-        stoch_body<NS, 0, WN>(P, prim, eta, zeta, kappa, chi, Dm, f0, r0, rc, n0, volinv, dtinv, dt, t);
-    else if (blockIdx.y == 1)
-        stoch_body<NS, 1, WN>(P, prim, eta, zeta, kappa, chi, Dm, f1, r1, rc, n1, volinv, dtinv, dt, t);
-    else
-        stoch_body<NS, 2, WN>(P, prim, eta, zeta, kappa, chi, Dm, f2, r2, rc, n2, volinv, dtinv, dt, t);
+    int i, j, k;
+    if (!box_index(P, t, D == 0, D == 1, D == 2, i, j, k)) return;
+    double ran[NS + 5], o[NS + 9];
+    ran[0] = 0.0;
+    const unsigned fo = off_of(F.flux[D], i, j, k);
+    const Fld flux = fld_of(F.flux[D], F.flux[D]), rn = fld_of(F.ran[D], F.flux[D]);
+    if (F.noise.mode == kNoisePhilox) {
+#pragma unroll
+        for (int c = 1; c < NS + 5; ++c) {
+            double A, B;
+            face_noise<D>(P, F.noise.K, c, i, j, k, A, B);
+            ran[c] = 1.0 * A + F.noise.w * B;
+        }
+    } else if (F.noise.mode == kNoiseSets) {
+        const Fld A = fld_of(F.noise.A[D], F.flux[D]), B = fld_of(F.noise.B[D], F.flux[D]);
+#pragma unroll
+        for (int c = 1; c < NS + 5; ++c) ran[c] = 1.0 * A(fo, c) + F.noise.w * B(fo, c);
+    } else {
+#pragma unroll
+        for (int c = 1; c < NS + 5; ++c) ran[c] = rn(fo, c);
+    }
+    if (F.noise.mode != kNoiseWeighted && F.keep)
+#pragma unroll
+        for (int c = 0; c < NS + 5; ++c) rn(fo, c) = ran[c];
+    const WallFace W = WALL ? wall_face<D>(P, i, j, k) : WallFace{false, false, 0, 0, 0};
+    const Arr& cell = F.prim;
+    FaceView V;
+    V.cons = fld_of(F.cons, cell);
+    V.prim = fld_of(F.prim, cell);
+    V.eta = fld_of(F.eta, cell);
+    V.zeta = fld_of(F.zeta, cell);
+    V.kappa = fld_of(F.kappa, cell);
+    V.chi = fld_of(F.chi, cell);
+    V.Dm = fld_of(F.D, cell);
+    V.visccorn = fld_of(F.visccorn, F.rancorn);
+    V.rancorn = fld_of(F.rancorn, F.rancorn);
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = 0; b < 3; ++b) V.corn[a][b] = fld_of(F.corn[a][b], F.rancorn);
+    V.c0 = off_of(cell, i, j, k);
+    V.cm = off_of(cell, i - (D == 0), j - (D == 1), k - (D == 2));
+    V.lo = V.cm;
+    V.up = V.c0;
+    if (WALL && W.any()) V.lo = V.up = off_of(cell, W.wi, W.wj, W.wk);
+    V.nd = off_of(F.rancorn, i, j, k);
+#pragma unroll
+    for (int c = 0; c < NS + 9; ++c) o[c] = 0.0;
+    if (P.stoch_on) stoch_part<NS, D, WALL>(P, V, W, ran, o, volinv, dtinv, F.dt, i, j, k);
+    diff_part<NS, D, WALL>(P, V, W, o);
+    corner_part<NS, D>(V, o);
+    if (P.advection_type == 1 || P.advection_type == 2) hyp_part<NS, D, WALL>(P, V, W, o, i, j, k);
+#pragma unroll
+    for (int c = 0; c < NS + 5; ++c) flux(fo, c) = o[c];
+    if (F.keep)
+#pragma unroll
+        for (int c = NS + 5; c < NS + 9; ++c) flux(fo, c) = o[c];
 }
 
-template <int NS>
-__global__ void __launch_bounds__(BLK) k_diff3(DevParams P, Arr prim, Arr eta, Arr kappa, Arr chi, Arr Dm,
-                                               Arr f0, Arr f1, Arr f2)
+template <int NS, bool WALL>
+__global__ void __launch_bounds__(BLK) k_flux(DevParams P, FluxArgs F, double volinv, double dtinv)
 {
-    const long t = (long)blockIdx.x * BLK + threadIdx.x;
-    if (blockIdx.y == 0)
-        diff_body<NS, 0>(P, prim, eta, kappa, chi, Dm, f0, t);
-    else if (blockIdx.y == 1)
-        diff_body<NS, 1>(P, prim, eta, kappa, chi, Dm, f1, t);
-    else
-        diff_body<NS, 2>(P, prim, eta, kappa, chi, Dm, f2, t);
-}
-
-// Per direction: the flux, the divergence pair and the tangential pair of corner arrays.
-struct CornerFaceSet {
-    Arr fl[3], c1[3], c2[3], ta1[3], ta2[3];
-};
-
-template <int NS>
-__global__ void __launch_bounds__(BLK) k_corner_face3(DevParams P, Arr prim, Arr vcorn, CornerFaceSet C)
-{
-    const long t = (long)blockIdx.x * BLK + threadIdx.x;
-    if (blockIdx.y == 0)
-        corner_face_body<NS, 0>(P, prim, C.fl[0], vcorn, C.c1[0], C.c2[0], C.ta1[0], C.ta2[0], t);
-    else if (blockIdx.y == 1)
-        corner_face_body<NS, 1>(P, prim, C.fl[1], vcorn, C.c1[1], C.c2[1], C.ta1[1], C.ta2[1], t);
-    else
-        corner_face_body<NS, 2>(P, prim, C.fl[2], vcorn, C.c1[2], C.c2[2], C.ta1[2], C.ta2[2], t);
-}
-
-template <int NS>
-__global__ void __launch_bounds__(BLK) k_hyp3(DevParams P, Arr cons, Arr prim, Arr f0, Arr f1, Arr f2)
-{
-    const long t = (long)blockIdx.x * BLK + threadIdx.x;
-    if (blockIdx.y == 0)
-        hyp_body<NS, 0>(P, cons, prim, f0, t);
-    else if (blockIdx.y == 1)
-        hyp_body<NS, 1>(P, cons, prim, f1, t);
-    else
-        hyp_body<NS, 2>(P, cons, prim, f2, t);
+    const unsigned item = xcd_block(blockIdx.x, gridDim.x), chunk = item / 3, d = item - 3 * chunk;
+    const long t = (long)chunk * BLK + threadIdx.x;
+    if (d == 0) flux_body<NS, 0, WALL>(P, F, volinv, dtinv, t);
+    else if (d == 1) flux_body<NS, 1, WALL>(P, F, volinv, dtinv, t);
+    else flux_body<NS, 2, WALL>(P, F, volinv, dtinv, t);
 }
 
 // ---- host launchers ---------------------------------------------------------------------
@@ -1144,45 +1197,25 @@ static void flux_passes(const DevParams& P, const FluxArgs& a, hipStream_t s)
 {
     const double volinv = 1. / (P.dx[0] * P.dx[1] * P.dx[2]);
     const double dtinv = 1. / a.dt;
-    long mf = nface(P, 0);
-    for (int d = 1; d < 3; ++d) mf = nface(P, d) > mf ? nface(P, d) : mf;
-    const dim3 grid(grid_for(mf, BLK), 3);   // every body checks its own direction's face count
-    NoiseW nw[3];
-    for (int d = 0; d < 3; ++d) nw[d] = NoiseW{a.nA[d], a.nB[d], a.rA, a.rB, a.w};
-    if (P.stoch_on && a.weigh)
-        k_stoch3<NS, true><<<grid, BLK, 0, s>>>(P, a.prim, a.eta, a.zeta, a.kappa, a.chi, a.D, a.flux[0], a.flux[1],
-                                                a.flux[2], a.ran[0], a.ran[1], a.ran[2], a.rancorn, nw[0], nw[1],
-                                                nw[2], volinv, dtinv, a.dt);
-    else if (P.stoch_on)
-        k_stoch3<NS, false><<<grid, BLK, 0, s>>>(P, a.prim, a.eta, a.zeta, a.kappa, a.chi, a.D, a.flux[0],
-                                                 a.flux[1], a.flux[2], a.ran[0], a.ran[1], a.ran[2], a.rancorn,
-                                                 nw[0], nw[1], nw[2], volinv, dtinv, a.dt);
-    k_diff3<NS><<<grid, BLK, 0, s>>>(P, a.prim, a.eta, a.kappa, a.chi, a.D, a.flux[0], a.flux[1], a.flux[2]);
-    // corn[a][b]: derivative direction a, velocity component b (cornx/corny/cornz of flux.cpp)
     const Arr(&c)[3][3] = a.corn;
     k_corner_node<<<grid_for(nnode(P), BLK), BLK, 0, s>>>(P, a.prim, a.eta, a.zeta, c[0][0], c[0][1], c[0][2],
                                                           c[1][0], c[1][1], c[1][2], c[2][0], c[2][1], c[2][2],
-                                                          a.visccorn, a.rancorn, a.rA, a.rB, a.w,
-                                                          (P.stoch_on && a.weigh) ? 1 : 0);
-    // x face: div pair (vy, wz), tangential (uy, uz); y: (ux, wz), (vx, vz); z: (vy, ux), (wx, wy)
-    CornerFaceSet C;
-    for (int d = 0; d < 3; ++d) C.fl[d] = a.flux[d];
-    C.c1[0] = c[1][1]; C.c2[0] = c[2][2]; C.ta1[0] = c[1][0]; C.ta2[0] = c[2][0];
-    C.c1[1] = c[0][0]; C.c2[1] = c[2][2]; C.ta1[1] = c[0][1]; C.ta2[1] = c[2][1];
-    C.c1[2] = c[1][1]; C.c2[2] = c[0][0]; C.ta1[2] = c[0][2]; C.ta2[2] = c[1][2];
-    k_corner_face3<NS><<<grid, BLK, 0, s>>>(P, a.prim, a.visccorn, C);
-    if (P.advection_type == 1 || P.advection_type == 2)
-        k_hyp3<NS><<<grid, BLK, 0, s>>>(P, a.cons, a.prim, a.flux[0], a.flux[1], a.flux[2]);
+                                                          a.visccorn, a.rancorn, a.noise);
+    long mf = nface(P, 0);
+    for (int d = 1; d < 3; ++d) mf = nface(P, d) > mf ? nface(P, d) : mf;
+    const unsigned grid = 3 * grid_for(mf, BLK);  // every body checks its own direction's face count
+    if (P.any_wall) k_flux<NS, true><<<grid, BLK, 0, s>>>(P, a, volinv, dtinv);
+    else k_flux<NS, false><<<grid, BLK, 0, s>>>(P, a, volinv, dtinv);
 }
 
 int ref_calculate_flux(const DevParams& P, const FluxArgs& a, int flux_ncomp[3], hipStream_t s)
 {
     const int nc = P.nvars + 4;
     for (int d = 0; d < 3; ++d) {
-        // flux_in.setVal(0) (flux.cpp:24-26): the stochastic pass writes all nvars + 4
-        // components itself; zero first only without it or for extra components
-        if (P.stoch_on && flux_ncomp[d] == nc) continue;
-        int r = fill_value(a.flux[d].p, a.flux[d].sn * flux_ncomp[d], 0.0, s);
+        // flux_in.setVal(0) (flux.cpp:24-26): the face pass writes all nvars + 4 components itself;
+        // any further ones are zeroed
+        if (flux_ncomp[d] == nc) continue;
+        int r = fill_value(a.flux[d].p + a.flux[d].sn * nc, a.flux[d].sn * (flux_ncomp[d] - nc), 0.0, s);
         if (r) return r;
     }
     NS_DISPATCH(P.ns, flux_passes<NS>(P, a, s));
@@ -1190,11 +1223,11 @@ int ref_calculate_flux(const DevParams& P, const FluxArgs& a, int flux_ncomp[3],
     return FHDX_OK;
 }
 
-int ref_stage(const DevParams& P, Arr out, Arr u0, Arr us, const Arr flux[3], Arr source, double dt, int mode,
-              hipStream_t s)
+int ref_stage(const DevParams& P, Arr out, Arr u0, Arr us, const Arr flux[3], Arr source, Arr prim, double dt,
+              int mode, hipStream_t s)
 {
     NS_DISPATCH(P.ns, (k_stage<NS><<<grid_for(ncell(P), BLK), BLK, 0, s>>>(P, out, u0, us, flux[0], flux[1],
-                                                                             flux[2], source, dt, mode)));
+                                                                             flux[2], source, prim, dt, mode)));
     FHDX_HIP_TRY(hipGetLastError());
     return FHDX_OK;
 }
@@ -1211,25 +1244,6 @@ int ref_chem_source(const DevParams& P, Arr prim, Arr source, Arr ranchem, doubl
 int ref_fill_chem_noise(const DevParams& P, const NoiseKey& K, Arr A, Arr B, hipStream_t s)
 {
     k_chem_noise<<<grid_for(ncell(P), BLK), BLK, 0, s>>>(P, K, A, B);
-    FHDX_HIP_TRY(hipGetLastError());
-    return FHDX_OK;
-}
-
-int ref_lincomb4(double* const dst[4], const double* const a[4], const double* const b[4], const long npts[4],
-                 const int nc[4], const int c0[4], double w, hipStream_t s)
-{
-    LinSet L;
-    long mx = 0;
-    for (int q = 0; q < 4; ++q) {
-        L.dst[q] = dst[q];
-        L.a[q] = a[q];
-        L.b[q] = b[q];
-        L.npts[q] = npts[q];
-        L.nc[q] = nc[q];
-        L.c0[q] = c0[q];
-        mx = npts[q] > mx ? npts[q] : mx;
-    }
-    k_lincomb4<<<grid_for(mx, BLK), BLK, 0, s>>>(L, w);
     FHDX_HIP_TRY(hipGetLastError());
     return FHDX_OK;
 }
