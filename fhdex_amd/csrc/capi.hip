@@ -509,8 +509,7 @@ int rk3_ref(fhdx_ctx* c, const StageArrays& A, const NoiseKey* K, double dt, hip
     for (int st = 0; st < 3; ++st) {
         int r;
         if ((r = rk3_stage(c, P, A, K, st == 2, st, dt, s))) return r;
-        if ((r = ref_fill_boundary2(P, make_arr(out[st]), P.nvars, make_arr(A.prim), P.nprim, s))) return r;
-        if ((r = ref_set_bc(P, make_arr(A.prim), make_arr(out[st]), s))) return r;  // timeStep.cpp:209, 314, 425
+        if ((r = ref_ghosts(P, make_arr(A.prim), make_arr(out[st]), s))) return r;  // timeStep.cpp:204-209, 309-314, 417-425
     }
     return FHDX_OK;
 }

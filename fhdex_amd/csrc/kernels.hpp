@@ -33,10 +33,10 @@ int ref_c2p(const DevParams& P, Arr prim, Arr cons, hipStream_t s);
 int ref_transport(const DevParams& P, Arr prim, Arr eta, Arr zeta, Arr kappa, Arr chi, Arr Dm, int* err,
                   hipStream_t s);
 int ref_fill_boundary(const DevParams& P, Arr a, int nc, hipStream_t s);
-// The same for two arrays in one launch (a stage's state and its primitive variables).
-int ref_fill_boundary2(const DevParams& P, Arr a, int nca, Arr b, int ncb, hipStream_t s);
 // setBC: the ghost cells outside walls, faces lo x .. hi z in turn (no-op when periodic).
 int ref_set_bc(const DevParams& P, Arr prim, Arr cons, hipStream_t s);
+// Every ghost cell of a whole-domain state and its prim: FillBoundary of both, then setBC.
+int ref_ghosts(const DevParams& P, Arr prim, Arr cons, hipStream_t s);
 int fill_value(double* p, long n, double v, hipStream_t s);
 // flux_ncomp: the components of each flux FAB (>= nvars + 4)
 int ref_calculate_flux(const DevParams& P, const FluxArgs& a, int flux_ncomp[3], hipStream_t s);

@@ -164,12 +164,8 @@ __global__ void __launch_bounds__(BLK) k_transport(DevParams P, Arr prima, Arr e
 
 // Periodic ghost fill of a cell FAB: ghost (i,j,k) <- valid (i mod n, ...) along periodic
 // directions; a ghost cell outside a wall has no periodic image and is left to setBC.
-// blockIdx.y selects the array: the step fills the stage state and its primitive variables
-// (independent arrays) in one launch.
-__global__ void __launch_bounds__(BLK) k_fill_boundary(DevParams P, Arr a0, int nc0, Arr a1, int nc1)
+__global__ void __launch_bounds__(BLK) k_fill_boundary(DevParams P, Arr a, int nc)
 {
-    const Arr a = blockIdx.y == 0 ? a0 : a1;
-    const int nc = blockIdx.y == 0 ? nc0 : nc1;
     const int g = P.ngc, n0 = P.n[0], n1 = P.n[1], n2 = P.n[2];
     const int gx = n0 + 2 * g, gy = n1 + 2 * g, gz = n2 + 2 * g;
     long t = (long)blockIdx.x * BLK + threadIdx.x;
@@ -299,6 +295,94 @@ __global__ void __launch_bounds__(BLK) k_set_bc(DevParams P, Arr prim, Arr cons,
     CO(c, 4) = rho * ie + 0.5 * rho * (v[1] * v[1] + v[2] * v[2] + v[3] * v[3]);
 #undef PR
 #undef CO
+}
+
+// One face of setBC in registers: pr, co hold the mirror cell's values and become the ghost cell's.
+// For algorithm_type 2, where every component is written (k_set_bc leaves the species alone otherwise).
+template <int NS>
+__device__ __forceinline__ void wall_ghost(const DevParams& P, int f, double* pr, double* co)
+{
+    const int D = f >> 1, bm = P.bcm[f], bt = P.bct[f], bv = P.bcv[f];
+    if (bm == 2 || bm == 3)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            pr[6 + s] = P.Yw[f][s];
+            pr[6 + NS + s] = P.Xw[f][s];
+        }
+    double Y[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) Y[s] = pr[6 + s];
+    if (bm == 3) {  // x reservoir (boundary.cpp:221-238, 260-288)
+        const double rho = P.rhow[f];
+        pr[0] = co[0] = rho;
+        pr[4] = P.tw[f];
+        pr[5] = P.pw[f];
+#pragma unroll
+        for (int q = 1; q < 4; ++q) co[q] = pr[q] = 0.0;
+        const double ie = eos_energy<NS>(P, Y, P.tw[f]);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) co[5 + s] = rho * Y[s];
+        co[4] = rho * ie + 0.5 * rho * (0.0 * 0.0 + 0.0 * 0.0 + 0.0 * 0.0);
+        return;
+    }
+    if (bt == 2) pr[4] = P.tw[f];
+#pragma unroll
+    for (int q = 1; q < 4; ++q)
+        if (bv == 2 || q == 1 + D) co[q] = pr[q] = 0.0;
+    const double T = pr[4], pt = pr[5];
+    double molmix = 0.;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) molmix += Y[s] / P.M(s);
+    molmix = quot(1., molmix);
+    const double rho = quot(quot(pt, quot(P.Runiv, molmix)), T);  // GetDensity, compressible_functions.H:1481-1495
+    const double ie = eos_energy<NS>(P, Y, T);
+    pr[0] = co[0] = rho;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) co[5 + s] = rho * Y[s];
+    if (bv == 2)
+#pragma unroll
+        for (int q = 1; q < 4; ++q) co[q] = rho * pr[q];
+    co[4] = rho * ie + 0.5 * rho * (pr[1] * pr[1] + pr[2] * pr[2] + pr[3] * pr[3]);
+}
+
+// FillBoundary and setBC of a stage's state and prim in one launch, one thread per ghost cell.  Each is
+// a function of one valid cell: its periodic image, mirrored in the walls, through the wall rules of
+// the directions it lies outside of, x before y before z (a pass of setBC reads what the one before
+// wrote).  So nothing is read that another thread writes, and the launch replaces one fill of the
+// grown box and up to three dependent setBC launches a stage: temp_grad (80x10x10, walls all round) 26 -> 6.4 us,
+// argon 128^3 54 -> 27 us.
+template <int NS>
+__global__ void __launch_bounds__(BLK) k_ghosts(DevParams P, Arr prima, Arr consa)
+{
+    int c[3];
+    if (!ghost_cell(P.ngc, P.n[0], P.n[1], P.n[2], (long)blockIdx.x * BLK + threadIdx.x, c[0], c[1], c[2])) return;
+    int m[3], face[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int n = P.n[d];
+        const bool lo = c[d] < 0, hi = c[d] >= n;
+        face[d] = -1;
+        m[d] = c[d];
+        if (P.periodic[d]) {
+            m[d] = (c[d] % n + n) % n;  // any number of periods away
+        } else if (lo || hi) {
+            m[d] = lo ? -c[d] - 1 : 2 * (n - 1) - c[d] + 1;
+            face[d] = 2 * d + (hi ? 1 : 0);
+        }
+    }
+    const Fld prim = fld_of(prima, prima), cons = fld_of(consa, prima);
+    const unsigned from = off_of(prima, m[0], m[1], m[2]), to = off_of(prima, c[0], c[1], c[2]);
+    double pr[2 * NS + 6], co[NS + 5];
+#pragma unroll
+    for (int q = 0; q < 2 * NS + 6; ++q) pr[q] = prim(from, q);
+#pragma unroll
+    for (int q = 0; q < NS + 5; ++q) co[q] = cons(from, q);
+    for (int d = 0; d < 3; ++d)
+        if (face[d] >= 0) wall_ghost<NS>(P, face[d], pr, co);
+#pragma unroll
+    for (int q = 0; q < 2 * NS + 6; ++q) prim(to, q) = pr[q];
+#pragma unroll
+    for (int q = 0; q < NS + 5; ++q) cons(to, q) = co[q];
 }
 
 __global__ void __launch_bounds__(BLK) k_fill(double* p, long n, double v)
@@ -1157,14 +1241,7 @@ int ref_transport(const DevParams& P, Arr prim, Arr eta, Arr zeta, Arr kappa, Ar
 
 int ref_fill_boundary(const DevParams& P, Arr a, int nc, hipStream_t s)
 {
-    k_fill_boundary<<<grid_for(ngrown(P), BLK), BLK, 0, s>>>(P, a, nc, a, nc);
-    FHDX_HIP_TRY(hipGetLastError());
-    return FHDX_OK;
-}
-
-int ref_fill_boundary2(const DevParams& P, Arr a, int nca, Arr b, int ncb, hipStream_t s)
-{
-    k_fill_boundary<<<dim3(grid_for(ngrown(P), BLK), 2), BLK, 0, s>>>(P, a, nca, b, ncb);
+    k_fill_boundary<<<grid_for(ngrown(P), BLK), BLK, 0, s>>>(P, a, nc);
     FHDX_HIP_TRY(hipGetLastError());
     return FHDX_OK;
 }
@@ -1180,6 +1257,18 @@ int ref_set_bc(const DevParams& P, Arr prim, Arr cons, hipStream_t s)
             if (e != d) slab *= P.bn[e] + 2 * g;
         NS_DISPATCH(P.ns, (k_set_bc<NS><<<grid_for(slab, BLK), BLK, 0, s>>>(P, prim, cons, d)));
     }
+    FHDX_HIP_TRY(hipGetLastError());
+    return FHDX_OK;
+}
+
+int ref_ghosts(const DevParams& P, Arr prim, Arr cons, hipStream_t s)
+{
+    if (P.any_wall && P.algorithm_type != 2) {  // setBC then leaves the species of a ghost cell alone
+        int r = ref_fill_boundary(P, cons, P.nvars, s);
+        if (!r) r = ref_fill_boundary(P, prim, P.nprim, s);
+        return r ? r : ref_set_bc(P, prim, cons, s);
+    }
+    NS_DISPATCH(P.ns, (k_ghosts<NS><<<grid_for(ngrown(P) - ncell(P), BLK), BLK, 0, s>>>(P, prim, cons)));
     FHDX_HIP_TRY(hipGetLastError());
     return FHDX_OK;
 }

@@ -94,13 +94,13 @@ __device__ inline void store_cell(const DevParams& P, const Fld& F, V value, int
     }
 }
 
-// ---- periodic ghost fill: thread t of the G^3 - n^3 ghost cells ---------------------------
+// ---- periodic ghost fill: thread t of the ghost cells of a box (the z slabs, the y slabs between
+// them, the x slabs); false past the last -----------------------------------------------------
 
-__device__ inline void ghost_body(const Arr& a, int nc, int g, int n0, int n1, int n2, long t)
+__device__ inline bool ghost_cell(int g, int n0, int n1, int n2, long t, int& i, int& j, int& k)
 {
     const int G0 = n0 + 2 * g, G1 = n1 + 2 * g;
     const long zs = 2L * g * G0 * G1, ys = 2L * g * G0 * n2, xs = 2L * g * n1 * n2;
-    int i, j, k;
     if (t < zs) {
         int kk = (int)(t / ((long)G0 * G1));
         long r = t % ((long)G0 * G1);
@@ -120,8 +120,15 @@ __device__ inline void ghost_body(const Arr& a, int nc, int g, int n0, int n1, i
         int ii = (int)(r % (2 * g));
         i = ii < g ? ii - g : n0 + ii - g;
     } else {
-        return;
+        return false;
     }
+    return true;
+}
+
+__device__ inline void ghost_body(const Arr& a, int nc, int g, int n0, int n1, int n2, long t)
+{
+    int i, j, k;
+    if (!ghost_cell(g, n0, n1, n2, t, i, j, k)) return;
     const int iv = (i + n0) % n0, jv = (j + n1) % n1, kv = (k + n2) % n2;
     for (int n = 0; n < nc; ++n) a(i, j, k, n) = a(iv, jv, kv, n);
 }
