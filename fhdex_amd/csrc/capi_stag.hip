@@ -131,39 +131,27 @@ int fill_stage_end(const fhdx_ctx* c, Arr cons, const Arr mom[3], const Arr vel[
 {
     FillList L{};
     L.g = c->p.ngc;
-    L.item[0] = FillItem{cons, -1, 0, c->dp.nvars};
+    L.add(cons, 0, c->dp.nvars);
     for (int d = 0; d < 3; ++d) {
-        L.item[1 + d] = FillItem{mom[d], d, 0, 1};
-        L.item[4 + d] = FillItem{vel[d], d, 0, 1};
+        L.add(mom[d], 1 + d, 1);
+        L.add(vel[d], 1 + d, 1);
     }
-    L.item[7] = FillItem{prim, -1, 0, c->dp.nprim};
-    int count = 8;
+    L.add(prim, 0, c->dp.nprim);
     if (tr) {
         const int NS = c->p.nspecies;
-        L.item[8] = FillItem{tr->eta, -1, 0, 1};
-        L.item[9] = FillItem{tr->zeta, -1, 0, 1};
-        L.item[10] = FillItem{tr->kappa, -1, 0, 1};
-        L.item[11] = FillItem{tr->chi, -1, 0, NS};
-        L.item[12] = FillItem{tr->D, -1, 0, NS * NS};
-        count = 13;
+        L.add(tr->eta, 0, 1);
+        L.add(tr->zeta, 0, 1);
+        L.add(tr->kappa, 0, 1);
+        L.add(tr->chi, 0, NS);
+        L.add(tr->D, 0, NS * NS);
     }
-    return stag_fill(c->dp, L, count, s);
-}
-
-// The density ghosts conservedToPrimitiveStag reads (face velocities at index 0).
-int fill_density(const fhdx_ctx* c, Arr cons, hipStream_t s)
-{
-    FillList L{};
-    L.g = c->p.ngc;
-    L.item[0] = FillItem{cons, -1, 0, 1};
-    return stag_fill(c->dp, L, 1, s);
+    return stag_fill(c->dp, L, s);
 }
 
 int c2p_with_ghosts(const fhdx_ctx* c, Arr prim, const Arr vel[3], Arr cons, const Arr mom[3], const StagTransport* tr,
                     hipStream_t s)
 {
-    int r = fill_density(c, cons, s);
-    if (!r) r = stag_c2p(c->dp, prim, vel, cons, mom, tr, s);
+    int r = stag_c2p(c->dp, prim, vel, cons, mom, tr, s);
     if (!r) r = fill_stage_end(c, cons, mom, vel, prim, tr, s);
     return r;
 }
@@ -242,7 +230,7 @@ int fhdx_calculate_flux_stag(fhdx_ctx* c, fhdx_fab cu, const fhdx_fab cumom[3], 
         return r;
     if (int r = ensure_stag(c)) return r;
     const StagArrays A = stag_arrays(c, cu, cumom, prim, vel, eta, zeta, kappa, chi, D, faceflux, edgeflux, cenflux);
-    return stag_flux(c->dp, A, make_noise_key(seed, step, 0), weight, dt, SS(stream));
+    return stag_flux(c->dp, A, make_noise_key(seed, step, 0), weight, dt, true, SS(stream));
 }
 
 int fhdx_rk3_step_stag(fhdx_ctx* c, fhdx_fab cu, const fhdx_fab cumom[3], fhdx_fab prim, const fhdx_fab vel[3],
@@ -292,7 +280,7 @@ int fhdx_rk3_step_stag(fhdx_ctx* c, fhdx_fab cu, const fhdx_fab cumom[3], fhdx_f
         const Arr* outm = st == 0 ? m1 : st == 1 ? m2 : m0;
         A.cu = us;
         for (int d = 0; d < 3; ++d) A.mom[d] = ms[d];
-        if ((r = stag_flux(c->dp, A, K, wts[st], dt, s))) return r;
+        if ((r = stag_flux(c->dp, A, K, wts[st], dt, st == 2, s))) return r;
         StagUpdate U;
         U.chem = chem;
         U.prim = A.prim;

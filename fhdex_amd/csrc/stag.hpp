@@ -30,14 +30,26 @@ struct StagUpdate {
     double w;
 };
 
-// Periodic ghost fill: array a (cell: nodal -1, face: nodal d), components c0 .. c0+nc-1.
+// Periodic ghost fill: nc consecutive components from p on, of a cell array (kind 0) or a face
+// array of direction kind-1; all arrays of a kind have one shape.
+constexpr int kFillComps = 4;  // most components of one item
 struct FillItem {
-    Arr a;
-    int nodal, c0, nc;
+    double* p;
+    int kind, nc;
 };
+// 37 items at eight species with the transport arrays: 4 for the state, 6 for prim, 16 for D, 2 for
+// chi, 3 coefficients, 3 momenta and 3 velocities.
 struct FillList {
-    FillItem item[13];
-    int g;  // ghost layers
+    Arr shape[4];
+    FillItem item[40];
+    int g;      // ghost layers
+    int count;
+    void add(const Arr& a, int kind, int nc)
+    {
+        shape[kind] = a;
+        for (int c = 0; c < nc; c += kFillComps)
+            item[count++] = FillItem{a.p + c * a.sn, kind, nc - c < kFillComps ? nc - c : kFillComps};
+    }
 };
 
 // The transport arrays conservedToPrimitiveStag may also fill (valid cells) from the prim it
@@ -48,14 +60,15 @@ struct StagTransport {
 };
 
 // calculateFluxStag with the noise A + w B of the step's Philox sets (key K).
-int stag_flux(const DevParams& P, const StagArrays& A, const NoiseKey& K, double w, double dt, hipStream_t s);
+// keep: store every component of faceflux, also those the stage update does not read.
+int stag_flux(const DevParams& P, const StagArrays& A, const NoiseKey& K, double w, double dt, bool keep, hipStream_t s);
 // Stage st (0, 1, 2) of RK3stepStag's combination.
 int stag_update(const DevParams& P, const StagUpdate& U, int st, double dt, hipStream_t s);
-// conservedToPrimitiveStag on the valid box (cons' density ghosts must be current); with tr set,
+// conservedToPrimitiveStag on the valid box (no ghost cell is read); with tr set,
 // also calculateTransportCoeffs of each valid cell's new prim (their ghosts are periodic images).
 int stag_c2p(const DevParams& P, Arr prim, const Arr vel[3], Arr cons, const Arr mom[3], const StagTransport* tr,
              hipStream_t s);
-// FillBoundary(periodicity) of the first `count` items.
-int stag_fill(const DevParams& P, const FillList& L, int count, hipStream_t s);
+// FillBoundary(periodicity) of the list's items.
+int stag_fill(const DevParams& P, const FillList& L, hipStream_t s);
 
 }  // namespace fhdx

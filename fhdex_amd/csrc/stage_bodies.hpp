@@ -66,6 +66,26 @@ inline Grid grid_of(const DevParams& P)
     return G;
 }
 
+// ---- views of caller arrays, and the order of blocks -----------------------------------------
+
+// The entry points check that every cell array of a call has one shape, and likewise its face arrays
+// of a direction and its node arrays, so a thread forms one byte offset per kind and every access is a
+// scalar base and that offset (Fld), not an index product of each array's own strides.
+__device__ __forceinline__ Fld fld_of(const Arr& a, const Arr& like) { return Fld{a.p, like.sn, like.sy, like.sz}; }
+__device__ __forceinline__ unsigned off_of(const Arr& a, int i, int j, int k)
+{
+    return (unsigned)((i - a.lo0) + (j - a.lo1) * a.sy + (k - a.lo2) * a.sz) << 3;
+}
+
+// Thread number with the blocks of an XCD contiguous: workgroup b runs on XCD b % 8, and XCD x takes
+// the block numbers [x nb/8, (x+1) nb/8), so the rows and planes that neighbouring blocks share are
+// fetched into one L2 instead of several.
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb)
+{
+    const unsigned xcd = b & 7, r = b >> 3, per = nb >> 3, rem = nb & 7;
+    return xcd * per + (xcd < rem ? xcd : rem) + r;
+}
+
 // ---- stores with periodic images ------------------------------------------------------------
 
 // Stores value(c), c < NC, for valid cell (i,j,k) at byte offset cb and at each periodic image of
