@@ -558,6 +558,7 @@ int fhdx_ctx_create(const fhdx_params* p, fhdx_ctx** out)
         delete c;
         return FHDX_ERR_HIP;
     }
+    c->fused.rec_in_update = records_in_update(p->nspecies, (long)p->n_cells[0] * p->n_cells[1] * p->n_cells[2]);
     // this device's copy of the no-allocation scratch, looked up once per device
     if ((r = noalloc_scratch_init(c->device))) {
         (void)hipFree(c->d_err);
@@ -1153,7 +1154,7 @@ int fhdx_ctx_autotune(fhdx_ctx* c, fhdx_fab cu, double dt, int trial_steps, fhdx
         return q;
     };
     // coordinate descent from the default shape: each parameter swept with the others fixed
-    fhdx_tune cur{64, 1, 1, 1, 0, 0, 0.};
+    fhdx_tune cur{64, 4, 1, 1, 0, 0, 0.};
     if (!r) {
         int q = trial(cur);
         if (q) fail(q, "trial step failed");

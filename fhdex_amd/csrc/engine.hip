@@ -12,14 +12,6 @@ namespace fhdx {
 
 constexpr int EB = 256;
 
-__device__ inline void dec3(long t, int nx, int ny, int& i, int& j, int& k)
-{
-    i = (int)(t % nx);
-    long r = t / nx;
-    j = (int)(r % ny);
-    k = (int)(r / ny);
-}
-
 __device__ inline NoiseKey inst_key(const Inst& in)
 {
     NoiseKey K;
@@ -36,52 +28,64 @@ __device__ inline double* stage_out(const Inst& in, int st) { return st == 0 ? i
 
 // Work items are taken in xcd_block order: the chunks of one instance (and the z neighbours a chunk
 // reads) stay on one XCD and its L2.
-#define EB_CELL_PROLOGUE                                       \
-    const WorkItem wi = W[xcd_block(blockIdx.x, gridDim.x)];    \
-    const Inst& in = I[wi.inst];                               \
+// The descriptor through the constant address space: its uniform fields come by scalar loads also
+// behind the kernel's own stores (no kernel writes a descriptor that another of its launch reads).
+__device__ __forceinline__ const Inst& inst_at(const Inst* I, int inst)
+{
+    typedef const Inst __attribute__((address_space(4))) * Ptr;
+    return *(const Inst*)((Ptr)I + __builtin_amdgcn_readfirstlane(inst));
+}
+
+#define EB_CELL_PROLOGUE(ITEM)                                 \
+    const WorkItem wi = W[ITEM];                               \
+    const Inst& in = inst_at(I, wi.inst);                      \
     const long t = (long)wi.chunk * EB + threadIdx.x;          \
     if (t >= in.ncell || in.step >= in.step_end) return;       \
     int i, j, k;                                               \
-    dec3(t, in.P.n[0], in.P.n[1], i, j, k);                    \
+    split3((unsigned)t, in.P.n[0], in.P.n[1], i, j, k);        \
     const Grid G = in.G;
 
 template <int NS>
 __global__ void __launch_bounds__(EB) kb_cells(const Inst* __restrict__ I, const WorkItem* __restrict__ W, int st)
 {
-    EB_CELL_PROLOGUE
+    EB_CELL_PROLOGUE(xcd_block(blockIdx.x, gridDim.x))
     cell_body<NS>(in.P, G.fld(stage_in(in, st)), G.fld(in.R), in.err, i, j, k, G.off(i, j, k));
 }
 
 __global__ void __launch_bounds__(EB) kb_nodes(const Inst* __restrict__ I, const WorkItem* __restrict__ W, double w)
 {
-    EB_CELL_PROLOGUE
+    EB_CELL_PROLOGUE(xcd_block(blockIdx.x, gridDim.x))
     node_body<true>(in.P, G.fld(in.R), G.fld(in.N), G.fld(in.R), G.fld(in.R), inst_key(in), w, i, j, k,
                     G.off(i, j, k));
 }
 
 template <int NS>
-__global__ void __launch_bounds__(EB) kb_faces(const Inst* __restrict__ I, const WorkItem* __restrict__ W, int st,
+__global__ void __launch_bounds__(EB, NS == 2 ? 4 : 1) kb_faces(const Inst* __restrict__ I, const WorkItem* __restrict__ W, int st,
                                                double w)
 {
-    constexpr int nv = NS + 5;
-    EB_CELL_PROLOGUE
+    // a chunk's three directions are consecutive items on one XCD (see k_faces)
+    const unsigned item = xcd_block(blockIdx.x, gridDim.x), chunk = item / 3, dir = item - 3 * chunk;
+    EB_CELL_PROLOGUE(chunk)
     const unsigned cb = G.off(i, j, k);
     const Fld Us = G.fld(stage_in(in, st)), R = G.fld(in.R), N = G.fld(in.N);
     const NoiseKey K = inst_key(in);  // noise evaluated in place (no A/B arrays)
-    double f[nv];
-    face_flux<NS, 0, true>(in.P, Us, R, N, R, R, K, w, in.volinv, in.dtinv, in.dt, i, j, k, cb, f);
-    store_face<NS, 0>(in.P, G.fld(in.F[0]), f, i, j, k, cb);
-    face_flux<NS, 1, true>(in.P, Us, R, N, R, R, K, w, in.volinv, in.dtinv, in.dt, i, j, k, cb, f);
-    store_face<NS, 1>(in.P, G.fld(in.F[1]), f, i, j, k, cb);
-    face_flux<NS, 2, true>(in.P, Us, R, N, R, R, K, w, in.volinv, in.dtinv, in.dt, i, j, k, cb, f);
-    store_face<NS, 2>(in.P, G.fld(in.F[2]), f, i, j, k, cb);
+    double f[NS + 5];
+#define FHDX_FACE(D)                                                                                          \
+    {                                                                                                         \
+        face_flux<NS, D, true>(in.P, Us, R, N, R, R, K, w, in.volinv, in.dtinv, in.dt, i, j, k, cb, f);       \
+        store_face<NS, D>(in.P, G.fld(in.F[D]), f, i, j, k, cb);                                              \
+    }
+    if (dir == 0) FHDX_FACE(0)
+    else if (dir == 1) FHDX_FACE(1)
+    else FHDX_FACE(2)
+#undef FHDX_FACE
 }
 
 // REC: also write the next stage's cell records (stages 1 and 2), so kb_cells runs once a step.
 template <int NS, bool REC>
 __global__ void __launch_bounds__(EB) kb_update(const Inst* __restrict__ I, const WorkItem* __restrict__ W, int st)
 {
-    EB_CELL_PROLOGUE
+    EB_CELL_PROLOGUE(xcd_block(blockIdx.x, gridDim.x))
     const Fld rn = G.fld(in.R);
     // prim is not written here: engine_read / fhdx_engine_state compute it from U on request
     update_body<NS>(in.P, G.fld(stage_out(in, st)), G.fld(in.U), G.fld(stage_in(in, st)), G.fld(in.F[0]),
@@ -97,7 +101,7 @@ __global__ void __launch_bounds__(EB) kb_prim(DevParams P, Grid G, const double*
     const long t = (long)blockIdx.x * EB + threadIdx.x;
     if (t >= ncell) return;
     int i, j, k;
-    dec3(t, P.n[0], P.n[1], i, j, k);
+    split3((unsigned)t, P.n[0], P.n[1], i, j, k);
     const unsigned cb = G.off(i, j, k);
     const Fld u = G.fld(const_cast<double*>(U));
     double c[NS + 5], pr[2 * NS + 6];
@@ -384,11 +388,13 @@ static void enqueue_group(Engine* e, int g, const double ws[3])
     const Inst* I = e->d_inst;
     const WorkItem* Wc = e->d_cells[g];
     // ghost images come with every store (store_cell): no fill launches inside the step
-    kb_cells<NS><<<nc, EB, 0, s>>>(I, Wc, 0);
+    // the records come with the update of the stage before where that pays for an ensemble's boxes
+    constexpr bool rec = NS <= 4;  // records_in_update's line for boxes of ensemble size
     for (int st = 0; st < 3; ++st) {
+        if (st == 0 || !rec) kb_cells<NS><<<nc, EB, 0, s>>>(I, Wc, st);
         kb_nodes<<<nc, EB, 0, s>>>(I, Wc, ws[st]);
-        kb_faces<NS><<<nc, EB, 0, s>>>(I, Wc, st, ws[st]);
-        if (st < 2) kb_update<NS, true><<<nc, EB, 0, s>>>(I, Wc, st);
+        kb_faces<NS><<<3 * nc, EB, 0, s>>>(I, Wc, st, ws[st]);
+        if (st < 2 && rec) kb_update<NS, rec><<<nc, EB, 0, s>>>(I, Wc, st);
         else kb_update<NS, false><<<nc, EB, 0, s>>>(I, Wc, st);
     }
 }

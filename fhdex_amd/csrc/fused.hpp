@@ -68,15 +68,26 @@ struct FusedWorkspace {
     double *rA = nullptr, *rB = nullptr;
     // launch shape (fhdx_ctx_autotune picks it by timing the candidates on the device)
     int tw_max = 64;           // tile width limit in x (16, 32, 64); tile height 256 / width
-    int rh = 1;                // tiles per region of the region-major block order
+    int rh = 4;                // rows of tiles per region of the region-major block order
     int kz = 1;                // z levels each tile block marches through
     bool noise_inline = true;  // Philox noise evaluated in the faces/nodes, or once into arrays
     int face_bpc = 0;          // cap on resident k_faces blocks per CU (0: none)
-    bool rec_in_update = false;  // stages 1-2: k_update writes the next stage's records
+    bool rec_in_update = false;  // stages 1-2: k_update writes the next stage's records (see records_in_update)
     Timing timing;
 };
 
 void fused_free(FusedWorkspace& w);
+
+// Whether a context's step starts with the next stage's records written by the update kernel: it saves
+// two launches and a read of the state a step, and costs the update kernel the transport's registers, so
+// it pays while launches and latency count or the transport is light.  ms a step, apart / in the update:
+// two species 32^3 .151/.138, 64^3 .361/.351, 128^3 2.62/2.48, 192^3 8.38/8.24, 256^3 19.57/19.84; four
+// species 32^3 .200/.182, 64^3 .605/.560, 128^3 4.11/4.06, 160^3 8.55/8.77; eight species 24^3 .390/.400,
+// 48^3 1.02/1.28, 64^3 2.02/2.24.
+inline bool records_in_update(int ns, long cells)
+{
+    return ns == 2 ? cells <= 8L << 20 : ns <= 4 && cells <= 3L << 20;
+}
 
 // Species counts above this evaluate the step's Philox noise into arrays (k_noise) before the
 // stages, whatever noise_inline says.  At NS = 8 the face kernel with the noise evaluated in

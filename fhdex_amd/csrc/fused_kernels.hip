@@ -24,14 +24,6 @@ namespace fhdx {
 
 constexpr int FB = 256;
 
-__device__ inline void decode3(long t, int nx, int ny, int& i, int& j, int& k)
-{
-    i = (int)(t % nx);
-    long r = t / nx;
-    j = (int)(r % ny);
-    k = (int)(r / ny);
-}
-
 // ---- periodic ghost fill: one thread per ghost cell --------------------------------------
 
 __global__ void __launch_bounds__(FB) k_fill_ghosts(Grid G, double* a, int nc, int g, int n0, int n1, int n2)
@@ -55,7 +47,7 @@ __global__ void __launch_bounds__(FB) k_copy_valid(Arr src, Grid G, double* dst,
     long t = (long)blockIdx.x * FB + threadIdx.x;
     if (t >= (long)n0 * n1 * n2) return;
     int i, j, k;
-    decode3(t, n0, n1, i, j, k);
+    split3((unsigned)t, n0, n1, i, j, k);
     const Arr d = G.view(dst);
     for (int c = 0; c < nc; ++c) d(i, j, k, c) = src(i, j, k, c);
 }
@@ -63,9 +55,9 @@ __global__ void __launch_bounds__(FB) k_copy_valid(Arr src, Grid G, double* dst,
 // The z levels of the block that owns tile cell (i, j): k runs over [k0, min(k0 + kz, nz)).  k is
 // wave-uniform; taking it through readfirstlane keeps every address scalar.
 // ZM false: one level (kz == 1), no loop, so the compiler keeps nothing live across levels.
-#define TILE_LEVELS(TM, ...)                                             \
+#define TILE_LEVELS(TM, BLOCK, ...)                                      \
     int i, j, k0;                                                        \
-    if (!tile_cell(TM, P.n[0], P.n[1], i, j, k0)) return;                \
+    if (!tile_cell(TM, (int)(BLOCK), P.n[0], P.n[1], i, j, k0)) return;  \
     if (!ZM) {                                                           \
         const int k = k0;                                                \
         __VA_ARGS__                                                      \
@@ -87,7 +79,7 @@ __global__ void __launch_bounds__(FB) k_noise(DevParams P, NoiseKey K, Grid G, d
     long t = (long)blockIdx.x * FB + threadIdx.x;
     if (t >= (long)P.n[0] * P.n[1] * P.n[2]) return;
     int i, j, k;
-    decode3(t, P.n[0], P.n[1], i, j, k);
+    split3((unsigned)t, P.n[0], P.n[1], i, j, k);
     const unsigned cb = G.off(i, j, k);
     const uint32_t lin = (uint32_t)t;
     double* As[3] = {A0, A1, A2};
@@ -118,27 +110,30 @@ __global__ void __launch_bounds__(FB) k_cells(DevParams P, Grid G, double* U, do
     long t = (long)blockIdx.x * FB + threadIdx.x;
     if (t >= (long)P.n[0] * P.n[1] * P.n[2]) return;
     int i, j, k;
-    decode3(t, P.n[0], P.n[1], i, j, k);
+    split3((unsigned)t, P.n[0], P.n[1], i, j, k);
     cell_body<NS, VW>(P, G.fld(U), G.fld(R), err, i, j, k, G.off(i, j, k));
 }
 
 // ---- tiles: 2-D (x, y) blocks of 256 threads, one z level per block, region-major order ----
 //
 // A tile is tw x th cells (tw = 1 << tx_shift = min(64, next power of two >= nx), th = 256/tw).
-// A region is a column of rh tiles stacked in y.  Block numbers run over the rh tiles of one z
-// level of a region, then up z, then to the next region.  Workgroup b runs on XCD b % 8, and XCD
-// x receives the contiguous number range x*nb/8 .. (x+1)*nb/8: the blocks an XCD holds at once
-// sit on neighbouring z levels of one region, so the z-1 / z+1 and y-1 neighbours a face or node
-// reads were fetched into that XCD's L2 a few blocks earlier.  With kz > 1 a block marches
-// through kz consecutive z levels (TILE_LEVELS), reusing the level below from cache.
+// A region is the whole width of the box times rh rows of tiles.  Block numbers run over the tiles of
+// one z level of a region, x first, then up z, then to the next region; XCD x takes a contiguous
+// range of them (xcd_block).  The blocks an XCD holds at once then sit on neighbouring z levels of
+// one region, and the x, y-1, z-1 and z+1 neighbours a face or node reads were fetched into that
+// XCD's L2 a few blocks earlier; only a region's two edge rows are fetched twice.  256^3 argon, ms a
+// step by rows of a region: 4 (rh 1) 20.6, 8 19.8, 16 (rh 4, the default) 19.3, 32 19.5, 64 19.8,
+// 256 21.3; with regions one tile wide and one tile high 21.3 (nodes 902 us a launch, 717 now; update
+// 1515, 1304).  rh 4 is also best or within 1 % at 64^3, 96^3, 128^3 and 160^3.  With kz > 1 a block
+// marches through kz consecutive z levels (TILE_LEVELS), reusing the level below from cache.
 
 struct TileMap {
     int tx_shift;  // tile width 1 << tx_shift (x), height 256 >> tx_shift (y)
-    int rh;        // tiles per region (y)
-    int nrx, nry;  // regions in x and y
+    int rh;        // rows of tiles per region (y)
+    int ntx, nry;  // tiles in x, regions in y
     int n2;        // z chunks of kz levels
     int kz;        // z levels a block marches through
-    unsigned blocks() const { return (unsigned)((long)nrx * nry * n2 * rh); }
+    unsigned blocks() const { return (unsigned)((long)ntx * nry * n2 * rh); }
 };
 
 static TileMap make_tiles(int n0, int n1, int n2, int rh, int tw_max, int kz)
@@ -153,26 +148,24 @@ static TileMap make_tiles(int n0, int n1, int n2, int rh, int tw_max, int kz)
     m.tx_shift = s;
     const int tx = 1 << s, ty = FB >> s;
     const int nty = (n1 + ty - 1) / ty;
-    m.rh = rh < 1 ? 1 : (rh > nty ? nty : rh);
-    m.nrx = (n0 + tx - 1) / tx;
-    m.nry = (nty + m.rh - 1) / m.rh;
+    rh = rh < 1 ? 1 : rh;
+    m.ntx = (n0 + tx - 1) / tx;
+    m.nry = (nty + rh - 1) / rh;
+    m.rh = (nty + m.nry - 1) / m.nry;  // regions of equal height: no empty tiles where rh does not divide nty
     m.n2 = n2;
     return m;
 }
 
-__device__ inline bool tile_cell(const TileMap& m, int n0, int n1, int& i, int& j, int& k)
+__device__ inline bool tile_cell(const TileMap& m, int t, int n0, int n1, int& i, int& j, int& k)
 {
-    const int nb = gridDim.x, b = blockIdx.x;
-    const int xcd = b & 7, r = b >> 3, per = nb >> 3, rem = nb & 7;
-    const int t = xcd * per + (xcd < rem ? xcd : rem) + r;
-    const int col = m.n2 * m.rh;
+    const int level = m.rh * m.ntx, col = m.n2 * level;  // tiles of a region's level, and of a region
     const int region = t / col, q = t - region * col;
-    k = q / m.rh;
-    const int sub = q - k * m.rh;
+    k = q / level;
+    const int sub = q - k * level;
     k *= m.kz;  // first z level of the block
-    const int rx = region % m.nrx, ry = region / m.nrx;
-    i = (rx << m.tx_shift) + (threadIdx.x & ((1 << m.tx_shift) - 1));
-    j = (ry * m.rh + sub) * (FB >> m.tx_shift) + (threadIdx.x >> m.tx_shift);
+    const int ty = sub / m.ntx, tx = sub - ty * m.ntx;
+    i = (tx << m.tx_shift) + (threadIdx.x & ((1 << m.tx_shift) - 1));
+    j = (region * m.rh + ty) * (FB >> m.tx_shift) + (threadIdx.x >> m.tx_shift);
     return i < n0 && j < n1;
 }
 
@@ -182,7 +175,7 @@ template <bool INL, bool ZM>
 __global__ void __launch_bounds__(FB) k_nodes(DevParams P, TileMap tm, Grid G, double* R, double* N, double* rA,
                                               double* rB, NoiseKey K, double w)
 {
-    TILE_LEVELS(tm, node_body<INL>(P, G.fld(R), G.fld(N), G.fld(rA), G.fld(rB), K, w, i, j, k, G.off(i, j, k));)
+    TILE_LEVELS(tm, xcd_block(blockIdx.x, gridDim.x), node_body<INL>(P, G.fld(R), G.fld(N), G.fld(rA), G.fld(rB), K, w, i, j, k, G.off(i, j, k));)
 }
 
 // ---- K3: the three lower faces of each cell (flux.cpp:71-2372) -------------------------------
@@ -194,11 +187,16 @@ struct FaceArgs {
     double w, volinv, dtinv, dt;
 };
 
-// The kernel's first argument, read anew for each direction: the compiler otherwise loads every
+// A work item is one direction of a tile: the three items of a tile are consecutive on one XCD, so the
+// cells they share come from its L2, and a small box has three times the blocks, each a third as
+// long.  32^3 argon: 25 us a launch with one thread for a cell's three faces, 15 us so; 97x61x45: 86
+// and 74 us; 256^3 and four species 128^3 the same within 2 %.
+//
+// The kernel's first argument is read anew in each branch: the compiler otherwise loads every
 // parameter once for all three, runs out of scalar registers and keeps them in vector lanes
-// (v_readlane/v_writelane were 540 of the kernel's 5620 vector instructions).  With the component
-// stride separate too (face_flux) it takes 125 VGPRs instead of 156, so four waves a SIMD instead
-// of three: 3.92 -> 3.78 ms a launch at 256^3 argon.
+// (v_readlane/v_writelane were 540 of 5620 vector instructions).  Two species are capped at 128
+// VGPRs (four waves a SIMD: 3.86 ms a launch at 256^3, 4.06 uncapped at 131); at four species a
+// cap at three waves spills (867 us at 128^3 uncapped, 1175 capped).
 __device__ __forceinline__ const DevParams& kernarg_params()
 {
     typedef const DevParams __attribute__((address_space(4))) * Ptr;
@@ -208,7 +206,7 @@ __device__ __forceinline__ const DevParams& kernarg_params()
 }
 
 template <int NS, bool INL, bool ZM>
-__global__ void __launch_bounds__(FB) k_faces(DevParams P, TileMap tm, Grid G, FaceArgs a)
+__global__ void __launch_bounds__(FB, NS == 2 ? 4 : 1) k_faces(DevParams P, TileMap tm, Grid G, FaceArgs a)
 {
     const Fld Us = G.fld(a.Us), R = G.fld(a.R), N = G.fld(a.N);
 #define FHDX_FACE(D)                                                                                            \
@@ -219,11 +217,12 @@ __global__ void __launch_bounds__(FB) k_faces(DevParams P, TileMap tm, Grid G, F
                               cb, f);                                                                           \
         store_face<NS, D>(Q, G.fld(a.F[D]), f, i, j, k, cb);                                                    \
     }
-    TILE_LEVELS(tm, {
+    const unsigned item = xcd_block(blockIdx.x, gridDim.x), tile = item / 3, dir = item - 3 * tile;
+    TILE_LEVELS(tm, tile, {
         const unsigned cb = G.off(i, j, k);
-        FHDX_FACE(0)
-        FHDX_FACE(1)
-        FHDX_FACE(2)
+        if (dir == 0) FHDX_FACE(0)
+        else if (dir == 1) FHDX_FACE(1)
+        else FHDX_FACE(2)
     })
 #undef FHDX_FACE
 }
@@ -241,7 +240,7 @@ __global__ void __launch_bounds__(FB) k_update(DevParams P, TileMap tm, Grid G, 
 {
     const Fld rn = G.fld(rec);
     const ChemStage ch{rn, K, w, dV};
-    TILE_LEVELS(tm, update_body<NS>(P, G.fld(out), G.fld(u0), G.fld(us), G.fld(fx), G.fld(fy), G.fld(fz), dt, mode,
+    TILE_LEVELS(tm, xcd_block(blockIdx.x, gridDim.x), update_body<NS>(P, G.fld(out), G.fld(u0), G.fld(us), G.fld(fx), G.fld(fy), G.fld(fz), dt, mode,
                                     G.fld(prim), write_prim, i, j, k, G.off(i, j, k), REC ? &rn : nullptr, err,
                                     CHEM ? &ch : nullptr);)
 }
@@ -345,8 +344,8 @@ static void launch_stage(const DevParams& P, FusedWorkspace& w, const Grid& G, d
     T.begin(KT_FACES, s);
     // a block cap per CU is imposed by reserving LDS the kernel does not use (160 KiB per CU)
     const unsigned lds = w.face_bpc == 2 ? 64u << 10 : (w.face_bpc == 3 ? 48u << 10 : 0u);
-    if (zm) k_faces<NS, INL, true><<<ntile, FB, lds, s>>>(P, tm, G, fa);
-    else k_faces<NS, INL, false><<<ntile, FB, lds, s>>>(P, tm, G, fa);
+    if (zm) k_faces<NS, INL, true><<<3 * ntile, FB, lds, s>>>(P, tm, G, fa);
+    else k_faces<NS, INL, false><<<3 * ntile, FB, lds, s>>>(P, tm, G, fa);
     T.end(s);
     T.begin(KT_UPDATE, s);
 #define FHDX_UPD(ZMV, RECV, CHEMV)                                                                     \

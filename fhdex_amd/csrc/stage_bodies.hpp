@@ -66,6 +66,16 @@ inline Grid grid_of(const DevParams& P)
     return G;
 }
 
+// Point t of an nx x ny x ... box, x fastest.  32 bits: a component is below 4 GiB, so a box has fewer
+// than 2^29 points (the 64-bit divisions are over a hundred instructions).
+__device__ __forceinline__ void split3(unsigned t, int nx, int ny, int& i, int& j, int& k)
+{
+    const unsigned r = t / (unsigned)nx, q = r / (unsigned)ny;
+    i = (int)(t - r * (unsigned)nx);
+    j = (int)(r - q * (unsigned)ny);
+    k = (int)q;
+}
+
 // ---- views of caller arrays, and the order of blocks -----------------------------------------
 
 // The entry points check that every cell array of a call has one shape, and likewise its face arrays
