@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(EB, NS == 2 ? 4 : 1) kb_faces(const Inst* __re
     double f[NS + 5];
 #define FHDX_FACE(D)                                                                                          \
     {                                                                                                         \
-        face_flux<NS, D, true>(in.P, Us, R, N, R, R, K, w, in.volinv, in.dtinv, in.dt, i, j, k, cb, f);       \
+        face_flux<NS, D, true, true>(in.P, Us, R, N, R, R, K, w, in.volinv, in.dtinv, in.dt, i, j, k, cb, f);       \
         store_face<NS, D>(in.P, G.fld(in.F[D]), f, i, j, k, cb);                                              \
     }
     if (dir == 0) FHDX_FACE(0)

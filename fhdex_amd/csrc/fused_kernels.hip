@@ -192,39 +192,49 @@ struct FaceArgs {
 // long.  32^3 argon: 25 us a launch with one thread for a cell's three faces, 15 us so; 97x61x45: 86
 // and 74 us; 256^3 and four species 128^3 the same within 2 %.
 //
-// The kernel's first argument is read anew in each branch: the compiler otherwise loads every
-// parameter once for all three, runs out of scalar registers and keeps them in vector lanes
-// (v_readlane/v_writelane were 540 of 5620 vector instructions).  Two species are capped at 128
-// VGPRs (four waves a SIMD: 3.86 ms a launch at 256^3, 4.06 uncapped at 131); at four species a
-// cap at three waves spills (867 us at 128^3 uncapped, 1175 capped).
-__device__ __forceinline__ const DevParams& kernarg_params()
+// The arguments are one struct, read anew in each branch: the compiler otherwise loads them once for
+// all three, runs out of scalar registers and keeps them in vector lanes (v_readlane/v_writelane
+// were 540 of 5620 vector instructions).  Two species are capped at 128 VGPRs (four waves a SIMD:
+// 3.86 ms a launch at 256^3, 4.06 uncapped at 131); at four species a cap at three waves spills
+// (867 us at 128^3 uncapped, 1175 capped).
+struct FaceKernel {
+    DevParams P;
+    TileMap tm;
+    Grid G;
+    FaceArgs a;
+};
+
+__device__ __forceinline__ const FaceKernel& face_args()
 {
-    typedef const DevParams __attribute__((address_space(4))) * Ptr;
+    typedef const FaceKernel __attribute__((address_space(4))) * Ptr;
     Ptr p = (Ptr)__builtin_amdgcn_kernarg_segment_ptr();
     asm("" : "+s"(p));
-    return *(const DevParams*)p;
+    return *(const FaceKernel*)p;
+}
+
+template <int NS, int D, bool INL>
+__device__ __forceinline__ void face_item(int i, int j, int k)
+{
+    const FaceKernel& A = face_args();
+    const Grid& G = A.G;
+    const FaceArgs& a = A.a;
+    const unsigned cb = G.off(i, j, k);
+    double f[NS + 5];
+    face_flux<NS, D, INL>(A.P, G.fld(a.Us), G.fld(a.R), G.fld(a.N), G.fld(a.A[D]), G.fld(a.B[D]), a.K, a.w, a.volinv,
+                          a.dtinv, a.dt, i, j, k, cb, f);
+    store_face<NS, D>(A.P, G.fld(a.F[D]), f, i, j, k, cb);
 }
 
 template <int NS, bool INL, bool ZM>
-__global__ void __launch_bounds__(FB, NS == 2 ? 4 : 1) k_faces(DevParams P, TileMap tm, Grid G, FaceArgs a)
+__global__ void __launch_bounds__(FB, NS == 2 ? 4 : 1) k_faces(FaceKernel A)
 {
-    const Fld Us = G.fld(a.Us), R = G.fld(a.R), N = G.fld(a.N);
-#define FHDX_FACE(D)                                                                                            \
-    {                                                                                                           \
-        const DevParams& Q = kernarg_params();                                                                  \
-        double f[NS + 5];                                                                                       \
-        face_flux<NS, D, INL>(Q, Us, R, N, G.fld(a.A[D]), G.fld(a.B[D]), a.K, a.w, a.volinv, a.dtinv, a.dt, i, j, k, \
-                              cb, f);                                                                           \
-        store_face<NS, D>(Q, G.fld(a.F[D]), f, i, j, k, cb);                                                    \
-    }
+    const DevParams& P = A.P;
     const unsigned item = xcd_block(blockIdx.x, gridDim.x), tile = item / 3, dir = item - 3 * tile;
-    TILE_LEVELS(tm, tile, {
-        const unsigned cb = G.off(i, j, k);
-        if (dir == 0) FHDX_FACE(0)
-        else if (dir == 1) FHDX_FACE(1)
-        else FHDX_FACE(2)
+    TILE_LEVELS(A.tm, tile, {
+        if (dir == 0) face_item<NS, 0, INL>(i, j, k);
+        else if (dir == 1) face_item<NS, 1, INL>(i, j, k);
+        else face_item<NS, 2, INL>(i, j, k);
     })
-#undef FHDX_FACE
 }
 
 // ---- K4: stage combination (+ primitive variables after the last stage) --------------------
@@ -327,7 +337,8 @@ static void launch_stage(const DevParams& P, FusedWorkspace& w, const Grid& G, d
     if (zm) k_nodes<INL, true><<<ntile, FB, 0, s>>>(P, tm, G, w.rec, w.node, w.rA, w.rB, K, wst);
     else k_nodes<INL, false><<<ntile, FB, 0, s>>>(P, tm, G, w.rec, w.node, w.rA, w.rB, K, wst);
     T.end(s);
-    FaceArgs fa;
+    FaceKernel fk{P, tm, G, {}};
+    FaceArgs& fa = fk.a;
     fa.Us = us;
     fa.R = w.rec;
     fa.N = w.node;
@@ -344,8 +355,8 @@ static void launch_stage(const DevParams& P, FusedWorkspace& w, const Grid& G, d
     T.begin(KT_FACES, s);
     // a block cap per CU is imposed by reserving LDS the kernel does not use (160 KiB per CU)
     const unsigned lds = w.face_bpc == 2 ? 64u << 10 : (w.face_bpc == 3 ? 48u << 10 : 0u);
-    if (zm) k_faces<NS, INL, true><<<3 * ntile, FB, lds, s>>>(P, tm, G, fa);
-    else k_faces<NS, INL, false><<<3 * ntile, FB, lds, s>>>(P, tm, G, fa);
+    if (zm) k_faces<NS, INL, true><<<3 * ntile, FB, lds, s>>>(fk);
+    else k_faces<NS, INL, false><<<3 * ntile, FB, lds, s>>>(fk);
     T.end(s);
     T.begin(KT_UPDATE, s);
 #define FHDX_UPD(ZMV, RECV, CHEMV)                                                                     \

@@ -916,7 +916,10 @@ __device__ inline double bm_log(double x)
         m = m * 0.5;
         e = e + 1;
     }
-    const double sr = quot(m - 1.0, m + 1.0);
+    // m + 1 in [1.7, 2.42) and a finite dividend: no special operands, so no div_fixup
+    const Rcp d = rcp_of(m + 1.0);
+    const double q = (m - 1.0) * d.r;
+    const double sr = __builtin_fma(__builtin_fma(-d.b, q, m - 1.0), d.r, q);
     const double z = sr * sr;
     double p = 1.0 / 23.0;
     p = fma(p, z, 1.0 / 21.0);
@@ -936,12 +939,33 @@ __device__ inline double bm_log(double x)
     return de * 0.6931467056274414 + fma(de, 4.7493250390316726e-07, lm);
 }
 
+// x with its sign flipped by the top bit of w (one three-operand instruction on the high word).
+__device__ __forceinline__ double flip_sign(double x, uint32_t w)
+{
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    const uint32_t hi = __builtin_amdgcn_bitop3_b32((uint32_t)(b >> 32), w, 0x80000000u, 0x78);  // a ^ (b & c)
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | (uint32_t)b));
+}
+
+// sqrt of x = +-0 or of a normal x above 1e-290: v_rsq_f64 of zero, infinite, is held at 1e300, and the
+// refinement then returns the zero; one instruction where root() tests and selects.
+__device__ __forceinline__ double root_small(double x)
+{
+    const double y = __builtin_fmin(__builtin_amdgcn_rsq(x), 1e300);
+    double s = x * y, h = y * 0.5;
+    const double e = __builtin_fma(-h, s, 0.5);
+    s = __builtin_fma(s, e, s);
+    h = __builtin_fma(h, e, h);
+    s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+    return __builtin_fma(__builtin_fma(-s, s, x), h, s);
+}
+
 // sin(pi t) and cos(pi t) for t in [0, 2): t = n/2 + r with |r| <= 1/4 (exact), Taylor series of
 // sin(pi r) to r^19 and cos(pi r) to r^18, then the quadrant n mod 4.
 __device__ inline void bm_sincospi(double t, double& sn, double& cs)
 {
     const double n = rint(2.0 * t);
-    const double r = t - 0.5 * n;
+    const double r = fma(-0.5, n, t);  // 0.5 n is exact, so this is t - 0.5 n
     const double r2 = r * r;
     double ps = -2.2948428997269873e-08;
     ps = fma(ps, r2, 7.952054001475513e-07);
@@ -964,11 +988,12 @@ __device__ inline void bm_sincospi(double t, double& sn, double& cs)
     pc = fma(pc, r2, 4.0587121264167685);
     pc = fma(pc, r2, -4.934802200544679);
     const double C = fma(pc, r2, 1.0);
-    // quadrant q = n mod 4: (sin, cos) = (S, C), (C, -S), (-S, -C), (-C, S)
-    const int q = ((int)n) & 3;
+    // quadrant q = n mod 4: (sin, cos) = (S, C), (C, -S), (-S, -C), (-C, S): the pair swapped by q's
+    // low bit, the signs flipped in the sign bits by bit 1 of q and of q + 1
+    const int q = (int)n;
     const double a = (q & 1) ? C : S, b = (q & 1) ? S : C;
-    sn = (q & 2) ? -a : a;
-    cs = ((q + 1) & 2) ? -b : b;
+    sn = flip_sign(a, (uint32_t)q << 30);
+    cs = flip_sign(b, ((uint32_t)q << 30) + 0x40000000u);
 }
 
 // The top 53 bits of hi:lo as a double (exact): its upper 21 and lower 32 bits joined by one fma.
@@ -983,7 +1008,7 @@ __device__ inline void normal_pair(U4 r, double& z0, double& z1)
     const double two_m53 = 1.1102230246251565e-16;
     double u1 = (top53(r.x, r.y) + 0.5) * two_m53;
     double u2 = top53(r.z, r.w) * two_m53;
-    double rad = root(-2.0 * bm_log(u1));
+    double rad = root_small(-2.0 * bm_log(u1));
     double s, c;
     bm_sincospi(2.0 * u2, s, c);
     z0 = rad * c;

@@ -387,10 +387,15 @@ __device__ inline double node_sum(const Fld& N, int c, unsigned cb, bool zorder,
     return s;
 }
 
-// The nvars face fluxes of face (i,j,k) of direction D into fo[] (energy fold included).
+// The nvars face fluxes of face (i,j,k) of direction D into fo[] (energy fold included).  A product by a
+// power of two that is then added is one fma: the product is exact, so the rounding is the sum's.
 // INL: the face's A/B noise is evaluated in place from Philox key K (the values fhdx_fill_noise
 // writes for that key); otherwise it is read from the step's arrays A, B.
-template <int NS, int D, bool INL>
+// APART: the corner and hyperbolic families start after the ones before, so fewer values are live at once.
+// The ensemble's face kernel, which reads its parameters through a descriptor, takes 352 us a launch so
+// over 48 uneven boxes (2.1 M cells), 366 without; the single box's 3.463 and 3.451 ms at 256^3, 807 and
+// 789 us for four species at 128^3.
+template <int NS, int D, bool INL, bool APART = false>
 __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A, Fld B, const NoiseKey& K, double w,
                                  double volinv, double dtinv, double dt, int i, int j, int k, unsigned cb, double* fo)
 {
@@ -403,6 +408,26 @@ __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A
     constexpr int ex = (D == 0), ey = (D == 1), ez = (D == 2);
     constexpr int nv = NS + 5;
     const RecLayout L{NS};
+    // The face's weighted noise first and by itself: scheduled among the loads and the fluxes, its thirty
+    // constants and the component bases filled the scalar registers (144 of them spilled to vector
+    // lanes, 10 so; 5194 and 4890 vector instructions): 3.62 -> 3.45 ms a launch at 256^3 argon.
+    double wn[nv];
+    wn[0] = 0.;
+    if (P.stoch_on)
+#pragma unroll
+        for (int n = 1; n < nv; ++n) {
+            if (INL) {
+                const uint32_t lin = (uint32_t)(((long)k * P.n[1] + j) * P.n[0] + i);
+                const double sc = (n <= 3) ? P.var_mom : (n == 4) ? P.var_ener : P.var_mass;
+                double za, zb;
+                noise_ab(K, (uint32_t)(16 * D + n), lin, za, zb);
+                const double a = za * sc, b = zb * sc;
+                wn[n] = 1.0 * a + w * b;
+            } else {
+                wn[n] = 1.0 * A(cb, n) + w * B(cb, n);
+            }
+        }
+    if (INL) __builtin_amdgcn_sched_barrier(0);
     // record values of the two cells, loaded once and shared by the flux families below
     const double TU = R(cb, RecLayout::T), TL = R(cb, RecLayout::T, -ex, -ey, -ez);
     const double etaU = R(cb, RecLayout::ETA), etaL = R(cb, RecLayout::ETA, -ex, -ey, -ez);
@@ -442,21 +467,6 @@ __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A
         double mup = etaU * Tu + etaL * Tl;
         double kp = kapU * Tu * Tu + kapL * Tl * Tl;
         double meanT = 0.5 * (Tu + Tl);
-        double wn[nv];
-        wn[0] = 0.;
-#pragma unroll
-        for (int n = 1; n < nv; ++n) {
-            if (INL) {
-                const uint32_t lin = (uint32_t)(((long)k * P.n[1] + j) * P.n[0] + i);
-                const double sc = (n <= 3) ? P.var_mom : (n == 4) ? P.var_ener : P.var_mass;
-                double za, zb;
-                noise_ab(K, (uint32_t)(16 * D + n), lin, za, zb);
-                const double a = za * sc, b = zb * sc;
-                wn[n] = 1.0 * a + w * b;
-            } else {
-                wn[n] = 1.0 * A(cb, n) + w * B(cb, n);
-            }
-        }
         double wi[nv];
         double fw1 = root(P.k_B * mup * volinv * dtinv);
         double fw4 = root(P.k_B * kp * volinv * dtinv);
@@ -484,7 +494,7 @@ __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A
             sum = sum + N(cb, NODE_S + 2, 1, 0, 0);
             sum = sum + N(cb, NODE_S + 3);
         }
-        wi[1 + D] = wi[1 + D] + 0.25 * nweight * sum;
+        wi[1 + D] = fma(0.25, nweight * sum, wi[1 + D]);
 #pragma unroll
         for (int n = 1; n < 4; ++n) f[n] = f[n] + wi[n];
         f[nv] = f[nv] + wi[4];
@@ -492,10 +502,8 @@ __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A
         double phidiag = wi[1 + D] * (velL(1 + D) + velU(1 + D));
         double phishear = wi[t1] * (velL(t1) + velU(t1)) +
                           wi[t2] * (velL(t2) + velU(t2));
-        phidiag = -0.5 * phidiag;
-        phishear = -0.5 * phishear;
-        f[nv + 1] = f[nv + 1] - phidiag;
-        f[nv + 2] = f[nv + 2] - phishear;
+        f[nv + 1] = fma(0.5, phidiag, f[nv + 1]);
+        f[nv + 2] = fma(0.5, phishear, f[nv + 2]);
         if (species) {
             double yy[NS], yyp[NS], DijY[NS * NS], sqD[NS * NS];
 #pragma unroll
@@ -563,7 +571,7 @@ __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A
         f[2] = f[2] - (D == 1 ? tau2 + divp : tau2);
         f[3] = f[3] - (D == 2 ? tau3 + divp : tau3);
         f[nv] = f[nv] - Qflux;
-        f[nv + 1] = f[nv + 1] - (half * phiflx);
+        f[nv + 1] = fma(-half, phiflx, f[nv + 1]);
         double meanT = 0.5 * (TL + TU);
         double meanP = 0.5 * (PL + PU);
         if (species) {
@@ -609,6 +617,7 @@ __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A
         }
     }
 
+    if (APART) __builtin_amdgcn_sched_barrier(0);
     // ---- corner terms (flux.cpp:1770-1980) ----
     {
         const bool zo = (D == 2);
@@ -624,16 +633,18 @@ __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A
         double s2 = node_sum<D>(N, a2, cb, zo, 0., true);
         constexpr int cn = 1 + D;
         constexpr int tc1 = (D == 0) ? 2 : 1, tc2 = (D == 2) ? 2 : 3;
-        f[cn] = f[cn] - 0.25 * vc4;
-        f[cn] = f[cn] + .25 * div8;
-        f[tc1] = f[tc1] - .25 * s1;
-        f[tc2] = f[tc2] - .25 * s2;
-        double phiflx = 0.25 * (vc4 - div8) * (velL(cn) + velU(cn));
-        phiflx = phiflx + .25 * s1 * (velL(tc1) + velU(tc1));
-        phiflx = phiflx + .25 * s2 * (velL(tc2) + velU(tc2));
-        f[nv + 1] = f[nv + 1] - 0.5 * phiflx;
+        f[cn] = fma(-0.25, vc4, f[cn]);
+        f[cn] = fma(.25, div8, f[cn]);
+        f[tc1] = fma(-.25, s1, f[tc1]);
+        f[tc2] = fma(-.25, s2, f[tc2]);
+        // four times the reference's phiflx, every factor 1/4 taken out to the last line
+        double phiflx = (vc4 - div8) * (velL(cn) + velU(cn));
+        phiflx = phiflx + s1 * (velL(tc1) + velU(tc1));
+        phiflx = phiflx + s2 * (velL(tc2) + velU(tc2));
+        f[nv + 1] = fma(-0.125, phiflx, f[nv + 1]);
     }
 
+    if (APART) __builtin_amdgcn_sched_barrier(0);
     // ---- hyperbolic (flux.cpp:2016-2372) ----
     if (P.advection_type == 1 || P.advection_type == 2) {
         const double wgt2 = 1. / 12.;
@@ -670,7 +681,7 @@ __device__ inline void face_flux(const DevParams& P, Fld Us, Fld R, Fld N, Fld A
 #pragma unroll
             for (int n = 0; n < NS; ++n) Yk[n] = cv[5 + n] / rho;
             double vsqr = pv[1] * pv[1] + pv[2] * pv[2] + pv[3] * pv[3];
-            double ie = cv[4] / rho - 0.5 * vsqr;
+            double ie = fma(-0.5, vsqr, cv[4] / rho);
             pv[4] = eos_temperature<NS>(P, ie, Yk);
             pv[5] = eos_pressure<NS>(P, Yk, cv[0], pv[4]);
         }
