@@ -1097,7 +1097,8 @@ __device__ inline void chem_source_cell(const DevParams& P, double T, double pre
 {
     const DevChem& C = P.chem;
     const double T0 = C.T0;
-    const double ctot = pres / P.Runiv / T;
+    const Rcp rT = rcp_of(T);
+    const double ctot = quot(pres, P.Runiv) / rT;
     const double Navo = C.Navo;
     double ck[NS];
 #pragma unroll
@@ -1106,12 +1107,12 @@ __device__ inline void chem_source_cell(const DevParams& P, double T, double pre
     for (int n = 0; n < NS; ++n) src[n] = 0.;
     for (int m = 0; m < C.nreaction; ++m) {
         double rate = C.rate[m];
-        rate *= chem_exp(-C.alpha[m] / P.Runiv * (1 / T - 1 / T0));
-        rate *= chem_pow(T / T0, C.beta[m]);
+        rate *= chem_exp(quot(-C.alpha[m], P.Runiv) * (1 / rT - quot(1, T0)));
+        rate *= chem_pow(quot(T, T0), C.beta[m]);
 #pragma unroll
         for (int n = 0; n < NS; ++n) rate *= chem_ipow(ck[n], C.R[m][n]);
         rate = (0. < rate) ? rate : 0.;  // std::max(0., rate)
-        const double W = ranchem(m) / sqrt(dt * dV);
+        const double W = quot(ranchem(m), root(dt * dV));
 #pragma unroll
         for (int n = 0; n < NS; ++n) {
             src[n] += P.molmass[n] * C.PR[m][n] * rate;

@@ -756,23 +756,10 @@ struct ChemStage {
 // div[] = (fx(i+1)-fx(i))/dx + (fy(j+1)-fy(j))/dy + (fz(k+1)-fz(k))/dz, evaluated left to right.
 template <int NS>
 __device__ __forceinline__ void update_from_div(const DevParams& P, const Fld& out, const Fld& u0, const Fld& us,
-                                       const double* div, double dt, int mode, const Fld& prim, int write_prim, int i,
-                                       int j, int k, unsigned cb, const Fld* rec_next = nullptr, int* err = nullptr,
-                                       const ChemStage* chem = nullptr)
+                                       const double* div, const double* src, double dt, int mode, const Fld& prim,
+                                       int write_prim, int i, int j, int k, unsigned cb, const Fld* rec_next = nullptr,
+                                       int* err = nullptr)
 {
-    // source S: zero (main_driver.cpp:241-242) but for the species equations under chemistry
-    double src[NS + 5];
-#pragma unroll
-    for (int n = 0; n < NS + 5; ++n) src[n] = 0.0;
-    if (chem && P.chem.nreaction > 0) {
-        const RecLayout L{NS};
-        double X[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) X[s] = chem->R(cb, L.X() + s);
-        const uint32_t lin = (uint32_t)(((long)k * P.n[1] + j) * P.n[0] + i);
-        chem_source_cell<NS>(P, chem->R(cb, RecLayout::T), chem->R(cb, RecLayout::P), X,
-                             [&](int m) { return chem_noise(chem->K, m, lin, chem->w); }, dt, chem->dV, &src[5]);
-    }
     double o[NS + 5];
 #pragma unroll
     for (int n = 0; n < NS + 5; ++n) {
@@ -811,13 +798,29 @@ __device__ __forceinline__ void update_body(const DevParams& P, const Fld& out, 
                                    int i, int j, int k, unsigned cb, const Fld* rec_next = nullptr,
                                    int* err = nullptr, const ChemStage* chem = nullptr)
 {
+    // source S: zero (main_driver.cpp:241-242) but for the species equations under chemistry
+    double src[NS + 5];
+#pragma unroll
+    for (int n = 0; n < NS + 5; ++n) src[n] = 0.0;
+    if (chem && P.chem.nreaction > 0) {
+        const RecLayout L{NS};
+        double X[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) X[s] = chem->R(cb, L.X() + s);
+        const uint32_t lin = (uint32_t)(((long)k * P.n[1] + j) * P.n[0] + i);
+        chem_source_cell<NS>(P, chem->R(cb, RecLayout::T), chem->R(cb, RecLayout::P), X,
+                             [&](int m) { return chem_noise(chem->K, m, lin, chem->w); }, dt, chem->dV, &src[5]);
+    }
+    // No load below is held in registers through the reactions: 221 -> 149 VGPRs, NO2/N2O4 96^3 187 -> 162 us
+    // a launch with records, 150 -> 127 without; capped at 128 VGPRs it spills (300 us).
+    if (chem) __builtin_amdgcn_sched_barrier(0);
     double div[NS + 5];
 #pragma unroll
     for (int n = 0; n < NS + 5; ++n)
         // face n holds face 0 of the periodic box (store_face)
         div[n] = (fx(cb, n, 1, 0, 0) - fx(cb, n)) / P.h(0) + (fy(cb, n, 0, 1, 0) - fy(cb, n)) / P.h(1) +
                  (fz(cb, n, 0, 0, 1) - fz(cb, n)) / P.h(2);
-    update_from_div<NS>(P, out, u0, us, div, dt, mode, prim, write_prim, i, j, k, cb, rec_next, err, chem);
+    update_from_div<NS>(P, out, u0, us, div, src, dt, mode, prim, write_prim, i, j, k, cb, rec_next, err);
 }
 
 }  // namespace fhdx
