@@ -223,6 +223,19 @@ __device__ __forceinline__ void stag_face(const DevParams& P, const StagArrays& 
     if (tid >= (long)fx * fy * fz) return;
     int i, j, k;
     cell_of(tid, fx, fy, i, j, k);
+    // The weighted noise of the face (heat, then the species) by itself, as in the collocated face_flux:
+    // 853 -> 833 us a launch at 160^3 argon, 112 -> 101 at 64^3 with four species.
+    double zn[NS + 1];
+    if (P.stoch_on) {
+        const uint32_t lin = wrapped_lin(P, i, j, k);
+#pragma unroll
+        for (int l = 0; l < NS + 1; ++l) {
+            double za, zb;
+            noise_ab(K, STAG_FACE_FIELD + 16u * D + (uint32_t)l, lin, za, zb);
+            zn[l] = 1.0 * za + w * zb;
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
     const Fld prim = fld_of(A.prim, A.prim), cu = fld_of(A.cu, A.prim), chi = fld_of(A.chi, A.prim),
               Dm = fld_of(A.D, A.prim), kappa = fld_of(A.kappa, A.prim), td = fld_of(A.td, A.td);
     // this cell and the one below the face; the face in its velocity's layout
@@ -257,14 +270,11 @@ __device__ __forceinline__ void stag_face(const DevParams& P, const StagArrays& 
 
     // stochastic part
     if (P.stoch_on) {
-        const uint32_t lin = wrapped_lin(P, i, j, k);
         double wn[NS + 1];
         const double kp = kapU * Tu * Tu + kapL * Tl * Tl;
         const double meanT = 0.5 * (Tu + Tl);
         const double fw0 = root(P.k_B * kp * volinv * dtinv);
-        double za, zb;
-        noise_ab(K, STAG_FACE_FIELD + 16u * D + 0u, lin, za, zb);
-        wn[0] = fw0 * (1.0 * za + w * zb);
+        wn[0] = fw0 * zn[0];
         f[nv] = wn[0];
         f[nv + 1] = 0.5 * vel_f * (td(o1, D, -ed0, -ed1, -ed2) + td(o1, D));
         double vsh = 0.0;
@@ -312,19 +322,12 @@ __device__ __forceinline__ void stag_face(const DevParams& P, const StagArrays& 
             MWmix = quot(1., MWmix);
             cholesky<NS>(DijY, sqD);
             const double wsp = root(quot(P.k_B * MWmix * volinv, P.Runiv * dt));
-            double zs[NS];
-#pragma unroll
-            for (int l = 0; l < NS; ++l) {
-                double a, b;
-                noise_ab(K, STAG_FACE_FIELD + 16u * D + 1u + (uint32_t)l, lin, a, b);
-                zs[l] = 1.0 * a + w * b;
-            }
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
 #pragma unroll
                 for (int l = 0; l <= s; ++l) {
                     const double fw = wsp * sqD[s * NS + l];
-                    wn[1 + s] = wn[1 + s] + fw * zs[l];
+                    wn[1 + s] = wn[1 + s] + fw * zn[1 + l];
                 }
                 f[5 + s] = wn[1 + s];
             }
