@@ -108,7 +108,8 @@ __global__ void __launch_bounds__(EB) kb_prim(DevParams P, Grid G, const double*
 #pragma unroll
     for (int n = 0; n < NS + 5; ++n) c[n] = u(cb, n);
     cons_to_prim_cell<NS>(P, c, pr);
-    store_cell<2 * NS + 6, true>(P, G.fld(prim), [&](int n) { return pr[n]; }, i, j, k, cb);
+    store_cell<2 * NS + 6, true>(P, G.fld(prim), [&](int n) { return pr[n]; }, i, j, k, cb,
+                                  all_images(P.ngc));
 }
 
 static int compute_prim(Engine* e, const EngineSlot& s)

@@ -98,25 +98,52 @@ __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb)
 
 // ---- stores with periodic images ------------------------------------------------------------
 
+// Ghost layers that a producing kernel stores: lo[d] below the box, hi[d] above it; faces: only images
+// across one axis, no edges or corners.  What only the next kernels read gets only what they read: with
+// records, 48 uneven boxes' update 225 -> 211 us a launch and cells 101 -> 93, four species 128^3 507 -> 489
+// and 279 -> 253.  Along x every layer is stored all the same: the ghosts of a row and of the next lie
+// side by side, and a line left partly written costs more than the stores saved (four species 128^3:
+// 3.94 ms a step with every layer, 4.01 with x cut too, 3.92 so).
+struct Images {
+    int lo[3], hi[3];
+    bool faces;
+};
+
+// A caller's array: every ghost cell.
+__device__ __forceinline__ Images all_images(int g) { return {{g, g, g}, {g, g, g}, false}; }
+
+// A stage state (kept in the workspace): the four-point interpolation of a face reads cells -2..1 along
+// its own axis, nothing reads edges or corners.
+__device__ __forceinline__ Images state_images(int g) { return {{g, 2, 2}, {g, 1, 1}, true}; }
+
+// The records: faces and nodes read the cells at -1 of each axis, the z edge viscosities eta(k-2) and the
+// z Soret flux chi(k+1); primitive interpolation (advection_type 1) reads -2..1.
+__device__ __forceinline__ Images record_images(const DevParams& P)
+{
+    const int g = P.ngc;
+    if (P.advection_type == 1) return {{g, 2, 2}, {g, 1, 1}, false};
+    return {{g, 1, 2}, {g, 0, 1}, false};
+}
+
 // Stores value(c), c < NC, for valid cell (i,j,k) at byte offset cb and at each periodic image of
-// the cell that lies in the ngc ghost layers (up to 7), so no separate ghost-fill pass is needed.
+// the cell in the layers of im (up to 7), so no separate ghost-fill pass is needed.
 // Requires n >= 2 ngc on every axis (a cell then has at most one image per axis).
 // NT: streaming stores for the cell itself (the images are few and stay ordinary stores).
 template <int NC, bool NT = false, typename V>
-__device__ inline void store_cell(const DevParams& P, const Fld& F, V value, int i, int j, int k, unsigned cb)
+__device__ inline void store_cell(const DevParams& P, const Fld& F, V value, int i, int j, int k, unsigned cb,
+                                  const Images& im)
 {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         if (NT) F.put_nt(cb, c, value(c));
         else F(cb, c) = value(c);
     }
-    const int g = P.ngc;
-    const int ax = i < g ? P.n[0] : (i >= P.n[0] - g ? -P.n[0] : 0);
-    const int ay = j < g ? P.n[1] : (j >= P.n[1] - g ? -P.n[1] : 0);
-    const int az = k < g ? P.n[2] : (k >= P.n[2] - g ? -P.n[2] : 0);
+    const int ax = i < im.hi[0] ? P.n[0] : (i >= P.n[0] - im.lo[0] ? -P.n[0] : 0);
+    const int ay = j < im.hi[1] ? P.n[1] : (j >= P.n[1] - im.lo[1] ? -P.n[1] : 0);
+    const int az = k < im.hi[2] ? P.n[2] : (k >= P.n[2] - im.lo[2] ? -P.n[2] : 0);
     if ((ax | ay | az) == 0) return;
     for (int m = 1; m < 8; ++m) {
-        if (((m & 1) && !ax) || ((m & 2) && !ay) || ((m & 4) && !az)) continue;
+        if (((m & 1) && !ax) || ((m & 2) && !ay) || ((m & 4) && !az) || (im.faces && (m & (m - 1)))) continue;
         const int d = ((m & 1) ? ax : 0) + ((m & 2) ? ay : 0) * F.sy + ((m & 4) ? az : 0) * F.sz;
         const unsigned cbi = cb + (unsigned)(d * 8);  // modulo 2^32: negative shifts wrap correctly
 #pragma unroll
@@ -210,7 +237,7 @@ __device__ __forceinline__ void cell_record(const DevParams& P, const double* c,
     }
 #pragma unroll
     for (int q = 0; q < NS * NS; ++q) rec[L.D() + q] = D[q];
-    store_cell<8 + 4 * NS + NS * NS>(P, R, [&](int q) { return rec[q]; }, i, j, k, cb);
+    store_cell<8 + 4 * NS + NS * NS>(P, R, [&](int q) { return rec[q]; }, i, j, k, cb, record_images(P));
 }
 
 template <int NS, bool VW = false>
@@ -782,13 +809,14 @@ __device__ __forceinline__ void update_from_div(const DevParams& P, const Fld& o
         for (int n = 0; n < 3; ++n) o[n + 1] += 2. / 3. * dt * r0 * g[n];
         o[4] += 2. / 3. * dt * (g[0] * r1 + g[1] * r2 + g[2] * r3);
     }
-    store_cell<NS + 5, true>(P, out, [&](int n) { return o[n]; }, i, j, k, cb);
+    store_cell<NS + 5, true>(P, out, [&](int n) { return o[n]; }, i, j, k, cb,
+                             mode < 2 ? state_images(P.ngc) : all_images(P.ngc));
     // the next stage's record depends on this cell's new state only: computed here from registers
     if (rec_next) cell_record<NS>(P, o, *rec_next, err, i, j, k, cb);
     if (write_prim) {
         double pr[2 * NS + 6];
         cons_to_prim_cell<NS>(P, o, pr);
-        store_cell<2 * NS + 6, true>(P, prim, [&](int n) { return pr[n]; }, i, j, k, cb);
+        store_cell<2 * NS + 6, true>(P, prim, [&](int n) { return pr[n]; }, i, j, k, cb, all_images(P.ngc));
     }
 }
 
