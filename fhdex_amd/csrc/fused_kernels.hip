@@ -6,15 +6,15 @@
 //   k_cells    conservedToPrimitive + transport coefficients, once per valid cell, into a
 //              ghost-padded record (u, v, w, T, p, eta, kappa, zeta, Y, X, clamped Y, chi, D);
 //   k_nodes    corner velocity gradients, visccorn and the stage-weighted node noise;
-//   k_faces    all four flux families (stochastic, diffusive, corner, hyperbolic) of the three
-//              lower faces of each cell, accumulated in registers in the reference's
-//              per-component order with the energy fold;
+//   k_faces    all four flux families (stochastic, diffusive, corner, hyperbolic) of a cell's lower
+//              face in one direction (three blocks a tile), accumulated in registers in the
+//              reference's per-component order with the energy fold;
 //   k_update   divergence + RK3 stage combination (+ the next stage's cell records after stages 1
 //              and 2, primitive variables after stage 3).
 // Every array of the box shares one layout (Grid), so a kernel computes each cell offset once
 // and addresses all arrays as scalar base + 32-bit offset.  Records, stage states and prim are
-// written with their periodic ghost images by the producing kernel; only the caller's cu gets
-// a ghost fill, once per step.  Every value is computed with the reference's operation order, so the step is
+// written with the periodic ghost images that are read later by the producing kernel; only the
+// caller's cu gets a ghost fill, once per step.  Every value is computed with the reference's operation order, so the step is
 // bit-identical to the reference-shaped path.
 #include "fused.hpp"
 #include "kernels.hpp"

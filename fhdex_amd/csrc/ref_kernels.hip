@@ -1,8 +1,9 @@
 // ref_kernels.hip -- the reference-shaped kernels of calculateFlux / RK3step on gfx950.
 //
-// One kernel per pass of the reference (transport, stochastic, diffusive, corner, corner-to-
-// face, hyperbolic fluxes, stage combination, noise), each thread owning one cell, face or
-// node.  These back the drop-in entry points that fill the reference's own intermediate
+// A stage is transport, corner nodes, faces (every flux family of a face and its noise in one pass, the
+// three directions in one launch), the stage combination with the conversion to primitive variables,
+// and every ghost cell in one launch; each thread owns one cell, face or node.  These back the drop-in
+// entry points that fill the reference's own intermediate
 // arrays (fhdx_calculate_flux, fhdx_rk3_step_ref).  Arithmetic follows the reference
 // operation by operation (see physics.hpp for why that is required).
 #include "kernels.hpp"

@@ -2,12 +2,11 @@
 //
 // Momentum and velocity live on faces (cumom[d], vel[d], nodal in d); density, energy and the
 // species densities in cells.  One stage of RK3stepStag (timeStepStag.cpp:13-1245) is
-//   transport (ref_kernels.hip) -> k_stag_cells (cells grown by 1: diagonal stresses and the
-//   cell-centred momentum fluxes) -> k_stag_edges (the three edge types: off-diagonal stresses
-//   and edge momentum fluxes) -> k_stag_faces<D> (mass, energy, species and the viscous-work,
-//   heat and Dufour components of faceflux) -> k_stag_update (cells and the three face
-//   momenta) -> ghost fill of the density -> k_stag_c2p -> ghost fill of state, momenta,
-//   velocities and prim,
+//   transport (ref_kernels.hip, stage 0 only) -> k_stag_stress (cells grown by 1: diagonal stresses
+//   and cell-centred momentum fluxes; the three edge types: off-diagonal stresses and edge momentum
+//   fluxes; one launch) -> k_stag_faces (mass, energy, species and the viscous-work, heat and Dufour
+//   components of faceflux; the three directions in one launch) -> k_stag_update (cells and the
+//   three face momenta) -> k_stag_c2p -> ghost fill of state, momenta, velocities and prim,
 // one thread per cell, edge or face.  The noise of a stage (A + w B of the step's two sets) is
 // evaluated in place from a counter-based Philox keyed by the wrapped global index, so duplicate
 // periodic faces and edges draw one value (OverrideSync's result) and nothing is stored.  Every

@@ -303,7 +303,8 @@ int fhdx_fill_chem_noise(fhdx_ctx* ctx, uint64_t seed, uint64_t step, uint32_t i
 /* ---- launch-shape tuning ---------------------------------------------------------------- */
 
 /* Launch shape of the fast path: tile width in x (16, 32 or 64 cells; the tile has 256 cells),
- * tiles per region of the region-major block order, how many z levels a tile block marches
+ * rows of tiles per region (a region spans the whole width) of the region-major block order, how
+ * many z levels a tile block marches
  * through, whether the Philox noise is evaluated in place by every stage (1) or written once per
  * step to arrays (0; always so for more than five species), and an optional cap on resident face-kernel blocks per CU (fewer blocks
  * in flight keep more of their neighbours' data in L2). */
