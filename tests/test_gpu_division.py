@@ -4,6 +4,7 @@ conservedToPrimitive divides five values of a cell by its density, and mass frac
 molar masses, so its results against numpy's IEEE division show the helper bit for bit: quotients that
 lie as close to a rounding boundary as 53-bit operands allow, ordinary ones over 2^+-300, zeros of both
 signs, infinities, NaN and zero divisors.  No tolerance: the values are equal or the test fails.
+Likewise the noise whose Box-Muller radius is zero, against the oracle's.
 """
 import numpy as np
 import pytest
@@ -72,3 +73,31 @@ def test_quotients_are_ieee(kind):
     np.testing.assert_array_equal(got[8:10], X)
     zero = np.concatenate([vel, Y]) == 0.0
     assert np.array_equal(np.signbit(got[[1, 2, 3, 6, 7]])[zero], np.signbit(np.concatenate([vel, Y]))[zero])
+
+
+# Counters whose Philox block has its first 53 bits all ones, solved for by running the rounds backwards:
+# u1 then rounds to 1, its logarithm is +0 and the radius the root of -0.  (step, instance, direction,
+# component, cell) at seed 9 in argon 16^3.
+ZERO_RADIUS = [(0x91696f0562fab3, 0xd3e6bb24, 2, 4, (4, 15, 10)), (0xc71df094702bd4, 0x240e31da, 1, 2, (15, 9, 0))]
+
+
+@pytest.mark.parametrize("step,instance,d,comp,cell", ZERO_RADIUS)
+def test_noise_of_a_zero_radius(orc, step, instance, d, comp, cell):
+    """The one zero a Box-Muller radius can be, -0: both values are the oracle's zeros, signs included."""
+    from fhdex_amd import compressible as fc
+    from fhdex_amd import lib as L
+    p = P.argon_gas(16).params
+    print(f"case zero radius, face direction {d}", flush=True)
+    st = orc.HostState(p)
+    orc.fill_noise(p, st, 9, step, instance)
+    i, j, k = cell
+    assert st.sA[d][comp, k, j, i] == 0.0 and st.sB[d][comp, k, j, i] == 0.0
+    ctx = L.Context(p)
+    nz = fc.NoiseSets(p)
+    fc.fill_noise(ctx, nz, 9, step, instance)
+    got = [(nz.A[q].t.cpu().numpy(), nz.B[q].t.cpu().numpy()) for q in range(3)]
+    ctx.close()
+    for q in range(3):
+        for dev, host in zip(got[q], (st.sA[q], st.sB[q])):
+            np.testing.assert_array_equal(dev, host)
+            assert np.array_equal(np.signbit(dev), np.signbit(host))
