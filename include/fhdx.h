@@ -322,8 +322,8 @@ typedef struct fhdx_tune {
 /* Times candidate launch shapes on trial_steps fast-path steps of a scratch copy of cu (cu is
  * not modified; HIP events on `stream`): one coordinate at a time (tile width, region height,
  * z levels, noise, face blocks per CU, records in update), each swept with the others at
- * their best so far.  Keeps the
- * fastest for this context and returns it in *best; trials (may be NULL) receives up to max_trials timed candidates, n_trials their
+ * their best so far, from the shape that an untuned context of this box runs (the first trial).
+ * Keeps the fastest for this context and returns it in *best; trials (may be NULL) receives up to max_trials timed candidates, n_trials their
  * count.  The choice is cached per (species count, box shape) for the process, so later
  * contexts of the same shape reuse it without timing (then n_trials = 0). */
 int fhdx_ctx_autotune(fhdx_ctx* ctx, fhdx_fab cu, double dt, int trial_steps, fhdx_tune* best,

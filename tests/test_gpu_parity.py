@@ -357,3 +357,27 @@ def test_launch_shapes_give_identical_bits(dev, orc, name, mk):
     assert np.array_equal(host(cu), st.cu)
     assert len(trials) >= 2 and best.ms_per_step == min(t.ms_per_step for t in trials)
     ctx.check()
+
+
+@pytest.mark.parametrize("name,mk", [("argon", lambda: P.argon_gas(0, shape=(24, 16, 12))),
+                                     ("species4", lambda: P.species_prefix(4, 0, 1, shape=(16, 12, 10))),
+                                     ("species8", lambda: P.species_prefix(8, 0, 1, shape=(16, 8, 8)))])
+def test_tuner_starts_from_the_untuned_shape(dev, orc, name, mk):
+    """The first shape the tuner times is the one an untuned context of the same box runs, so tuning
+    never settles on a shape that timed slower than not tuning."""
+    torch, fc, L = dev
+    cfg = mk()
+    p = cfg.params
+    say(f"case tuner's first shape, {name} {tuple(p.n_cells)}")
+    st = perturbed_state(p, cfg, orc, seed=22, amp=0.01, vel=500.0)
+    untuned = L.Context(p).get_tune().as_dict()
+    ctx = L.Context(p)
+    ctx.set_tune(16, 2, 1, 1, 0, 1 - untuned["records_in_update"])  # whatever the context holds just then
+    cu = to_dev(torch, fc, st.cu, (-p.ngc,) * 3)
+    best, trials = ctx.autotune(cu.fab, cfg.dt, trial_steps=1)
+    first = trials[0].as_dict()
+    assert {q: v for q, v in first.items() if q != "ms_per_step"} == \
+        {q: v for q, v in untuned.items() if q != "ms_per_step"}
+    assert best.ms_per_step <= trials[0].ms_per_step
+    assert ctx.get_tune().region_tiles == best.region_tiles
+    ctx.check()
