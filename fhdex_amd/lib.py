@@ -187,6 +187,7 @@ class Context:
         h = C.c_void_p()
         check(lib().fhdx_ctx_create(C.byref(p), C.byref(h)), "fhdx_ctx_create")
         self.h = h
+        self._untuned = self.get_tune()
 
     def close(self):
         if self.h:
@@ -212,10 +213,16 @@ class Context:
                                       C.byref(n), stream), "fhdx_ctx_autotune")
         return t, [trials[q] for q in range(n.value)]
 
-    def set_tune(self, tile_width: int, region_tiles: int = 1, z_levels: int = 1, noise_inline: int = 1,
-                 face_blocks_per_cu: int = 0, records_in_update: int = 0):
-        t = Tune(tile_width, region_tiles, z_levels, noise_inline, face_blocks_per_cu,
-                 records_in_update, 0.0)
+    def set_tune(self, tile_width: int | None = None, region_tiles: int | None = None, z_levels: int | None = None,
+                 noise_inline: int | None = None, face_blocks_per_cu: int | None = None,
+                 records_in_update: int | None = None):
+        """Set the launch shape (fhdx_ctx_set_tune); what is not given is as in an untuned context of the box."""
+        u = self._untuned
+        fields = [default if v is None else int(v) for v, default in
+                  ((tile_width, u.tile_width), (region_tiles, u.region_tiles), (z_levels, u.z_levels),
+                   (noise_inline, u.noise_inline), (face_blocks_per_cu, u.face_blocks_per_cu),
+                   (records_in_update, u.records_in_update))]
+        t = Tune(*fields, 0.0)
         check(lib().fhdx_ctx_set_tune(self.h, C.byref(t)), "fhdx_ctx_set_tune")
 
     def set_chemistry(self, chem: Chemistry):

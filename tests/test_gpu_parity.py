@@ -381,3 +381,17 @@ def test_tuner_starts_from_the_untuned_shape(dev, orc, name, mk):
     assert best.ms_per_step <= trials[0].ms_per_step
     assert ctx.get_tune().region_tiles == best.region_tiles
     ctx.check()
+
+
+def test_set_tune_leaves_the_rest_untuned(dev):
+    """What a caller of set_tune does not give is as in an untuned context, whatever was set before."""
+    torch, fc, L = dev
+    say("case set_tune defaults")
+    for p in (P.argon_gas(16).params, P.species_prefix(8, 12, 1).params):
+        ctx = L.Context(p)
+        untuned = ctx.get_tune().as_dict()
+        ctx.set_tune(32, 7, 2, 0, 2, 1 - untuned["records_in_update"])
+        ctx.set_tune(16)
+        assert ctx.get_tune().as_dict() == {**untuned, "tile_width": 16}
+        ctx.set_tune(records_in_update=1 - untuned["records_in_update"])
+        assert ctx.get_tune().as_dict() == {**untuned, "records_in_update": 1 - untuned["records_in_update"]}
