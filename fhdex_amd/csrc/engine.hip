@@ -389,8 +389,8 @@ static void enqueue_group(Engine* e, int g, const double ws[3])
     const Inst* I = e->d_inst;
     const WorkItem* Wc = e->d_cells[g];
     // ghost images come with every store (store_cell): no fill launches inside the step
-    // the records come with the update of the stage before where that pays for an ensemble's boxes
-    constexpr bool rec = NS <= 4;  // records_in_update's line for boxes of ensemble size
+    // the records come with the update of the stage before where that pays (see records_in_update)
+    constexpr bool rec = NS <= kEngineRecordsMaxNS;
     for (int st = 0; st < 3; ++st) {
         if (st == 0 || !rec) kb_cells<NS><<<nc, EB, 0, s>>>(I, Wc, st);
         kb_nodes<<<nc, EB, 0, s>>>(I, Wc, ws[st]);

@@ -78,15 +78,24 @@ struct FusedWorkspace {
 
 void fused_free(FusedWorkspace& w);
 
-// Whether a context's step starts with the next stage's records written by the update kernel: it saves
-// two launches and a read of the state a step, and costs the update kernel the transport's registers, so
-// it pays while launches and latency count or the transport is light.  ms a step, apart / in the update:
-// two species 32^3 .151/.138, 64^3 .361/.351, 128^3 2.62/2.48, 192^3 8.38/8.24, 256^3 19.57/19.84; four
-// species 32^3 .200/.182, 64^3 .605/.560, 128^3 4.11/4.06, 160^3 8.55/8.77; eight species 24^3 .390/.400,
-// 48^3 1.02/1.28, 64^3 2.02/2.24.
+// Whether a context's step has the next stage's records written by the update kernel: it saves two
+// launches and a read of the state a step, and costs the update kernel the transport's registers, so it
+// pays while launches and latency count or the transport is light.  ms a step, apart / in the update:
+//   two species    32^3 .112/.104, 64^3 .302/.290, 80^3 .726/.740, 97x61x45 .365/.363, 128^3 2.365/2.339,
+//                  192^3 7.94/7.87, 208^3 11.39/11.54, 256^3 18.87/19.19
+//   three          32^3 .132/.124, 64^3 .377/.371, 80^3 .918/.959, 100^3 1.80/1.83, 128^3 2.96/2.93
+//   four           32^3 .160/.149, 40^3 .246/.244, 44^3 .288/.293, 48^3 .294/.306, 64^3 .494/.512, 128^3 3.85/3.96
+//   five           24^3 .164/.151, 32^3 .201/.181, 48^3 .365/.401, 64^3 .628/.664, 128^3 4.64/5.16
+//   six            24^3 .237/.212, 32^3 .288/.263, 48^3 .593/.625, 64^3 1.238/1.233, 96^3 4.58/4.83
+//   seven          16^3 .242/.251, 24^3 .285/.281, 32^3 .341/.337, 48^3 .738/.892
+//   eight          16^3 .292/.326, 32^3 .404/.420, 48^3 .896/1.174, 64^3 1.83/2.06
+// The ensemble engine's boxes together fill the chip, so there the species count alone decides: a step of 48
+// uneven boxes, apart / in the update, for two to eight species 1.891/1.885, 2.36/2.33, 3.09/3.04,
+// 4.83/5.01, 6.53/6.61, 8.20/8.78, 10.07/11.43.
+constexpr int kEngineRecordsMaxNS = 4;
 inline bool records_in_update(int ns, long cells)
 {
-    return ns == 2 ? cells <= 8L << 20 : ns <= 4 && cells <= 3L << 20;
+    return cells <= (ns == 2 ? 8L << 20 : ns == 3 ? 256L << 10 : ns == 4 ? 64L << 10 : ns <= 6 ? 32L << 10 : 0L);
 }
 
 // Species counts above this evaluate the step's Philox noise into arrays (k_noise) before the
