@@ -102,7 +102,10 @@ inline bool records_in_update(int ns, long cells)
 // stages, whatever noise_inline says.  At NS = 8 the face kernel with the noise evaluated in
 // place (256 VGPRs + 236 AGPRs, no scratch) returned values that differ from the same kernel
 // reading the noise from arrays, and from the oracle; its cause was not found.  NS 6 and 7 take
-// the array kernels too, so one kernel family serves every wide mixture.
+// the array kernels too, so one kernel family serves every wide mixture.  The reference-shaped face
+// kernel (k_flux) is another body and draws its noise in place at every species count: its forms for
+// five to eight species, periodic and with walls, are held to the oracle's bits and to their own with the
+// noise from sets, by the tests of walls and ragged boxes.
 constexpr int kInlineNoiseMaxNS = 5;
 
 // The file-scope device scratch of fhdx_rk3_step_noalloc (noalloc.hip): its size, the lookup of

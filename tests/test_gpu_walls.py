@@ -3,8 +3,8 @@ calculateFlux (one-sided face branches, StochFlux, BCWallSpeciesFlux) with injec
 RK3 steps of the reference-shaped path with Philox noise, on the reference's wall decks
 (exec/compressible/inputs_regression_{slip_wall_adiabatic, noslip_reservoir_isothermal,
 temp_grad, RT_3d}, inputs_giantfluct_3d) at reduced and at full size, a bulk-viscosity
-variant, a box with walls in x only, one with x reservoirs and a periodic box one cell deep.  The GPU
-reads the wall-side cell for both sides of a wall face where the oracle spells out the doubled
+variant, a box with walls in x only, one with x reservoirs, a periodic box one cell deep, and walls
+around five to eight species.  The GPU reads the wall-side cell for both sides of a wall face where the oracle spells out the doubled
 terms; every comparison is exact.  The fused step refuses walls with FHDX_ERR_UNSUPPORTED.
 """
 import sys
@@ -43,6 +43,15 @@ def x_reservoirs():
     return P.Config("x_reservoirs", p, base.rho0, base.rhobar, base.T_init, base.dt, 1)
 
 
+def wide_walls(ns):
+    """Five to eight species (the face kernel's widest forms): no-slip isothermal walls in x, of fixed
+    composition below and closed above, slip adiabatic closed walls in y, periodic z."""
+    cfg = P.species_prefix(ns, 0, 1, shape=(9, 6, 7))
+    P.set_walls(cfg.params, [(2, 2), (1, 1), (-1, -1)], [(2, 2), (1, 1), (-1, -1)], [(2, 1), (1, 1), (-1, -1)],
+                t_lo=(310.0, 0.0, 0.0), t_hi=(295.0, 0.0, 0.0), bc_Yk=[1.0 / ns] * ns)
+    return cfg
+
+
 def one_cell_deep():
     """A periodic three-species box one cell deep in z (the quasi-2-D shape of
     exec/compressible/inputs_test_3d): ghosts are images two periods away."""
@@ -68,6 +77,10 @@ CASES = [
     ("visc_type_3", visc3_walls),
     ("x_walls", x_walls),
     ("x_reservoirs", x_reservoirs),
+    ("walls_species5", lambda: wide_walls(5)),
+    ("walls_species6", lambda: wide_walls(6)),
+    ("walls_species7", lambda: wide_walls(7)),
+    ("walls_species8", lambda: wide_walls(8)),
 ]
 
 
@@ -182,6 +195,36 @@ def test_rk3_steps_match_oracle(dev, orc, name, mk):
     say(f"  cu exact={np.array_equal(got_cu, st.cu)} prim exact={np.array_equal(got_prim, st.prim)}")
     assert np.array_equal(got_cu, st.cu)            # ghosts included: setBC after the last stage
     assert np.array_equal(got_prim, st.prim)
+
+
+@pytest.mark.parametrize("walls", [False, True])
+@pytest.mark.parametrize("ns", [5, 6, 7, 8])
+def test_noise_in_place_equals_noise_from_sets(dev, orc, ns, walls):
+    """Two steps of a box of many blocks with the noise drawn inside the face kernel and with the same noise
+    filled into sets first: the widest forms of the face kernel keep the bits either way."""
+    torch, fc, L = dev
+    cfg = P.species_prefix(ns, 0, 1, shape=(45, 24, 20))
+    p = cfg.params
+    if walls:
+        P.set_walls(p, [(2, 2), (1, 1), (-1, -1)], [(2, 2), (1, 1), (-1, -1)], [(2, 1), (1, 1), (-1, -1)],
+                    t_lo=(310.0, 0.0, 0.0), t_hi=(295.0, 0.0, 0.0), bc_Yk=[1.0 / ns] * ns)
+    say(f"case noise in place and from sets, {ns} species, walls {walls}")
+    st = perturbed_state(p, cfg, orc, seed=14, amp=0.02, vel=300.0)
+    ctx = L.Context(p)
+    outs = []
+    for in_place in (True, False):
+        ds = fc.DeviceState(p)
+        ds.cu.t.copy_(torch.from_numpy(st.cu))
+        ds.prim.t.copy_(torch.from_numpy(st.prim))
+        nz = None if in_place else fc.NoiseSets(p)
+        for step in range(2):
+            if nz is not None:
+                fc.fill_noise(ctx, nz, 23, step)
+            fc.RK3step(ctx, ds, cfg.dt, noise=nz, seed=23, step=step)
+        outs.append([ds.cu.t, ds.prim.t, ds.rancorn.t] + [f.t for f in ds.flux] + [f.t for f in ds.stochFlux])
+    ctx.check()
+    for a, b in zip(*outs):
+        assert bool(torch.isfinite(a).all()) and torch.equal(a, b)
 
 
 def test_set_bc_rejects_bad_shapes(dev):
