@@ -22,14 +22,22 @@ constexpr int MS = FHDX_MAX_SPECIES;
 // The compiler's FP64 division is 11 VALU instructions (two div_scale, rcp, four fma, a mul and a
 // fma of the quotient, div_fmas, div_fixup) with four wait states before div_fmas, and the step
 // divides several hundred times per cell, most often by a constant of the run (dx, a molar mass) or
-// several times by one value (rho, a mean pressure).  Rcp holds a divisor and its reciprocal to
-// the last bit, so each further quotient is 4 instructions: q = a r, the exact remainder
-// a - b q, q corrected by it, div_fixup (zero, infinite and NaN operands).  These are the
-// compiler's own steps with the two scalings left out, and with r correctly rounded the corrected
-// quotient is the IEEE one (Markstein, IBM J. Res. Dev. 34, 1990; Brisebarre, Muller and Raina,
-// IEEE Trans. Comput. 53, 2004), so the bits are those of a / b.  What the scalings are for:
-// divisors or quotients outside about 2^+-1000 and dividends below 2^-968, where the last bit may
-// differ.
+// several times by one value (rho, a mean pressure).  Rcp holds a divisor and its reciprocal, so each
+// further quotient is 4 instructions: q = a r, the remainder a - b q, q corrected by it, div_fixup
+// (zero, infinite and NaN operands).
+//
+// Which bits.  With r the rounded reciprocal (the constants', from the host) the corrected quotient is
+// the IEEE one (Markstein, IBM J. Res. Dev. 34, 1990; Brisebarre, Muller and Raina, IEEE Trans. Comput.
+// 53, 2004).  rcp_of's r is not always the rounded reciprocal: Newton's iteration misses it for
+// significands next to 2^53, 2^53 - 1 before all.  Its quotient then is wrong only where a / b lies
+// within 2^-50 of its last place of a rounding boundary, and then by one last place; of 6144 pairs sought
+// there three are.  rcp_of's quotients are the compiler's own steps without the scalings: its division
+// gave the same bits on every pair compared, those three among them.
+//
+// What the scalings are for: with a dividend below 2^-968 the last place may differ, and a divisor below
+// 2^-1024, whose reciprocal is infinite, gives an infinite quotient.  No other operands differ, to the
+// ends of the range.
+//
 // 256^3 argon: the face kernel 4.49 ms a launch with the compiler's divisions and roots, 3.92 ms with
 // these (its vector instructions 6545 and 5620).
 struct Rcp {
@@ -42,7 +50,8 @@ __device__ __forceinline__ double operator/(double a, const Rcp& d)
     return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d.b, q, a), d.r, q), d.b, a);
 }
 
-// The reciprocal by two Newton steps from v_rcp_f64, as the compiler's division refines it.
+// The reciprocal by two Newton steps from v_rcp_f64, as the compiler's division refines it (within one
+// last place of 1 / b).
 __device__ __forceinline__ Rcp rcp_of(double b)
 {
     double r = __builtin_amdgcn_rcp(b);
@@ -53,8 +62,9 @@ __device__ __forceinline__ Rcp rcp_of(double b)
 
 __device__ __forceinline__ double quot(double a, double b) { return a / rcp_of(b); }
 
-// sqrt of x = +-0 or x >= 2^-767 (infinity and NaN included): the compiler's refinement of
-// v_rsq_f64 without the scaling of smaller x, 13 instructions for 19.
+// sqrt of x = +-0 or x >= 2^-767 (infinity and NaN included): v_rsq_f64 refined by Goldschmidt's
+// coupled iteration of the root and half its reciprocal, then two corrections by the remainder x - s s; the
+// compiler's sqrt without its scaling of smaller x, 13 instructions for 19.
 __device__ __forceinline__ double root(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
@@ -948,7 +958,7 @@ __device__ __forceinline__ double flip_sign(double x, uint32_t w)
 }
 
 // sqrt of x = +-0 or of a normal x above 1e-290: the reciprocal root of |x|, +infinity at either zero, is
-// held at 1e300, and the refinement then returns x; one instruction where root() tests and selects.
+// held at 1e300, and root()'s refinement then returns x; one instruction where root() tests and selects.
 // (The reciprocal root of -0 itself is -infinity, which no minimum holds back, and -0 is the zero that a
 // Box-Muller radius can be: -2 times the logarithm of u1 = 1.  The magnitude is a source modifier of
 // v_rsq_f64 and costs nothing.)
