@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 
 BOXES = [(2, (65, 17, 4)), (2, (4, 5, 6)), (3, (15, 33, 7)), (4, (33, 70, 5)), (5, (5, 4, 67)), (6, (9, 5, 7)),
          (7, (6, 9, 5)), (8, (17, 6, 9))]
-STAG_BOXES = [(2, (65, 5, 4)), (4, (4, 33, 5)), (8, (17, 4, 6))]
+STAG_BOXES = [(2, (65, 5, 4)), (3, (9, 6, 4)), (4, (4, 33, 5)), (5, (6, 9, 4)), (6, (5, 7, 6)),
+              (7, (4, 6, 9)), (8, (17, 4, 6))]
 
 
 def config(ns, shape):
