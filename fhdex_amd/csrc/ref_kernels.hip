@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(BLK) k_set_bc(DevParams P, Arr prim, Arr cons,
 }
 
 // One face of setBC in registers: pr, co hold the mirror cell's values and become the ghost cell's.
-// For algorithm_type 2, where every component is written (k_set_bc leaves the species alone otherwise).
+// For algorithm_type 2, where every component is written (walls are refused otherwise).
 template <int NS>
 __device__ __forceinline__ void wall_ghost(const DevParams& P, int f, double* pr, double* co)
 {
@@ -1246,11 +1246,6 @@ int ref_set_bc(const DevParams& P, Arr prim, Arr cons, hipStream_t s)
 
 int ref_ghosts(const DevParams& P, Arr prim, Arr cons, hipStream_t s)
 {
-    if (P.any_wall && P.algorithm_type != 2) {  // setBC then leaves the species of a ghost cell alone
-        int r = ref_fill_boundary(P, cons, P.nvars, s);
-        if (!r) r = ref_fill_boundary(P, prim, P.nprim, s);
-        return r ? r : ref_set_bc(P, prim, cons, s);
-    }
     NS_DISPATCH(P.ns, (k_ghosts<NS><<<grid_for(ngrown(P) - ncell(P), BLK), BLK, 0, s>>>(P, prim, cons)));
     FHDX_HIP_TRY(hipGetLastError());
     return FHDX_OK;

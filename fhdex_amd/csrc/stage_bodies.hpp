@@ -760,16 +760,6 @@ __device__ inline void store_face(const DevParams& P, const Fld& Fo, const doubl
     }
 }
 
-template <int NS, int D, bool INL>
-__device__ inline void face_body(const DevParams& P, const Fld& Us, const Fld& R, const Fld& N, const Fld& A,
-                                 const Fld& B, const NoiseKey& K, const Fld& Fo, double w, double volinv, double dtinv,
-                                 double dt, int i, int j, int k, unsigned cb)
-{
-    double fo[NS + 5];
-    face_flux<NS, D, INL>(P, Us, R, N, A, B, K, w, volinv, dtinv, dt, i, j, k, cb, fo);
-    store_face<NS, D>(P, Fo, fo, i, j, k, cb);
-}
-
 // ---- stage combination (+ primitive variables after the last stage) -----------------------
 
 // What a stage update needs for the chemistry source: the stage's cell records (T, p, X of the
