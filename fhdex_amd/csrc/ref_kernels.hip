@@ -390,29 +390,13 @@ struct FaceView {
     unsigned c0, cm, lo, up, nd;
 };
 
-template <int NS, int D, bool WALL>
-__device__ __forceinline__ void stoch_part(const DevParams& P, const FaceView& V, const WallFace& W, const double* ran,
-                                           double* o, double volinv, double dtinv, double dt, int i, int j, int k)
+// The edge terms of the face, fac sqrt(mu) rancorn summed over its four edges.
+template <int D, bool WALL>
+__device__ __forceinline__ double edge_sum(const DevParams& P, const FaceView& V, bool wall, int i, int j, int k)
 {
-    const Fld &prim = V.prim, &eta = V.eta, &zeta = V.zeta, &kappa = V.kappa, &chi = V.chi, &Dm = V.Dm;
-    const unsigned lo = V.lo, up = V.up;
-    const bool wall = WALL && W.any();
+    const Fld &prim = V.prim, &eta = V.eta, &zeta = V.zeta;
+    const unsigned up = V.up;
     constexpr Rcp three{3., 1. / 3.};
-    const int nv = NS + 5;
-
-    double Tu = prim(up, 4), Tl = prim(lo, 4);
-    double mup = eta(up, 0) * Tu + eta(lo, 0) * Tl;
-    double kp = kappa(up, 0) * Tu * Tu + kappa(lo, 0) * Tl * Tl;
-    double meanT = 0.5 * (Tu + Tl);
-    double w[NS + 5];
-    double fw1 = root(P.k_B * mup * volinv * dtinv);
-    double fw4 = root(P.k_B * kp * volinv * dtinv);
-    w[1] = fw1 * ran[1];
-    w[2] = fw1 * ran[2];
-    w[3] = fw1 * ran[3];
-    w[4] = fw4 * ran[4];
-    double nweight = root(P.k_B * volinv * dtinv);
-
     // tangential-wall factors of the four edges (pp, mp, pm, mm) over transverse axes (A, B)
     constexpr int TA = (D == 0) ? 1 : 0, TB = (D == 2) ? 1 : 2;
     double fac[4] = {1., 1., 1., 1.};
@@ -476,7 +460,41 @@ __device__ __forceinline__ void stoch_part(const DevParams& P, const FaceView& V
         double term = fac[c] * root(mu) * V.rancorn(V.nd, 0, nd[0], nd[1], nd[2]);
         sum = (c == 0) ? term : sum + term;
     }
-    w[1 + D] = w[1 + D] + 0.25 * nweight * sum;
+    return sum;
+}
+
+// Seven and eight species with walls: the edges, whose two forms are a divergent branch, before the noise and
+// all else that is held in registers through them.  With them here at eight (256 VGPRs, 242 AGPRs) the
+// compiler put copies of two noise values at the head of the block behind the branch, before the execution
+// mask is whole again, and the lanes that had gone the other way lost them.  Fewer species have no such copies.
+// 48^3 with walls, us a step here / first: four species 384/406, five 649/673, six 741/751, seven 1044/924.
+template <int NS, bool WALL>
+constexpr bool kEdgesFirst = WALL && NS > 6;
+
+template <int NS, int D, bool WALL>
+__device__ __forceinline__ void stoch_part(const DevParams& P, const FaceView& V, bool wall, double edges,
+                                           const double* ran, double* o, double volinv, double dtinv, double dt,
+                                           int i, int j, int k)
+{
+    const Fld &prim = V.prim, &eta = V.eta, &kappa = V.kappa, &chi = V.chi, &Dm = V.Dm;
+    const unsigned lo = V.lo, up = V.up;
+    const int nv = NS + 5;
+
+    double Tu = prim(up, 4), Tl = prim(lo, 4);
+    double mup = eta(up, 0) * Tu + eta(lo, 0) * Tl;
+    double kp = kappa(up, 0) * Tu * Tu + kappa(lo, 0) * Tl * Tl;
+    double meanT = 0.5 * (Tu + Tl);
+    double w[NS + 5];
+    double fw1 = root(P.k_B * mup * volinv * dtinv);
+    double fw4 = root(P.k_B * kp * volinv * dtinv);
+    w[1] = fw1 * ran[1];
+    w[2] = fw1 * ran[2];
+    w[3] = fw1 * ran[3];
+    w[4] = fw4 * ran[4];
+    double nweight = root(P.k_B * volinv * dtinv);
+
+    if (!kEdgesFirst<NS, WALL>) edges = edge_sum<D, WALL>(P, V, wall, i, j, k);
+    w[1 + D] = w[1 + D] + 0.25 * nweight * edges;
 
     // this face's flux after the stochastic pass: the reference adds to a zeroed array
     // (flux.cpp:24-26), so each term is 0.0 + term
@@ -1107,28 +1125,6 @@ __device__ __forceinline__ void flux_body(const DevParams& P, const FluxArgs& F,
 {
     int i, j, k;
     if (!box_index(P, t, D == 0, D == 1, D == 2, i, j, k)) return;
-    double ran[NS + 5], o[NS + 9];
-    ran[0] = 0.0;
-    const unsigned fo = off_of(F.flux[D], i, j, k);
-    const Fld flux = fld_of(F.flux[D], F.flux[D]), rn = fld_of(F.ran[D], F.flux[D]);
-    if (F.noise.mode == kNoisePhilox) {
-#pragma unroll
-        for (int c = 1; c < NS + 5; ++c) {
-            double A, B;
-            face_noise<D>(P, F.noise.K, c, i, j, k, A, B);
-            ran[c] = 1.0 * A + F.noise.w * B;
-        }
-    } else if (F.noise.mode == kNoiseSets) {
-        const Fld A = fld_of(F.noise.A[D], F.flux[D]), B = fld_of(F.noise.B[D], F.flux[D]);
-#pragma unroll
-        for (int c = 1; c < NS + 5; ++c) ran[c] = 1.0 * A(fo, c) + F.noise.w * B(fo, c);
-    } else {
-#pragma unroll
-        for (int c = 1; c < NS + 5; ++c) ran[c] = rn(fo, c);
-    }
-    if (F.noise.mode != kNoiseWeighted && F.keep)
-#pragma unroll
-        for (int c = 0; c < NS + 5; ++c) rn(fo, c) = ran[c];
     const WallFace W = WALL ? wall_face<D>(P, i, j, k) : WallFace{false, false, 0, 0, 0};
     const Arr& cell = F.prim;
     FaceView V;
@@ -1151,9 +1147,33 @@ __device__ __forceinline__ void flux_body(const DevParams& P, const FluxArgs& F,
     V.up = V.c0;
     if (WALL && W.any()) V.lo = V.up = off_of(cell, W.wi, W.wj, W.wk);
     V.nd = off_of(F.rancorn, i, j, k);
+    double edges = 0.;
+    if (kEdgesFirst<NS, WALL> && P.stoch_on) edges = edge_sum<D, WALL>(P, V, W.any(), i, j, k);
+    double ran[NS + 5], o[NS + 9];
+    ran[0] = 0.0;
+    const unsigned fo = off_of(F.flux[D], i, j, k);
+    const Fld flux = fld_of(F.flux[D], F.flux[D]), rn = fld_of(F.ran[D], F.flux[D]);
+    if (F.noise.mode == kNoisePhilox) {
+#pragma unroll
+        for (int c = 1; c < NS + 5; ++c) {
+            double A, B;
+            face_noise<D>(P, F.noise.K, c, i, j, k, A, B);
+            ran[c] = 1.0 * A + F.noise.w * B;
+        }
+    } else if (F.noise.mode == kNoiseSets) {
+        const Fld A = fld_of(F.noise.A[D], F.flux[D]), B = fld_of(F.noise.B[D], F.flux[D]);
+#pragma unroll
+        for (int c = 1; c < NS + 5; ++c) ran[c] = 1.0 * A(fo, c) + F.noise.w * B(fo, c);
+    } else {
+#pragma unroll
+        for (int c = 1; c < NS + 5; ++c) ran[c] = rn(fo, c);
+    }
+    if (F.noise.mode != kNoiseWeighted && F.keep)
+#pragma unroll
+        for (int c = 0; c < NS + 5; ++c) rn(fo, c) = ran[c];
 #pragma unroll
     for (int c = 0; c < NS + 9; ++c) o[c] = 0.0;
-    if (P.stoch_on) stoch_part<NS, D, WALL>(P, V, W, ran, o, volinv, dtinv, F.dt, i, j, k);
+    if (P.stoch_on) stoch_part<NS, D, WALL>(P, V, WALL && W.any(), edges, ran, o, volinv, dtinv, F.dt, i, j, k);
     diff_part<NS, D, WALL>(P, V, W, o);
     corner_part<NS, D>(V, o);
     if (P.advection_type == 1 || P.advection_type == 2) hyp_part<NS, D, WALL>(P, V, W, o, i, j, k);
@@ -1164,14 +1184,39 @@ __device__ __forceinline__ void flux_body(const DevParams& P, const FluxArgs& F,
         for (int c = NS + 5; c < NS + 9; ++c) flux(fo, c) = o[c];
 }
 
+// The arguments are one struct, read anew in each direction's branch, as k_faces does.  Taken as they
+// come, the compiler loads those of all three branches at once (147 to 269 scalar registers spilled to vector
+// lanes, 6 to 88 so), and at five and more species with walls it copied the parameters, 1960 bytes a lane, to
+// scratch: 48^3 with walls, five species 994 us a step, 649 so (796 in four passes); eight 1888 and 1258 (1810).
+struct FluxKernel {
+    DevParams P;
+    FluxArgs F;
+    double volinv, dtinv;
+};
+
+__device__ __forceinline__ const FluxKernel& flux_args()
+{
+    typedef const FluxKernel __attribute__((address_space(4))) * Ptr;
+    Ptr p = (Ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm("" : "+s"(p));
+    return *(const FluxKernel*)p;
+}
+
+template <int NS, int D, bool WALL>
+__device__ __forceinline__ void flux_item(long t)
+{
+    const FluxKernel& A = flux_args();
+    flux_body<NS, D, WALL>(A.P, A.F, A.volinv, A.dtinv, t);
+}
+
 template <int NS, bool WALL>
-__global__ void __launch_bounds__(BLK) k_flux(DevParams P, FluxArgs F, double volinv, double dtinv)
+__global__ void __launch_bounds__(BLK) k_flux(FluxKernel A)
 {
     const unsigned item = xcd_block(blockIdx.x, gridDim.x), chunk = item / 3, d = item - 3 * chunk;
     const long t = (long)chunk * BLK + threadIdx.x;
-    if (d == 0) flux_body<NS, 0, WALL>(P, F, volinv, dtinv, t);
-    else if (d == 1) flux_body<NS, 1, WALL>(P, F, volinv, dtinv, t);
-    else flux_body<NS, 2, WALL>(P, F, volinv, dtinv, t);
+    if (d == 0) flux_item<NS, 0, WALL>(t);
+    else if (d == 1) flux_item<NS, 1, WALL>(t);
+    else flux_item<NS, 2, WALL>(t);
 }
 
 // ---- host launchers ---------------------------------------------------------------------
@@ -1271,8 +1316,8 @@ static void flux_passes(const DevParams& P, const FluxArgs& a, hipStream_t s)
     long mf = nface(P, 0);
     for (int d = 1; d < 3; ++d) mf = nface(P, d) > mf ? nface(P, d) : mf;
     const unsigned grid = 3 * grid_for(mf, BLK);  // every body checks its own direction's face count
-    if (P.any_wall) k_flux<NS, true><<<grid, BLK, 0, s>>>(P, a, volinv, dtinv);
-    else k_flux<NS, false><<<grid, BLK, 0, s>>>(P, a, volinv, dtinv);
+    if (P.any_wall) k_flux<NS, true><<<grid, BLK, 0, s>>>(FluxKernel{P, a, volinv, dtinv});
+    else k_flux<NS, false><<<grid, BLK, 0, s>>>(FluxKernel{P, a, volinv, dtinv});
 }
 
 int ref_calculate_flux(const DevParams& P, const FluxArgs& a, int flux_ncomp[3], hipStream_t s)
