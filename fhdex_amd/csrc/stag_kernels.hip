@@ -457,14 +457,42 @@ __device__ __forceinline__ void stag_face(const DevParams& P, const StagArrays& 
 // zero momentum ones and the four parts of the energy flux) are not stored; the last stage of a
 // step, and calculateFluxStag, store all.  Argon 160^3: 1096 us a stage in three launches with index
 // products of each array's strides, 940 us with the directions one after another, 818 us so.
+//
+// The arguments are one struct, read anew in each direction's branch (see k_flux): 140 to 271 scalar
+// registers spilled to vector lanes, 2 to 16 so, and six species fit two waves a SIMD.  A step of 48^3, us:
+// seven species 984 and 838 (908 with a launch a direction), eight 1300 and 1083 (1315), two 237 and 222; argon
+// 160^3 5477 and 5385.
+struct StagFaceKernel {
+    DevParams P;
+    StagArrays A;
+    NoiseKey K;
+    double w, dt;
+    int keep;
+};
+
+__device__ __forceinline__ const StagFaceKernel& stag_face_args()
+{
+    typedef const StagFaceKernel __attribute__((address_space(4))) * Ptr;
+    Ptr p = (Ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm("" : "+s"(p));
+    return *(const StagFaceKernel*)p;
+}
+
+template <int NS, int D>
+__device__ __forceinline__ void stag_face_item(long t)
+{
+    const StagFaceKernel& F = stag_face_args();
+    stag_face<NS, D>(F.P, F.A, F.K, F.w, F.dt, F.keep, t);
+}
+
 template <int NS>
-__global__ void __launch_bounds__(SB) k_stag_faces(DevParams P, StagArrays A, NoiseKey K, double w, double dt, int keep)
+__global__ void __launch_bounds__(SB) k_stag_faces(StagFaceKernel F)
 {
     const unsigned item = xcd_block(blockIdx.x, gridDim.x), chunk = item / 3, d = item - 3 * chunk;
     const long t = (long)chunk * SB + threadIdx.x;
-    if (d == 0) stag_face<NS, 0>(P, A, K, w, dt, keep, t);
-    else if (d == 1) stag_face<NS, 1>(P, A, K, w, dt, keep, t);
-    else stag_face<NS, 2>(P, A, K, w, dt, keep, t);
+    if (d == 0) stag_face_item<NS, 0>(t);
+    else if (d == 1) stag_face_item<NS, 1>(t);
+    else stag_face_item<NS, 2>(t);
 }
 
 // ---- stage update: timeStepStag.cpp:470-538, 771-857, 1106-1199 --------------------------
@@ -806,7 +834,8 @@ int stag_flux(const DevParams& P, const StagArrays& A, const NoiseKey& K, double
     k_stag_stress<<<dim3(grid_for(ngrown1, SB), 4), SB, 0, s>>>(P, A, K, w, dt);
     long nf = 0;
     for (int d = 0; d < 3; ++d) nf = std::max(nf, (long)(P.n[0] + (d == 0)) * (P.n[1] + (d == 1)) * (P.n[2] + (d == 2)));
-    STAG_NS_DISPATCH(P.ns, (k_stag_faces<NS><<<3 * grid_for(nf, SB), SB, 0, s>>>(P, A, K, w, dt, keep ? 1 : 0)));
+    STAG_NS_DISPATCH(P.ns, (k_stag_faces<NS><<<3 * grid_for(nf, SB), SB, 0, s>>>(
+                                  StagFaceKernel{P, A, K, w, dt, keep ? 1 : 0})));
     FHDX_HIP_TRY(hipGetLastError());
     return FHDX_OK;
 }
