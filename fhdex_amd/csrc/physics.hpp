@@ -329,11 +329,16 @@ __device__ inline void hcb_binary(const DevParams& P, double density, double tem
 }
 
 // D_GIO1 (compressible_functions.H:647-778; D_GIO at :513-646 is the same arithmetic): the
-// three-term series of the multicomponent diffusion matrix, D[j*NS+i] = Diff_ij Ykp_i.
-template <int NS>
-__device__ __forceinline__ void d_gio_series(const Rcp (&Dbin)[NS][NS], const double* Ykp, const double* Xkp,
+// three-term series of the multicomponent diffusion matrix, D[j*NS+i] = Diff_ij Ykp_i.  Dbin: the binary
+// coefficients as kept divisors where they stay in registers, or plain (Valk-Waldmann, whose matrices live
+// in scratch: with kept divisors they took twice the room, eight species 48^3 7430 us a reference-shaped step,
+// 6780 so, 7040 before the series went by columns).
+template <int NS, typename Div>
+__device__ __forceinline__ void d_gio_series(const Div (&Dbin)[NS][NS], const double* Ykp, const double* Xkp,
                                              double* D)
 {
+    // columns one after the other where the inputs are in registers; the Valk-Waldmann solves' are in scratch
+    constexpr bool apart = NS > 4 && sizeof(Div) == sizeof(Rcp);
     double Di[NS], Minv[NS], Mmat[NS], PJ[NS][NS];
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
@@ -376,7 +381,7 @@ __device__ __forceinline__ void d_gio_series(const Rcp (&Dbin)[NS][NS], const do
             for (int k = 0; k < NS; ++k) s = s + Pm(i, k) * J[k];
             PJ[i][j] = s;
         }
-        if (NS > 4) __builtin_amdgcn_sched_barrier(0);
+        if (apart) __builtin_amdgcn_sched_barrier(0);
     }
     // Diff <- PJ Diff + P Minv P^T, three times: the columns are independent, so one column's
     // start, iterate and result are all that is live beside PJ (the whole matrices are 5 NS^2
@@ -408,7 +413,7 @@ __device__ __forceinline__ void d_gio_series(const Rcp (&Dbin)[NS][NS], const do
         }
 #pragma unroll
         for (int i = 0; i < NS; ++i) D[j * NS + i] = col[i] * Ykp[i];
-        if (NS > 4) __builtin_amdgcn_sched_barrier(0);
+        if (apart) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -632,8 +637,7 @@ __device__ inline int vw_transport(const DevParams& P, double density, double T,
 {
     const double kB = P.k_B, pi = 3.1415926535897932;
     double mk[NS], xx[NS], yy[NS];
-    double Dflat[NS * NS], om[NS * NS], a1[NS * NS], a2[NS * NS], ab[NS * NS];
-    Rcp Dbin[NS][NS];
+    double Dflat[NS * NS], om[NS * NS], a1[NS * NS], a2[NS * NS], ab[NS * NS], Dbin[NS][NS];
     for (int n = 0; n < NS; ++n) mk[n] = P.molmass[n] * (kB / P.Runiv);
     for (int ii = 0; ii < NS; ++ii) {
         double sumXk = 0.;
@@ -657,7 +661,7 @@ __device__ inline int vw_transport(const DevParams& P, double density, double T,
             ab[i * NS + j] = 8.0 / (3.0 * kB) * mu * mu * (-.5 * s11bar);
             Dflat[i * NS + j] = 3.0 / 16.0 * sqrt(2.0 * pi * vw_cube(kB) * (mi + mj) / mi / mj) /
                                 (pi * vw_sq(diamat)) * T * sqrtT / pressure;
-            Dbin[i][j] = rcp_of(Dflat[i * NS + j]);
+            Dbin[i][j] = Dflat[i * NS + j];
             om[i * NS + j] = sqrt(pi * kB / (2.0 * mu)) * vw_sq(diamat) * sqrtT;
             a1[i * NS + j] = (5.0 / (kB) * mi * mj / (mi + mj) * Fij * s11bar) / sqrtT;
             a2[i * NS + j] = (5.0 / (kB) * mi * mj * mi * mj / (vw_cube(mi + mj)) * Fijstar * s11bar) / sqrtT;
