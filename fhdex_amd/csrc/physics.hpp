@@ -961,14 +961,14 @@ __device__ __forceinline__ double flip_sign(double x, uint32_t w)
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | (uint32_t)b));
 }
 
-// sqrt of x = +-0 or of a normal x above 1e-290: the reciprocal root of |x|, +infinity at either zero, is
-// held at 1e300, and root()'s refinement then returns x; one instruction where root() tests and selects.
-// (The reciprocal root of -0 itself is -infinity, which no minimum holds back, and -0 is the zero that a
-// Box-Muller radius can be: -2 times the logarithm of u1 = 1.  The magnitude is a source modifier of
-// v_rsq_f64 and costs nothing.)
+// sqrt of x = +-0 or of a normal x above 1e-290: the magnitude of v_rsq_f64, infinite at either zero, is held
+// at 1e300, and root()'s refinement then returns x; one instruction where root() tests and selects.
+// (v_rsq_f64 of -0 is -infinity, which no minimum holds back, and -0 is the zero that a Box-Muller radius can
+// be: -2 times the logarithm of u1 = 1.  The magnitude is a source modifier of the minimum and costs
+// nothing.)
 __device__ __forceinline__ double root_small(double x)
 {
-    const double y = __builtin_fmin(__builtin_amdgcn_rsq(__builtin_fabs(x)), 1e300);
+    const double y = __builtin_fmin(__builtin_fabs(__builtin_amdgcn_rsq(x)), 1e300);
     double s = x * y, h = y * 0.5;
     const double e = __builtin_fma(-h, s, 0.5);
     s = __builtin_fma(s, e, s);
