@@ -151,7 +151,8 @@ static TileMap make_tiles(int n0, int n1, int n2, int rh, int tw_max, int kz)
     rh = rh < 1 ? 1 : rh;
     m.ntx = (n0 + tx - 1) / tx;
     m.nry = (nty + rh - 1) / rh;
-    m.rh = (nty + m.nry - 1) / m.nry;  // regions of equal height: no empty tiles where rh does not divide nty
+    // regions of equal height: at most nry - 1 rows of tiles lie past the box, where rh does not divide nty
+    m.rh = (nty + m.nry - 1) / m.nry;
     m.n2 = n2;
     return m;
 }
@@ -178,7 +179,7 @@ __global__ void __launch_bounds__(FB) k_nodes(DevParams P, TileMap tm, Grid G, d
     TILE_LEVELS(tm, xcd_block(blockIdx.x, gridDim.x), node_body<INL>(P, G.fld(R), G.fld(N), G.fld(rA), G.fld(rB), K, w, i, j, k, G.off(i, j, k));)
 }
 
-// ---- K3: the three lower faces of each cell (flux.cpp:71-2372) -------------------------------
+// ---- K3: a lower face of each cell, one direction a block (flux.cpp:71-2372) --------------------
 
 struct FaceArgs {
     double *Us, *R, *N;
