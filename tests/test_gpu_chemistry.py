@@ -136,3 +136,60 @@ def test_chemistry_rejections(dev, orc):
         ens.add(p, cfg.dt, 1, st.cu)
     assert e.value.status == 2
     ens.close()
+
+
+def wide_chemistry(ns, shape):
+    """A two-reaction mixture of ns species (forward and back between the first pair and the last species),
+    with temperature-dependent rates that move the partial densities by up to 1 % in two steps."""
+    cfg = P.species_prefix(ns, 0, 1, shape=shape)
+    cfg.params.nreaction = 2
+    pair, last = [1, 1] + [0] * (ns - 2), [0] * (ns - 1) + [1]
+    if ns == 2:
+        pair = [2, 0]
+    cfg.chem = P.make_chemistry([pair, last], [last, pair], [1.3e13, 3.0e7], 300.0, reaction_type=1,
+                                alpha=[1.0e10, -2.0e10], beta=[0.5, -1.1])
+    return cfg
+
+
+@pytest.mark.parametrize("ns,shape", [(2, (7, 5, 6)), (3, (9, 5, 4)), (4, (6, 7, 5)), (5, (5, 6, 7)), (6, (8, 4, 5)),
+                                      (7, (5, 8, 4)), (8, (6, 5, 7))])
+def test_reacting_steps_at_every_species_count(dev, orc, ns, shape):
+    """Two steps of the fused path (records from either kernel), of the reference-shaped and of the
+    staggered step: each is an instantiation a species count, and each equals the oracle bit for bit."""
+    from fhdex_amd import stag as S
+    from tests.helpers import perturbed_stag_state
+    torch, fc, L = dev
+    cfg = wide_chemistry(ns, shape)
+    p = cfg.params
+    g = p.ngc
+    say(f"case reacting steps, {ns} species {shape}")
+    st = perturbed_state(p, cfg, orc, seed=15, amp=0.02, vel=300.0)
+    start, start_prim = (torch.from_numpy(a.copy()).cuda() for a in (st.cu, st.prim))
+    assert orc.advance_chem(p, cfg.chem, st.cu, st.prim, 2, cfg.dt, seed=6, step0=0) == 0
+    ctx = L.Context(p)
+    ctx.set_chemistry(cfg.chem)
+    for rec in (0, 1):
+        ctx.set_tune(records_in_update=rec)
+        cu, prim = fc.MultiFab(start.clone(), (-g,) * 3), fc.MultiFab.cell(p, p.nprimvars)
+        for step in range(2):
+            fc.rk3_step(ctx, cu, prim, cfg.dt, 6, step)
+        assert np.array_equal(valid(p, cu.t.cpu().numpy()), valid(p, st.cu)), f"fused, records {rec}"
+        assert np.array_equal(valid(p, prim.t.cpu().numpy()), valid(p, st.prim)), f"fused prim, records {rec}"
+    ds = fc.DeviceState(p)
+    ds.cu.t.copy_(start)
+    ds.prim.t.copy_(start_prim)
+    for step in range(2):
+        fc.RK3step(ctx, ds, cfg.dt, noise=None, seed=6, step=step)
+    ctx.check()
+    assert np.array_equal(valid(p, ds.cu.t.cpu().numpy()), valid(p, st.cu)), "reference-shaped"
+    assert np.array_equal(valid(p, ds.prim.t.cpu().numpy()), valid(p, st.prim)), "reference-shaped prim"
+    host = perturbed_stag_state(p, cfg, orc, seed=16, amp=0.02, vel=3e3)
+    ss = S.StagState(p)
+    for dst, src in [(ss.cu, host.cu), (ss.prim, host.prim), *zip(ss.cumom, host.mom), *zip(ss.vel, host.vel)]:
+        dst.t.copy_(torch.from_numpy(src))
+    for step in range(2):
+        S.RK3stepStag(ctx, ss, cfg.dt, 8, step)
+    ctx.check()
+    assert host.advance(2, cfg.dt, 8, 0, chem=cfg.chem) == 0
+    for dst, src in [(ss.cu, host.cu), (ss.prim, host.prim), *zip(ss.cumom, host.mom), *zip(ss.vel, host.vel)]:
+        assert np.array_equal(dst.t.cpu().numpy(), src), "staggered"
